@@ -470,21 +470,22 @@ int argmin_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *X, i
     Carve cv;
     const size_t o_x64 = cv.take(stage_bytes(dtype, true, nx, tx));
     const size_t o_y64 = cv.take(stage_bytes(dtype, true, ny, ty));
-    const size_t o_d64 = cv.take((size_t)np * 8);
+    const size_t o_sq64 = cv.take((size_t)np * 8);  // certified: of the candidates
     const size_t o_heap = cv.take((size_t)nx * (size_t)k * 16);
-    size_t o_x32 = 0, o_y32 = 0, o_sq32 = 0, o_cnt = 0, o_off = 0, o_pa = 0, o_pb = 0, o_sq64 = 0,
-           o_mx = 0;
+    size_t o_d64 = 0, o_x32 = 0, o_y32 = 0, o_sq32 = 0, o_cnt = 0, o_off = 0, o_pa = 0, o_pb = 0,
+           o_mx = 0, o_words = 0;
     if (certified) {
         o_x32 = cv.take(stage_bytes(dtype, false, nx, tx));
         o_y32 = cv.take(stage_bytes(dtype, false, ny, ty));
         o_sq32 = cv.take((size_t)np * 4);
         o_cnt = cv.take((size_t)nx * 8);
-        o_off = cv.take((size_t)(nx + 1) * 8);
+        o_off = cv.take((size_t)nx * 8);
         o_pa = cv.take((size_t)np * 4);
         o_pb = cv.take((size_t)np * 4);
-        o_mx = cv.take(8);
+        o_words = cv.take(argmin_words_bytes(nx, ny));
+        o_mx = cv.take(16);  // candidate count, then the |x| max
     } else {
-        o_sq64 = cv.take((size_t)np * 8);
+        o_d64 = cv.take((size_t)np * 8);
     }
     void *wsp = nullptr;
     RC(ws_reserve(ctx, cv.total, &wsp));
@@ -495,65 +496,45 @@ int argmin_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *X, i
     const double *w64 = nullptr;
     const float *w32 = nullptr;
     if (m->kind == WBX_WDTW) RC(cached_weights(ctx, tx > ty ? tx : ty, m->g, &w64, &w32));
-    double *D64 = (double *)(ws + o_d64);
+    double *sq64 = (double *)(ws + o_sq64);
+    wbx_metric m64 = *m;
+    m64.precision = WBX_FP64;
     if (!certified) {
         PairSpec ps{PAIR_GRID, np, ny, nullptr, nullptr};
-        double *sq = (double *)(ws + o_sq64);
-        wbx_metric m64 = *m;
-        m64.precision = WBX_FP64;
+        double *D64 = (double *)(ws + o_d64);
         RC(run_pairs<double>(&m64, ps, series<double>(x64.ptr, x64.stride, tx),
-                             series<double>(y64.ptr, y64.stride, ty), w64, sq, st));
-        RC(launch_finish<double>(ps, sq, D64, ny, st));
-    } else {
-        Staged<float> x32, y32;
-        RC(stage<float>(dtype, X, nx, tx, xstr, ws, o_x32, &x32, st));
-        RC(stage<float>(dtype, Y, ny, ty, ystr, ws, o_y32, &y32, st));
-        float *sq32 = (float *)(ws + o_sq32);
-        PairSpec ps{PAIR_GRID, np, ny, nullptr, nullptr};
-        RC(run_pairs<float>(m, ps, series<float>(x32.ptr, x32.stride, tx),
-                            series<float>(y32.ptr, y32.stride, ty), w32, sq32, st));
-        double absmax = 0.0;
-        const bool exact_inputs = dtype == WBX_F32;
-        if (!exact_inputs) {
-            unsigned *mx = (unsigned *)(ws + o_mx);
-            WBX_HIP_CHECK(hipMemsetAsync(mx, 0, 4, st));
-            RC(launch_absmax_rows<double>((const double *)X, nx, tx, xstr, mx, st));
-            RC(launch_absmax_rows<double>((const double *)Y, ny, ty, ystr, mx, st));
-            unsigned hb = 0;
-            WBX_HIP_CHECK(hipMemcpyAsync(&hb, mx, 4, hipMemcpyDeviceToHost, st));
-            WBX_HIP_CHECK(hipStreamSynchronize(st));
-            float f;
-            memcpy(&f, &hb, 4);
-            absmax = (double)f;
-        }
-        ErrBound eb = make_err_bound((int)tx, (int)ty, m->kind == WBX_WDTW, absmax, exact_inputs);
-        int64_t total = 0;
-        int32_t *pa = (int32_t *)(ws + o_pa), *pb = (int32_t *)(ws + o_pb);
-        RC(launch_argmin_candidates(sq32, nx, ny, (int)k, eb, (int64_t *)(ws + o_cnt),
-                                    (int64_t *)(ws + o_off), pa, pb, &total, st));
-        RC(launch_fill_f64(D64, np, WBX_INF_D, st));
-        // exact FP64 values for the candidates; sq64 reuses the sq32+cnt area
-        // only if large enough, so give it the pa/pb-sized tail instead.
-        double *sq64 = (double *)(ws + o_sq32);  // np*4 bytes >= total*8 when total <= np/2
-        double *tmp = nullptr;
-        if ((size_t)total * 8 > (size_t)np * 4) {
-            if (hipMalloc(&tmp, (size_t)total * 8) != hipSuccess)
-                return fail(WBX_ENOMEM, "candidate buffer allocation failed");
-            sq64 = tmp;
-        }
-        PairSpec pl{PAIR_LIST, total, ny, pa, pb};
-        wbx_metric m64 = *m;
-        m64.precision = WBX_FP64;
-        int rc = run_pairs<double>(&m64, pl, series<double>(x64.ptr, x64.stride, tx),
-                                   series<double>(y64.ptr, y64.stride, ty), w64, sq64, st);
-        if (!rc) rc = launch_finish<double>(pl, sq64, D64, ny, st);
-        if (tmp) {
-            (void)hipStreamSynchronize(st);
-            (void)hipFree(tmp);
-        }
-        if (rc) return rc;
+                             series<double>(y64.ptr, y64.stride, ty), w64, sq64, st));
+        RC(launch_finish<double>(ps, sq64, D64, ny, st));
+        return launch_argmin_replay(D64, nx, ny, k, lb, ws + o_heap, idx, dist, st);
     }
-    return launch_argmin_replay(D64, nx, ny, k, lb, ws + o_heap, idx, dist, st);
+    Staged<float> x32, y32;
+    RC(stage<float>(dtype, X, nx, tx, xstr, ws, o_x32, &x32, st));
+    RC(stage<float>(dtype, Y, ny, ty, ystr, ws, o_y32, &y32, st));
+    float *sq32 = (float *)(ws + o_sq32);
+    PairSpec ps{PAIR_GRID, np, ny, nullptr, nullptr};
+    RC(run_pairs<float>(m, ps, series<float>(x32.ptr, x32.stride, tx),
+                        series<float>(y32.ptr, y32.stride, ty), w32, sq32, st));
+    const bool exact_inputs = dtype == WBX_F32;
+    unsigned long long *cnt = (unsigned long long *)(ws + o_mx);
+    unsigned *mx = (unsigned *)(ws + o_mx + 8);
+    if (!exact_inputs) {  // the largest |input| stays on the device
+        RC(launch_fill_i32((int *)mx, 1, 0, st));
+        RC(launch_absmax_rows<double>((const double *)X, nx, tx, xstr, mx, st));
+        RC(launch_absmax_rows<double>((const double *)Y, ny, ty, ystr, mx, st));
+    }
+    const ErrBound eb =
+        make_err_bound((int)tx, (int)ty, m->kind == WBX_WDTW, 1.0, exact_inputs);
+    int64_t total = 0;
+    int64_t *offs = (int64_t *)(ws + o_off), *counts = (int64_t *)(ws + o_cnt);
+    int32_t *pa = (int32_t *)(ws + o_pa), *pb = (int32_t *)(ws + o_pb);
+    RC(launch_argmin_candidates(sq32, nx, ny, (int)k, eb, exact_inputs ? nullptr : mx,
+                                ws + o_words, offs, counts, cnt, pa, pb, &total, st));
+    if (total > 0) {
+        PairSpec pl{PAIR_LIST, total, ny, pa, pb};
+        RC(run_pairs<double>(&m64, pl, series<double>(x64.ptr, x64.stride, tx),
+                             series<double>(y64.ptr, y64.stride, ty), w64, sq64, st));
+    }
+    return launch_argmin_replay_list(sq64, offs, counts, pb, nx, k, ws + o_heap, idx, dist, st);
 }
 
 // -------------------------------------------------------------- subsequence

@@ -15,8 +15,8 @@
 // pair j can be pushed only if d_j < T_j, where T_j is the k-th smallest of
 // d_0..d_{j-1}; T_j <= the k-th smallest hi over j' < j.  So every j with
 // lo_j < that running k-th smallest hi is a candidate and nothing else can be
-// pushed.  Candidates are re-evaluated exactly in FP64 and the replay runs on
-// exact values; non-candidates are +inf and are never pushed.
+// pushed.  Candidates are re-evaluated exactly in FP64 and the replay runs over
+// each row's candidates in column order; the others are never pushed.
 #include "wbx_internal.h"
 
 namespace wbx {
@@ -50,85 +50,133 @@ __device__ __forceinline__ void dist_bounds(float c, const ErrBound &eb, double 
 
 constexpr int KMAX = 32;
 
-// One lane per x row.  write == 0: count candidates; write == 1: emit them at
-// offs[i] into (pa, pb).
-__global__ __launch_bounds__(64) void k_argmin_candidates(const float *__restrict__ sq,
-                                                          int64_t nx, int64_t ny, int k,
-                                                          ErrBound eb, int write,
-                                                          int64_t *__restrict__ counts,
-                                                          const int64_t *__restrict__ offs,
-                                                          int32_t *__restrict__ pa,
-                                                          int32_t *__restrict__ pb) {
-    const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
-    if (i >= nx) return;
-    double top[KMAX];
-    int nf = 0;
-    int64_t cnt = 0;
-    const int64_t base = write ? offs[i] : 0;
-    for (int64_t j = 0; j < ny; ++j) {
-        double lo, hi;
-        dist_bounds(sq[i * ny + j], eb, lo, hi);
-        const double tup = nf < k ? WBX_INF_D : top[k - 1];
-        if (lo < tup) {
-            if (write) {
-                pa[base + cnt] = (int32_t)i;
-                pb[base + cnt] = (int32_t)j;
-            }
-            ++cnt;
-        }
-        // keep the k smallest hi values, ascending
-        if (nf < k || hi < top[k - 1]) {
-            int q = nf < k ? nf++ : k - 1;
-            while (q > 0 && top[q - 1] > hi) {
-                top[q] = top[q - 1];
-                --q;
-            }
-            top[q] = hi;
-        }
-    }
-    if (!write) counts[i] = cnt;
+__device__ __forceinline__ double lane_value(double v, int q) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, q);
+    const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), q);
+    return __builtin_bit_cast(double, hi << 32 | lo);
 }
 
-// Exclusive scan of counts (nx values) into offs[0..nx], one block.
-__global__ __launch_bounds__(1024) void k_scan_counts(const int64_t *__restrict__ counts,
-                                                      int64_t nx, int64_t *__restrict__ offs) {
-    __shared__ int64_t part[1024];
-    const int t = threadIdx.x;
-    const int64_t per = (nx + 1023) / 1024;
-    const int64_t s = (int64_t)t * per, e = s + per < nx ? s + per : nx;
-    int64_t acc = 0;
-    for (int64_t q = s; q < e; ++q) acc += counts[q];
-    part[t] = acc;
-    __syncthreads();
-    if (t == 0) {
-        int64_t run = 0;
-        for (int q = 0; q < 1024; ++q) {
-            int64_t v = part[q];
-            part[q] = run;
-            run += v;
+// One wave per x row.  The k smallest hi values so far sit in lanes 0 .. k - 1
+// in ascending order (+inf where there are fewer), T is the k-th.  64 costs
+// are read together; T only falls, so a cost whose lo is not below the T at
+// the start of its 64 can neither be a candidate nor change T (hi >= lo), and
+// one comparison with the cost at which lo reaches T drops it.  The others
+// are taken in column order, which selects what a scan of the row selects.
+// A row's candidates are one bit per column in `words` (the lane that stores
+// a word reads it back); when the row is done the wave reserves their places in the pair list with one atomic and writes
+// them there in column order (the order of the rows in the list is free).
+//
+// Bound by the latency of the loads and of the selection steps (a row needs
+// about k ln(ny / k) of them).  500 rows of 4000, k = 5: 40 us.  One
+// lane per row, in two passes with a division and a square root for every
+// cost, took 2 x 2390 us there: 8 waves, their loads ny floats apart.
+__global__ __launch_bounds__(64) void k_argmin_candidates(
+    const float *__restrict__ sq, int64_t nx, int64_t ny, int k, ErrBound eb,
+    const unsigned *__restrict__ absmax_bits, uint64_t *words, int64_t *__restrict__ offs,
+    int64_t *__restrict__ counts, unsigned long long *__restrict__ total,
+    int32_t *__restrict__ pa, int32_t *__restrict__ pb) {
+    const int64_t i = (int64_t)blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
+    if (i >= nx) return;  // uniform
+    const int lane = threadIdx.x;
+    if (absmax_bits) {  // A was made for |x| <= 1
+        const double m = (double)__uint_as_float(*absmax_bits);
+        eb.A *= m * m;
+    }
+    const float *__restrict__ row = sq + i * ny;
+    const int64_t nw = (ny + 63) / 64;
+    uint64_t *wrow = words + i * nw;
+    // the starting +inf goes through a vector register: as a constant in a
+    // scalar pair the compiler writes it with one 32-bit literal, which is 0
+    double top = WBX_INF_D;
+    asm volatile("" : "+v"(top));
+    double T = lane_value(top, 0), cth = T;
+    int64_t cnt = 0;
+    constexpr int UC = 4;  // groups of 64 costs in flight
+    for (int64_t w0 = 0; w0 < nw; w0 += UC) {
+        float cv[UC];
+#pragma unroll
+        for (int u = 0; u < UC; ++u) {
+            const int64_t j = (w0 + u) * 64 + lane;
+            cv[u] = j < ny ? row[j] : 0.0f;
         }
-        offs[nx] = run;
+#pragma unroll
+        for (int u = 0; u < UC; ++u) {
+            const int64_t j = (w0 + u) * 64 + lane;
+            if (w0 + u >= nw) break;  // uniform
+            const float c = cv[u];
+            // a cost that is not finite has lo = 0
+            uint64_t mask = __ballot(j < ny && (!(c < WBX_INF_F) || (double)c < cth));
+            uint64_t word = 0;
+            if (mask) {
+                double lo, hi;
+                dist_bounds(c, eb, lo, hi);
+                while (mask) {
+                    const int q = __builtin_ctzll(mask);
+                    mask &= mask - 1;
+                    if (lane_value(lo, q) < T) word |= (uint64_t)1 << q;
+                    const double hq = lane_value(hi, q);
+                    if (hq < T) {
+                        const int pos =
+                            __popcll(__ballot(lane < k && top <= hq));
+                        const double below = __shfl_up(top, 1);
+                        top = lane < pos ? top : lane == pos ? hq : below;
+                        T = lane_value(top, k - 1);
+                    }
+                }
+                // lo(c) < T only if c is below this
+                cth = (T * T / (1.0 - eb.e64) * eb.e_up + eb.A) * (1.0 + 1e-9);
+                cnt += __popcll(word);
+            }
+            if (lane == (int)((w0 + u) & 63)) wrow[w0 + u] = word;
+        }
     }
-    __syncthreads();
-    acc = part[t];
-    for (int64_t q = s; q < e; ++q) {
-        offs[q] = acc;
-        acc += counts[q];
+    unsigned long long base = 0;
+    if (lane == 0) {
+        base = atomicAdd(total, (unsigned long long)cnt);
+        offs[i] = (int64_t)base;
+        counts[i] = cnt;
     }
+    base = (unsigned long long)__shfl((long long)base, 0);
+    for (int64_t w0 = 0; w0 < nw; w0 += 64) {
+        const int64_t wi = w0 + lane;
+        uint64_t word = wi < nw ? wrow[wi] : 0;  // stored by this lane
+        const int own = __popcll(word);
+        int inc = own;  // inclusive scan over the lanes
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(inc, d);
+            if (lane >= d) inc += o;
+        }
+        unsigned long long q = base + (unsigned long long)(inc - own);
+        while (word) {
+            const int e = __builtin_ctzll(word);
+            word &= word - 1;
+            pa[q] = (int32_t)i;
+            pb[q] = (int32_t)(wi * 64 + e);
+            ++q;
+        }
+        base += (unsigned long long)__shfl(inc, 63);
+    }
+}
+
+size_t argmin_words_bytes(int64_t nx, int64_t ny) {
+    return (size_t)nx * (size_t)((ny + 63) / 64) * 8;
 }
 
 int launch_argmin_candidates(const float *sq, int64_t nx, int64_t ny, int k, const ErrBound &eb,
-                             int64_t *counts, int64_t *offs, int32_t *pa, int32_t *pb,
+                             const unsigned *absmax_bits, void *words, int64_t *offs,
+                             int64_t *counts, unsigned long long *total, int32_t *pa, int32_t *pb,
                              int64_t *total_host, hipStream_t st) {
     if (k > KMAX) return fail(WBX_EUNSUPPORTED, "certified argmin supports k <= %d", KMAX);
-    const dim3 grid((unsigned)((nx + 63) / 64));
-    hipLaunchKernelGGL(k_argmin_candidates, grid, dim3(64), 0, st, sq, nx, ny, k, eb, 0, counts,
-                       offs, pa, pb);
-    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, counts, nx, offs);
-    hipLaunchKernelGGL(k_argmin_candidates, grid, dim3(64), 0, st, sq, nx, ny, k, eb, 1, counts,
-                       offs, pa, pb);
+    int rc = launch_fill_i32((int *)total, 2, 0, st);
+    if (rc) return rc;
+    const int64_t gx = nx < 65535 ? nx : 65535;
+    hipLaunchKernelGGL(k_argmin_candidates, dim3((unsigned)gx, (unsigned)((nx + gx - 1) / gx)),
+                       dim3(64), 0, st, sq, nx, ny, k, eb, absmax_bits, (uint64_t *)words, offs,
+                       counts, total, pa, pb);
     WBX_HIP_CHECK(hipGetLastError());
-    WBX_HIP_CHECK(hipMemcpyAsync(total_host, offs + nx, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    WBX_HIP_CHECK(hipMemcpyAsync(total_host, total, sizeof(int64_t), hipMemcpyDeviceToHost, st));
     WBX_HIP_CHECK(hipStreamSynchronize(st));
     return WBX_OK;
 }

@@ -272,6 +272,12 @@ int launch_argmin_replay(const double *D, int64_t nx, int64_t ny, int64_t k,
                          const double *lower_bound, void *heaps, int64_t *idx, double *dist,
                          hipStream_t st);
 
+// The same over each row's candidates only: row i's are sq / pb[off[i] ..
+// off[i] + cnt[i]), squared costs and columns (ascending).
+int launch_argmin_replay_list(const double *sq, const int64_t *off, const int64_t *cnt,
+                              const int32_t *pb, int64_t nx, int64_t k, void *heaps, int64_t *idx,
+                              double *dist, hipStream_t st);
+
 // End-of-series lengths: len[i] = index of the first EOS of row i (or t).
 template <typename T>
 int launch_eos_lengths(const T *X, int64_t n, int64_t stride, int t, int32_t *len,
@@ -431,8 +437,14 @@ struct ErrBound {
     double e_up, e_dn, A, e64;
 };
 ErrBound make_err_bound(int lx, int ly, int weighted, double absmax, int inputs_exact);
+// Row i's candidates are (pa, pb)[offs[i] .. offs[i] + counts[i]), columns
+// ascending; *total_host their number over all rows (the call waits for it).
+// absmax_bits (nullable): device float bits of max |input|, with eb made for
+// inputs up to 1.  words: argmin_words_bytes of scratch.
+size_t argmin_words_bytes(int64_t nx, int64_t ny);
 int launch_argmin_candidates(const float *sq, int64_t nx, int64_t ny, int k, const ErrBound &eb,
-                             int64_t *counts, int64_t *offs, int32_t *pa, int32_t *pb,
+                             const unsigned *absmax_bits, void *words, int64_t *offs,
+                             int64_t *counts, unsigned long long *total, int32_t *pa, int32_t *pb,
                              int64_t *total_host, hipStream_t st);
 
 }  // namespace wbx
