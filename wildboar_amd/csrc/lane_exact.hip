@@ -13,10 +13,20 @@ namespace {
 template <int B>
 void launch_exact(const PairSpec &ps, Series<float> xs, Series<float> ys, const LaneGeo &g,
                   float *sq, hipStream_t st) {
-    // rows per window shift as the padded kernels use for the same width
-    constexpr int U = (B + 7) / 8 * 8 <= 88 ? 8 : 4;
-    dim3 grid((unsigned)((ps.n_pairs + 63) / 64));
-    hipLaunchKernelGGL((k_lane_dtw_exact<B, U>), grid, dim3(64), 0, st, ps, xs, ys, g, sq);
+    // rows per window shift: 8 while the x registers of a wave without a
+    // shared x fit too
+    constexpr int U = 8, U1 = B <= 88 ? 8 : 4;
+    const int64_t waves = (ps.n_pairs + 63) / 64;
+    // A shared x saves 8-12 % of the time; waves that end with a row of the
+    // matrix are partly idle, so it is taken while they are at most 6 % more.
+    const int64_t waves_xu =
+        ps.mode == PAIR_GRID ? ps.n_pairs / ps.ny * ((ps.ny + 63) / 64) : INT64_MAX;
+    if (waves_xu <= waves + waves / 16 && waves_xu <= INT32_MAX)
+        hipLaunchKernelGGL((k_lane_dtw_exact<B, U, true>), dim3((unsigned)waves_xu), dim3(64), 0,
+                           st, ps, xs, ys, g, sq);
+    else
+        hipLaunchKernelGGL((k_lane_dtw_exact<B, U1, false>), dim3((unsigned)waves), dim3(64), 0, st,
+                           ps, xs, ys, g, sq);
 }
 
 }  // namespace

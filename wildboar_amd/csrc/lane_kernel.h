@@ -23,6 +23,16 @@
 // slot B-1 never sees them.  Exact instantiations (BP == B, odd B, the band
 // of every pair of equal lengths) compute no padding slot and need no reset.
 //
+// Exact instantiations, x of a wave.  Where the 64 pairs of a wave share
+// their x series (a matrix whose rows are cut into waves of 64 columns), x
+// comes by scalar loads and is an SGPR operand of v_sub.  In straight-line
+// rows on real data that alone is 19.6 -> 23.0e12 cells/s: one register-file
+// read less per cell, which the card's power limit turns into clock (constant
+// series run 17 % faster than random walks with the same instructions).
+// A cell's minimum and fma are one asm block on its row register, so the row
+// is updated in place; left to itself the allocator keeps a second copy of it
+// (B = 75: 236 registers for 157 values) and, at B = 101, spills.
+//
 // WDTW (WeightedDtwMetric, distance/_elastic.pyx:3322-3341) multiplies each
 // cell's squared difference by w[|i - j|]; in band coordinates |i - j| =
 // |k - off| is fixed per slot, so every lane of a launch uses the same weight
@@ -32,18 +42,18 @@
 // prefix-sum weights w[j - 1] (w[0] for j = 0, :893-906), a second LDS row.
 #pragma once
 
+#include <type_traits>
+
 #include "lane_common.h"
 
 namespace wbx {
 
 // pen[q] is +inf for slot BP-8+q == B and -inf otherwise (uniform values), so
-// max(row, pen) resets slot B without a branch.  EX: the band is exactly BP
-// slots (B == BP), the last slot's up input is the constant +inf and no slot
-// needs a reset.
+// max(row, pen) resets slot B without a branch.
 // AD: the amercing recursion (adtw_distance, distance/_elastic.pyx:943-1008),
 // m = min3(up + p, left + p, diag); row 0 runs with p = 0 (its prefix sum
 // carries no penalty).
-template <int BP, bool AD = false, bool WT = false, bool EX = false>
+template <int BP, bool AD = false, bool WT = false>
 __device__ __forceinline__ void lane_row(float (&row)[BP], const float *yw, float xi,
                                          const float (&pen)[8], float p = 0.0f,
                                          const float *wslot = nullptr) {
@@ -65,13 +75,11 @@ __device__ __forceinline__ void lane_row(float (&row)[BP], const float *yw, floa
         row[k] = c;
         left = c;
     }
-    if constexpr (!EX) {
 #pragma unroll
-        for (int q = 1; q < 8; ++q) row[BP - 8 + q] = fmaxf(row[BP - 8 + q], pen[q]);
-    }
+    for (int q = 1; q < 8; ++q) row[BP - 8 + q] = fmaxf(row[BP - 8 + q], pen[q]);
 }
 
-template <int BP, int U, bool AD = false, bool WT = false, bool EX = false>
+template <int BP, int U, bool AD = false, bool WT = false>
 __device__ __forceinline__ void lane_dtw_body(PairSpec ps, Series<float> xs,
                                                  Series<float> ys, LaneGeo g, float pen_ad,
                                                  const float *__restrict__ weights,
@@ -109,14 +117,14 @@ __device__ __forceinline__ void lane_dtw_body(PairSpec ps, Series<float> xs,
 
     int i_begin = 0;
     if constexpr (WT) {
-        lane_row<BP, false, true, EX>(row, yw, X[0], pen, 0.0f, lw[0]);
+        lane_row<BP, false, true>(row, yw, X[0], pen, 0.0f, lw[0]);
 #pragma unroll
         for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
         yw[W - 1] = ldy(Y, 1 - off + W - 1, ly);
         i_begin = 1;
     }
     if constexpr (AD) {
-        lane_row<BP, true, false, EX>(row, yw, X[0], pen, 0.0f);
+        lane_row<BP, true, false>(row, yw, X[0], pen, 0.0f);
 #pragma unroll
         for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
         yw[W - 1] = ldy(Y, 1 - off + W - 1, ly);
@@ -125,7 +133,7 @@ __device__ __forceinline__ void lane_dtw_body(PairSpec ps, Series<float> xs,
     // Leading rows one at a time so the rest is a whole number of U-groups.
     const int rem = (lx - i_begin) % U;
     for (int i = i_begin; i < i_begin + rem; ++i) {
-        lane_row<BP, AD, WT, EX>(row, yw, X[i], pen, pen_ad, WT ? lw[WT ? 1 : 0] : nullptr);
+        lane_row<BP, AD, WT>(row, yw, X[i], pen, pen_ad, WT ? lw[WT ? 1 : 0] : nullptr);
 #pragma unroll
         for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
         yw[W - 1] = ldy(Y, i + 1 - off + W - 1, ly);
@@ -145,7 +153,7 @@ __device__ __forceinline__ void lane_dtw_body(PairSpec ps, Series<float> xs,
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if constexpr (WT) asm volatile("" ::: "memory");
-                lane_row<BP, AD, WT, EX>(row, yw + u, xv[u], pen, pen_ad,
+                lane_row<BP, AD, WT>(row, yw + u, xv[u], pen, pen_ad,
                                          WT ? lw[WT ? 1 : 0] : nullptr);
             }
 #pragma unroll
@@ -192,7 +200,7 @@ __device__ __forceinline__ void lane_dtw_body(PairSpec ps, Series<float> xs,
                 // in registers across the loop (the band row and y window
                 // fill them)
                 if constexpr (WT) asm volatile("" ::: "memory");
-                lane_row<BP, AD, WT, EX>(row, yw + u, xv[u], pen, pen_ad,
+                lane_row<BP, AD, WT>(row, yw + u, xv[u], pen, pen_ad,
                                          WT ? lw[WT ? 1 : 0] : nullptr);
             }
 #pragma unroll
@@ -219,16 +227,144 @@ template <int BP, int U, bool AD = false, bool WT = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AD || WT ? 1 : 2))) void
 k_lane_dtw(PairSpec ps, Series<float> xs, Series<float> ys, LaneGeo g, float pen_ad,
            const float *__restrict__ weights, float *__restrict__ sq) {
-    lane_dtw_body<BP, U, AD, WT, false>(ps, xs, ys, g, pen_ad, weights, sq);
+    lane_dtw_body<BP, U, AD, WT>(ps, xs, ys, g, pen_ad, weights, sq);
 }
 
-// Exact bands, plain DTW.  Two waves per SIMD (at most 256 registers) is what
-// keeps the VALU busy -- one wave issues about half as often -- so the
-// allocator is held to it; the band row and y window fit (2B + 3 registers).
-template <int B, int U>
+// One row of an exact band (m = min3(up, left, diag), c = fma(d, d, m)
+// in the row register itself; the outermost slots lack one input).
+template <int B>
+__device__ __forceinline__ void exact_row(float (&row)[B], const float *yw, float xi) {
+    float left = WBX_INF_F;
+#pragma unroll
+    for (int k = 0; k < B; ++k) {
+        const float d = xi - yw[k];
+        if (k == 0)
+            asm("v_min_f32 %0, %1, %0\n\tv_fmac_f32 %0, %2, %2"
+                : "+v"(row[k])
+                : "v"(row[1]), "v"(d));
+        else if (k + 1 < B)
+            asm("v_min3_f32 %0, %1, %2, %0\n\tv_fmac_f32 %0, %3, %3"
+                : "+v"(row[k])
+                : "v"(row[k + 1]), "v"(left), "v"(d));
+        else
+            asm("v_min_f32 %0, %1, %0\n\tv_fmac_f32 %0, %2, %2"
+                : "+v"(row[k])
+                : "v"(left), "v"(d));
+        left = row[k];
+    }
+}
+
+// x of a wave that shares one series: constant address space, so the loads
+// are scalar.
+typedef const float __attribute__((address_space(4))) *cfloat;
+
+// Exact bands, plain DTW.  XU: grid pairs, wave blk runs row blk / nb against
+// columns 64 (blk % nb) .. + 63, nb = ceil(ny / 64); else wave blk runs pairs
+// 64 blk .. + 63 of any kind, x per lane.  Two waves per SIMD (at most 256
+// registers) keep the VALU busy -- one wave issues about half as often.
+// Bound by VALU issue and the clock that power allows; groups of 8 rows move
+// the window half as often as groups of 4 (13 instead of 26 moves a row at
+// B = 101), longer groups gain nothing.  2000 x 2000 x 512 on one box, x per
+// lane -> XU: B = 23 2.92 -> 2.67 ms, B = 49 5.52 -> 5.23, B = 75 8.83 -> 8.10,
+// B = 101 12.02 -> 10.73, B = 111 13.05 -> 11.70.
+template <int B, int U, bool XU>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_lane_dtw_exact(
     PairSpec ps, Series<float> xs, Series<float> ys, LaneGeo g, float *__restrict__ sq) {
-    lane_dtw_body<B, U, false, false, true>(ps, xs, ys, g, 0.0f, nullptr, sq);
+    constexpr int W = B + U - 1;
+    static_assert(U % 4 == 0, "groups of whole 16-byte loads");
+    const int lane = threadIdx.x;
+    const int lx = g.lx, ly = g.ly, off = g.off;
+    int64_t a, b, p0;
+    bool live;
+    if constexpr (XU) {
+        const unsigned ny = (unsigned)ps.ny, nb = (ny + 63) / 64;
+        const unsigned blk = (unsigned)xcd_block(blockIdx.x, gridDim.x);
+        const unsigned ra = (unsigned)__builtin_amdgcn_readfirstlane((int)(blk / nb));
+        const unsigned j = (blk - ra * nb) * 64 + lane;
+        live = j < ny;
+        a = ra;
+        b = live ? j : ny - 1;
+        p0 = a * ps.ny + j;
+    } else {
+        p0 = xcd_block(blockIdx.x, gridDim.x) * 64 + lane;
+        live = p0 < ps.n_pairs;
+        decode_pair(ps, live ? p0 : ps.n_pairs - 1, a, b);
+    }
+    using XP = typename std::conditional<XU, cfloat, const float *>::type;
+    const XP X = (XP)xs.row(a);
+    const float *__restrict__ Y = ys.row(b);
+
+    float row[B];
+#pragma unroll
+    for (int k = 0; k < B; ++k) row[k] = (k == off) ? 0.0f : WBX_INF_F;
+    // the first window, 8 loads at a time: all of them in flight would need
+    // an address register pair each
+    float yw[W];
+#pragma unroll
+    for (int m = 0; m < W; ++m) {
+        yw[m] = ldy(Y, m - off, ly);
+        if ((m & 7) == 7) __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // leading rows one at a time so the rest is a whole number of groups
+    const int rem = lx % U;
+    for (int i = 0; i < rem; ++i) {
+        exact_row<B>(row, yw, X[i]);
+#pragma unroll
+        for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
+        yw[W - 1] = ldy(Y, i + 1 - off + W - 1, ly);
+    }
+    // x of the current group; the loop loads the next group's with the
+    // group's new window entries (columns jn .. jn + U - 1, jn > 0) before
+    // the rows run.  The lanes share the geometry: when both lie inside their
+    // rows (every group but the last one or two) they are plain loads, else x
+    // is clamped into the row (never used past it) and y is +inf outside it.
+    float xv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) xv[u] = X[min(rem + u, lx - 1)];
+    // the loads above are waited for here: left in flight, the wait for them
+    // inside the loop would cover the group's own loads too
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    for (int i0 = rem; i0 < lx; i0 += U) {
+        float xn[U], yn[U];
+        const int jn = i0 - off + W;
+        if (i0 + 2 * U <= lx && jn + U <= ly) {
+#pragma unroll
+            for (int u = 0; u < U; u += 4) {
+                const f4a bv = *(const f4a *)(Y + jn + u);
+                if constexpr (XU) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) xn[u + q] = X[i0 + U + u + q];
+                } else {
+                    const f4a av = *(const f4a *)(X + i0 + U + u);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) xn[u + q] = av[q];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) yn[u + q] = bv[q];
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                xn[u] = X[min(i0 + U + u, lx - 1)];
+                yn[u] = ldy(Y, jn + u, ly);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) exact_row<B>(row, yw + u, xv[u]);
+#pragma unroll
+        for (int m = 0; m < W - U; ++m) yw[m] = yw[m + U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            yw[W - U + u] = yn[u];
+            xv[u] = xn[u];
+        }
+    }
+    float res = WBX_INF_F;
+#pragma unroll
+    for (int k = 0; k < B; ++k)
+        if (k == g.kf) res = row[k];
+    if (live) sq[p0] = res;
 }
 
 }  // namespace wbx
