@@ -18,6 +18,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "lane_common.h"
 #include "subseq_fast.h"
 #include "subseq_mfma.h"
 #include "wbx_internal.h"
@@ -270,18 +271,36 @@ int run_pairs(const wbx_metric *m, const PairSpec &ps, Series<T> xs, Series<T> y
             ProfScope pf(st, KERN_FULL);
             return launch_full_dtw<T>(ps, xs, ys, sq, st);
         }
-        // one pair per lane while that is faster than a group of lanes per
-        // pair (measured on MI355X, 1000 x 1000 x 256: float32 DTW lanes up
-        // to 112 slots; float32 WDTW and float64 lanes up to 40 slots -- at
-        // 49 slots the group kernel is 1.1-1.4x faster, at 23 the lanes
-        // 1.6-1.8x); ADTW stays on the lanes (no group form)
+        // One pair per lane does the fewest instructions per cell, a group of
+        // lanes per pair has the shorter chain: whichever is estimated
+        // faster for this many pairs.  Per row, a lane wave alone on its SIMD
+        // takes 5.5 ns a slot and shares it at 3.3 (float32 DTW; measured at
+        // B = 23, 49, 101; at 20000 pairs of 512, B = 101, 293 us against
+        // 124 us of six lanes a pair, at 100000 359 against 469).  Padded
+        // widths, weights and float64 cost more; float32 WDTW and float64
+        // lanes are for bands up to 40 slots (at 49 the group kernel is
+        // 1.1-1.4x faster at any size); ADTW has no group form.
+        constexpr bool dbl = !std::is_same<T, float>::value;
         bool lane;
-        if constexpr (std::is_same<T, float>::value)
+        double lane_ns = 0.0;
+        const int64_t lane_waves = (ps.n_pairs + 63) / 64;
+        if constexpr (!dbl) {
             lane = lane_supported(xs.len, ys.len, m->r, wt, w_fixed) && (!wt || B <= 40);
-        else
-            lane = lane64_pairs_class(B, wt) != 0 && (B <= 40 || pen);
+            const bool exact = !wt && lane_exact_supported(B);
+            const int slots = exact ? B : (B + 7) / 8 * 8;
+            lane_ns = pair_launch_ns(lane_waves, bd.lx, (exact ? 20.0 : 30.0) + (wt ? 7.5 : 5.5) * slots,
+                                     (wt ? 4.8 : 3.4) * slots);
+        } else {
+            const int slots = lane64_pairs_class(B, wt);
+            lane = slots != 0 && (B <= 40 || pen);
+            lane_ns = pair_launch_ns(lane_waves, bd.lx, (wt ? 13.5 : 11.5) * slots,
+                                     (wt ? 13.0 : 11.0) * slots);
+        }
         GroupGeo gg{};
-        const bool group = !pen && group_plan(B, bd.lx, !std::is_same<T, float>::value, wt, &gg);
+        double group_ns = 0.0;
+        const bool group =
+            !pen && group_plan(B, bd.lx, ps.n_pairs, dbl, wt, &gg, &group_ns);
+        if (group && group_ns < lane_ns) lane = false;
         if (policy == 2 && group) lane = false;  // group kernel wherever it applies
         if (lane) {
             ProfScope pf(st, KERN_LANE);

@@ -28,6 +28,8 @@
 // stays +inf).
 #pragma clang fp contract(off)
 
+#include <type_traits>
+
 #include "wbx_internal.h"
 
 namespace wbx {
@@ -205,8 +207,7 @@ __device__ __forceinline__ void gstep(GLane<T, R, U, WT> &L, int u, T x, int lx,
     L.l = L.shortl ? L.row[R - 1] : L.row[R];
 }
 
-// Single steps s in [s0, s1) (fill / drain / remainder), window shifted by
-// one each step.
+// Single steps, the window shifted by one each step.
 template <typename T, int R, int U, bool WT, bool SEL, bool W0>
 __device__ __forceinline__ void gsingle(GLane<T, R, U, WT> &L, int steps, const T *__restrict__ X,
                                         const T *__restrict__ Y, int lx, int ly, const T *w0) {
@@ -264,55 +265,73 @@ __global__ __launch_bounds__(64) void k_group_dtw(PairSpec ps, Series<T> xs, Ser
             w0[m] = wv[c0 < top ? c0 : top];
         }
     }
-    // fill: steps [0, n); lanes before their row 0 keep their state
-    const int fill = g.n;
-    gsingle<T, R, U, WT, true, WT>(L, fill, X, Y, lx, ly, w0);
-    // steady: steps [n, lx), every lane inside rows [1, lx)
-    int steady = lx - fill;
-    if (steady > 0) {
-        const int rem = steady % U;
-        gsingle<T, R, U, WT, false, false>(L, rem, X, Y, lx, ly, w0);
-        T xv[U], yn[U];
+    auto shift_in = [&](const T(&ynew)[U]) {
+#pragma unroll
+        for (int m = 0; m < W - U; ++m) L.yw[m] = L.yw[m + U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) L.yw[W - U + u] = ynew[u];
+        L.r += U;
+        L.yj += U;
+    };
+    // Steps go in groups of U, each group's x rows and window entries loaded
+    // a group ahead.  Steps in which some lane is outside its rows (the first
+    // n - 1 and those past row lx - 1 of lane 0) keep that lane's state
+    // through a select per cell.  Short strips have many such steps (n = 17
+    // for R = 2 at band 49) and are for calls too small to hide a load at
+    // each, so their edge steps go in groups too: 50 pairs of 256, R = 2:
+    // 24.7 -> 20.8 us.  Long strips make them one at a time: the up to 2 U - 2
+    // more steps with selects cost 2-5 % of a large call, and both weight
+    // vectors at once a wave per SIMD (R = 24: 185 registers instead of 154).
+    constexpr bool kEdgeGroups = R <= 6;
+    const int steps = lx + g.n - 1;
+    int s = 0;
+    if constexpr (!kEdgeGroups) {
+        s = g.n + (lx > g.n ? (lx - g.n) % U : 0);
+        gsingle<T, R, U, WT, true, WT>(L, g.n, X, Y, lx, ly, w0);
+        gsingle<T, R, U, WT, false, false>(L, s - g.n, X, Y, lx, ly, w0);
+    }
+    T xv[U], yn[U];
+    group_loads<T, U>(X, Y, L.r, L.yj + W, lx, ly, xv, yn);
+    auto edge_group = [&](auto w0_steps) {
+        constexpr bool W0 = decltype(w0_steps)::value;
+        T xb[U], yb[U];
+        group_loads<T, U>(X, Y, L.r + U, L.yj + W + U, lx, ly, xb, yb);
+#pragma unroll
+        for (int u = 0; u < U; ++u) gstep<T, R, U, WT, true, W0>(L, u, xv[u], lx, w0);
+        shift_in(yn);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            xv[u] = ldx(X, L.r + u, lx);
-            yn[u] = ldyg(Y, L.yj + W + u, ly);
+            xv[u] = xb[u];
+            yn[u] = yb[u];
         }
-        // groups in pairs: the second group's x and y entries go to registers
-        // the first does not read, and the next pair's to xv / yn, so no
-        // group copies its successor's loads
-        auto shift_in = [&](const T(&ynew)[U]) {
+    };
+    if constexpr (kEdgeGroups)
+        for (; s < g.n; s += U) edge_group(std::integral_constant<bool, WT>());
+    // steady groups in pairs: the second group's x and y entries go to
+    // registers the first does not read, and the next pair's to xv / yn, so
+    // no group copies its successor's loads
+    for (; s + 2 * U <= lx; s += 2 * U) {
+        T xb[U], yb[U];
+        group_loads<T, U>(X, Y, L.r + U, L.yj + W + U, lx, ly, xb, yb);
 #pragma unroll
-            for (int m = 0; m < W - U; ++m) L.yw[m] = L.yw[m + U];
+        for (int u = 0; u < U; ++u) gstep<T, R, U, WT, false, false>(L, u, xv[u], lx, w0);
+        shift_in(yn);
+        group_loads<T, U>(X, Y, L.r + U, L.yj + W + U, lx, ly, xv, yn);
 #pragma unroll
-            for (int u = 0; u < U; ++u) L.yw[W - U + u] = ynew[u];
-            L.r += U;
-            L.yj += U;
-        };
-        int s = rem;
-        for (; s + 2 * U <= steady; s += 2 * U) {
-            T xb[U], yb[U];
-            group_loads<T, U>(X, Y, L.r + U, L.yj + W + U, lx, ly, xb, yb);
-#pragma unroll
-            for (int u = 0; u < U; ++u) gstep<T, R, U, WT, false, false>(L, u, xv[u], lx, w0);
-            shift_in(yn);
-            group_loads<T, U>(X, Y, L.r + U, L.yj + W + U, lx, ly, xv, yn);
-#pragma unroll
-            for (int u = 0; u < U; ++u) gstep<T, R, U, WT, false, false>(L, u, xb[u], lx, w0);
-            shift_in(yb);
-        }
-        if (s < steady) {  // one group left
-#pragma unroll
-            for (int u = 0; u < U; ++u) gstep<T, R, U, WT, false, false>(L, u, xv[u], lx, w0);
-            shift_in(yn);
-        }
-    } else {
-        steady = 0;
+        for (int u = 0; u < U; ++u) gstep<T, R, U, WT, false, false>(L, u, xb[u], lx, w0);
+        shift_in(yb);
     }
-    // drain: steps [max(n, lx), lx + n - 1); lanes past row lx - 1 keep it
-    const int done = fill + steady;
-    const int drain = lx + g.n - 1 - done;
-    gsingle<T, R, U, WT, true, false>(L, drain, X, Y, lx, ly, w0);
+    if (s + U <= lx) {  // one group left
+#pragma unroll
+        for (int u = 0; u < U; ++u) gstep<T, R, U, WT, false, false>(L, u, xv[u], lx, w0);
+        shift_in(yn);
+        s += U;
+        if constexpr (kEdgeGroups) group_loads<T, U>(X, Y, L.r, L.yj + W, lx, ly, xv, yn);
+    }
+    if constexpr (kEdgeGroups)
+        for (; s < steps; s += U) edge_group(std::false_type());
+    else if (s < steps)
+        gsingle<T, R, U, WT, true, false>(L, steps - s, X, Y, lx, ly, w0);
 
     const int nslots = L.shortl ? R : S;
     if (valid && g.kf >= k0 && g.kf < k0 + nslots) {
@@ -328,10 +347,14 @@ __global__ __launch_bounds__(64) void k_group_dtw(PairSpec ps, Series<T> xs, Ser
 constexpr int kGroupR32[] = {2, 3, 4, 6, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40};
 constexpr int kGroupR64[] = {2, 3, 4, 6, 8, 10, 12, 14, 16, 20, 24};
 
+// Steps per group: a narrow strip's four steps are shorter than a load.
+template <int R>
+constexpr int kGroupU = R <= 6 ? 8 : 4;
+
 template <typename T, int R, bool WT>
 void launch_group_one(const PairSpec &ps, Series<T> xs, Series<T> ys, const GroupGeo &g,
                       const T *w, T *sq, hipStream_t st) {
-    constexpr int U = 4;
+    constexpr int U = kGroupU<R>;
     const dim3 grid((unsigned)((ps.n_pairs + g.P - 1) / g.P));
     hipLaunchKernelGGL((k_group_dtw<T, R, U, WT>), grid, dim3(64), 0, st, ps, xs, ys, g, w, sq);
 }
@@ -365,34 +388,45 @@ int launch_group_r(int R, const PairSpec &ps, Series<T> xs, Series<T> ys, const 
 
 }  // namespace
 
-// Chooses the strip size R and lanes per pair n for band width B: among the
-// compiled R with n R <= B <= n (R + 1), n <= 64, the one with the most
-// band cells per VALU instruction of a wave step, counting the 64 / n pairs a
-// wave holds, the per-row cost k (R + 1) + 8 (cells, two DPP moves and their
-// group-edge selects, the short-lane select) and the fill and drain steps.
-bool group_plan(int B, int lx, bool fp64, bool weighted, GroupGeo *g) {
+// Chooses the strip size R and lanes per pair n for band width B among the
+// compiled R with n R <= B <= n (R + 1), n <= 64: the smallest time of
+// n_pairs pairs.  A call that fills the chip wants few, long strips (less
+// overhead per cell), one that leaves it idle short ones (fewer cells in
+// turn): pair_launch_ns has the figures.
+bool group_plan(int B, int lx, int64_t n_pairs, bool fp64, bool weighted, GroupGeo *g,
+                double *ns) {
     const int *tab = fp64 ? kGroupR64 : kGroupR32;
     const int nt = fp64 ? (int)(sizeof(kGroupR64) / sizeof(int))
                         : (int)(sizeof(kGroupR32) / sizeof(int));
-    const double k = fp64 ? (weighted ? 6.0 : 5.0) : (weighted ? 4.0 : 3.0);
+    // A step of a wave alone on its SIMD, and each further wave's share of
+    // it, in ns for strips of S = R + 1 slots (MI355X, 256 x 256 series,
+    // band 49, R = 2 .. 24, 50 and 400000 pairs): the first is the chain of
+    // the step's cells and its two DPP moves, the second its instructions.
+    const double l0 = fp64 ? (weighted ? 60.0 : 62.0) : 43.0;
+    const double l1 = fp64 ? (weighted ? 13.0 : 10.5) : (weighted ? 7.0 : 5.6);
+    const double i0 = fp64 ? (weighted ? 35.0 : 33.0) : (weighted ? 14.0 : 17.0);
+    const double i1 = fp64 ? (weighted ? 12.0 : 10.2) : (weighted ? 6.4 : 4.5);
     // float64 weighted lanes hold two weight vectors: keep them to 17 slots
     const int rmax = fp64 && weighted ? 16 : 1 << 30;
-    double best = -1.0;
+    double best = 0.0;
     for (int t = 0; t < nt; ++t) {
         const int R = tab[t];
         if (R > rmax) continue;
         const int n = (B + R) / (R + 1);  // ceil(B / (R + 1))
         if (n < 1 || n > 64 || (int64_t)n * R > B) continue;
         const int P = 64 / n;
-        const double score = (double)P * B / (k * (R + 1) + 8.0) * lx / (double)(lx + n - 1);
-        if (score > best) {
-            best = score;
+        const double S = R + 1;
+        const double time = pair_launch_ns((n_pairs + P - 1) / P, lx + n - 1, l0 + l1 * S,
+                                           i0 + i1 * S);
+        if (best == 0.0 || time < best) {
+            best = time;
             g->n = n;
             g->a = B - n * R;
             g->P = P;
             g->R = R;
         }
     }
+    if (ns) *ns = best;
     return best > 0.0;
 }
 
@@ -410,7 +444,7 @@ int launch_group_dtw(const PairSpec &ps, Series<T> xs, Series<T> ys, double r, c
     g.kf = bd.ly - bd.lx + bd.off;
     g.nw = n_weights;
     const bool dbl = std::is_same<T, double>::value;
-    if (!group_plan(bd.B, bd.lx, dbl, weights != nullptr, &g))
+    if (!group_plan(bd.B, bd.lx, ps.n_pairs, dbl, weights != nullptr, &g, nullptr))
         return fail(WBX_EUNSUPPORTED, "group kernel: band %d", bd.B);
     return weights ? launch_group_r<T, true>(g.R, ps, xs, ys, g, weights, sq, st)
                    : launch_group_r<T, false>(g.R, ps, xs, ys, g, nullptr, sq, st);

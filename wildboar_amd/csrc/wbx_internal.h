@@ -224,7 +224,17 @@ struct GroupGeo {
     int n, a, P, R;          // lanes per pair, lanes with R + 1 slots, pairs per wave, strip size
     int nw;                  // weight vector length
 };
-bool group_plan(int B, int lx, bool fp64, bool weighted, GroupGeo *g);
+bool group_plan(int B, int lx, int64_t n_pairs, bool fp64, bool weighted, GroupGeo *g, double *ns);
+
+// Estimated ns of a launch of `waves` one-wave blocks that each make `steps`
+// steps: a step takes `alone` ns for a wave that has its SIMD to itself and
+// each further wave on the SIMD adds `share` (its instructions).  With whole
+// waves on the 1024 SIMDs of the chip it is within 15 % of the group and lane
+// kernels at 50 to 400000 pairs.
+inline double pair_launch_ns(int64_t waves, int64_t steps, double alone, double share) {
+    const int64_t deep = (waves + 1023) / 1024;
+    return 5000.0 + (double)steps * (alone + (double)(deep - 1) * share);
+}
 
 // Differentiable DTW / WDTW with band checkpoints (train_seg.hip); mode 0:
 // all pairs, 1: paired.
