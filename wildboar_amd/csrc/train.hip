@@ -25,6 +25,7 @@
 //  k_sum_*           fixed-order sums of per-pair gradients into dX, dY
 //                    (the backward is bitwise deterministic).
 #include "lane_common.h"
+#include "train_small.h"
 
 namespace wbx {
 
@@ -486,6 +487,20 @@ __global__ __launch_bounds__(256) void k_dy_paired(const float *__restrict__ gw,
 constexpr int TRAIN_MAX_BP = 112;
 constexpr int COL_CHUNK = 256;  // x series per column partial: 16 partials for 4096
 
+int64_t sum_cols_part_floats(int64_t nx, int64_t ny, int64_t ly) {
+    return (nx + COL_CHUNK - 1) / COL_CHUNK * ny * ly;
+}
+
+void launch_sum_cols(const float *gw, int64_t nx, int64_t ny, int ly, int lyp, float *part,
+                     float *dY, int64_t ldy_, hipStream_t st) {
+    const unsigned blocks = (unsigned)((ny * ly + 255) / 256);
+    const int nc = (int)((nx + COL_CHUNK - 1) / COL_CHUNK);
+    hipLaunchKernelGGL(k_sum_cols_partial, dim3(blocks, (unsigned)nc), dim3(256), 0, st, gw, nx,
+                       ny, ly, lyp, COL_CHUNK, part);
+    hipLaunchKernelGGL(k_sum_cols_final, dim3(blocks), dim3(256), 0, st, part, nc, ny, ly, dY,
+                       ldy_);
+}
+
 static int train_bp(int B) { return (B + 7) / 8 * 8; }
 
 template <int BP, int U>
@@ -561,7 +576,7 @@ static int train_geo(const wbx_metric *m, int64_t tx, int64_t ty, TrainGeo *out)
 // the column partials.
 struct TrainScratch {
     bool xred;
-    int64_t nbc, nc, xt, pt, gw, yp, gx, xpart, part, total;  // byte offsets / sizes
+    int64_t nbc, xt, pt, gw, yp, gx, xpart, part, total;  // byte offsets / sizes
 };
 
 static TrainScratch train_scratch(int mode, int64_t nx, int64_t ny, int64_t tx, int64_t ty) {
@@ -585,13 +600,12 @@ static TrainScratch train_scratch(int mode, int64_t nx, int64_t ny, int64_t tx, 
     }
     t.xred = ny % 64 == 0;
     t.nbc = t.xred ? ny / 64 : 0;
-    t.nc = (nx + COL_CHUNK - 1) / COL_CHUNK;
     t.gx = o;
     if (!t.xred) o += al(waves * tx * 64 * 4);
     t.xpart = o;
     if (t.xred && t.nbc > 1) o += al(nx * t.nbc * tx * 4);
     t.part = o;
-    o += al(t.nc * ny * ty * 4);
+    o += al(sum_cols_part_floats(nx, ny, ty) * 4);
     t.total = o;
     return t;
 }
@@ -615,6 +629,11 @@ int wbx_dtw_train_sizes(const wbx_metric *metric, int mode, int64_t nx, int64_t 
     int rc = train_geo(metric, tx, ty, &tg);
     if (rc) return rc;
     const int64_t np = mode == 0 ? nx * ny : nx;
+    const Band bd = make_band((int)tx, (int)ty, metric->r);
+    if (small_train_ok(np, bd)) {
+        small_train_sizes(mode, nx, ny, bd, state_bytes, scratch_bytes);
+        return WBX_OK;
+    }
     const int64_t waves = (np + 63) / 64;
     const int64_t planes = waves * tx * 2 * tg.NW * 64 * 4;
     if (state_bytes) *state_bytes = planes + ((np * 4 + 255) / 256) * 256;
@@ -645,6 +664,8 @@ int wbx_dev_dtw_train_forward(const wbx_metric *metric, int mode, const float *X
     uint32_t *dirs = (uint32_t *)state;
     float *sq = (float *)((char *)state + waves * tx * 2 * tg.NW * 64 * 4);
     Series<float> xs{X, x_stride, (int)tx, nullptr}, ys{Y, y_stride, (int)ty, nullptr};
+    const Band bd = make_band((int)tx, (int)ty, metric->r);
+    if (small_train_ok(ps.n_pairs, bd)) return small_train_forward(ps, xs, ys, bd, D, state, st);
     switch (tg.BP) {
 #define FWD_CASE(BPV, UV) \
     case BPV: train_fwd_one<BPV, UV>(ps, xs, ys, tg.g, sq, dirs, st); break;
@@ -678,6 +699,11 @@ int wbx_dev_dtw_train_backward(const wbx_metric *metric, int mode, const float *
     hipStream_t st = (hipStream_t)stream;
     PairSpec ps{mode == 0 ? PAIR_GRID : PAIR_DIAG, mode == 0 ? nx * ny : nx, mode == 0 ? ny : nx,
                 nullptr, nullptr};
+    const Band bd = make_band((int)tx, (int)ty, metric->r);
+    if (small_train_ok(ps.n_pairs, bd))
+        return small_train_backward(ps, Series<float>{X, x_stride, (int)tx, nullptr},
+                                    Series<float>{Y, y_stride, (int)ty, nullptr}, bd, nx, ny, G,
+                                    state, dX, ldx, dY, ldy_, scratch, st);
     const int64_t waves = (ps.n_pairs + 63) / 64;
     const uint32_t *dirs = (const uint32_t *)state;
     const float *sq = (const float *)((const char *)state + waves * tx * 2 * tg.NW * 64 * 4);
@@ -723,10 +749,7 @@ int wbx_dev_dtw_train_backward(const wbx_metric *metric, int mode, const float *
         else if (ts.nbc > 1)
             hipLaunchKernelGGL(k_sum_xpart, dim3(gx_blocks), dim3(256), 0, st, go.xpart, nx, ts.nbc,
                                (int)tx, dX, ldx);
-        hipLaunchKernelGGL(k_sum_cols_partial, dim3(gy_blocks, (unsigned)ts.nc), dim3(256), 0, st,
-                           go.gw, nx, ny, (int)ty, go.lyp, COL_CHUNK, part);
-        hipLaunchKernelGGL(k_sum_cols_final, dim3(gy_blocks), dim3(256), 0, st, part, (int)ts.nc,
-                           ny, (int)ty, dY, ldy_);
+        launch_sum_cols(go.gw, nx, ny, (int)ty, go.lyp, part, dY, ldy_, st);
     } else {
         hipLaunchKernelGGL(k_dy_paired, dim3(gy_blocks), dim3(256), 0, st, go.gw, ny, (int)ty,
                            go.lyp, dY, ldy_);

@@ -1,0 +1,461 @@
+// train_small.hip -- differentiable DTW of few pairs: barycenter steps (one
+// mean against a cluster's series) and other calls that would leave most of
+// the chip idle with one pair per lane (train.hip).
+//
+//  k_small_train     the forward with n = ceil(B / 4) lanes per pair, four
+//                    band slots each, one row behind the lane before
+//                    (group.hip's schedule).  Every lane writes one byte per
+//                    row: which of its four cells took the diagonal (low
+//                    nibble) and the up (high nibble) predecessor.
+//  k_small_backward  one wave per pair.  The path is walked on the scalar
+//                    unit: a row's decision bytes are scalar loads, the exit
+//                    of a row is a bit scan of the bytes at or below the
+//                    current slot.  The rows' column ranges go to LDS and the
+//                    64 lanes form the gradient terms of rows, then columns,
+//                    with the arithmetic and order of k_lane_backtrack.
+//  k_sum_pairs       dX from the per-pair rows.
+//
+// Bound by latency: the chain of cells of a row in the forward, the chain of
+// rows in the walk.  1 x 512 pairs of 256, r = 0.1, against one pair per lane
+// (8 waves): forward 221 -> 26 us, backward 334 -> 51 us.
+#include <type_traits>
+
+#include "train_small.h"
+
+namespace wbx {
+
+namespace {
+
+constexpr int SS = 4;        // slots per lane
+constexpr int SU = 8;        // steps whose loads are issued together
+constexpr int kSmallMaxB = 112;
+constexpr int kSmallMaxLen = 2048;  // LDS of the backward
+// Pairs up to which the small form is used: both forms on 256-step series at
+// B = 49 take the same time at about 20000 pairs (one pair per lane takes
+// 560 us from 64 to 60000 pairs).
+constexpr int64_t kSmallPairs = 16384;
+
+__device__ __forceinline__ float sshr1(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x138,
+                                                      0xF, 0xF, false));
+}
+__device__ __forceinline__ float sshl1(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x130,
+                                                      0xF, 0xF, false));
+}
+
+// c = min3(up, left, dg) + (x - y)^2 with the two decision bits shifted into
+// pd (min came from diag) and pu (from up); see train_cell in train.hip.
+__device__ __forceinline__ float small_cell(float up, float left, float dg, float x, float y,
+                                            uint32_t &pd, uint32_t &pu) {
+    const float m = fminf(fminf(up, left), dg);
+    float c = m, d;
+    uint64_t sa, sb;
+    asm("v_cmp_eq_f32_e64 %[sa], %[c], %[dg]\n\t"
+        "v_cmp_eq_f32_e64 %[sb], %[c], %[up]\n\t"
+        "v_sub_f32_e32 %[d], %[x], %[y]\n\t"
+        "v_fmac_f32_e32 %[c], %[d], %[d]\n\t"
+        "v_addc_co_u32_e64 %[pd], %[sa], %[pd], %[pd], %[sa]\n\t"
+        "v_addc_co_u32_e64 %[pu], %[sb], %[pu], %[pu], %[sb]"
+        : [c] "+v"(c), [pd] "+v"(pd), [pu] "+v"(pu), [d] "=&v"(d), [sa] "=&s"(sa),
+          [sb] "=&s"(sb)
+        : [dg] "v"(dg), [up] "v"(up), [x] "v"(x), [y] "v"(y));
+    return c;
+}
+
+struct SmallGeo {
+    int lx, ly, off, B, kf;
+    int n, P, rb;  // lanes per pair, pairs per wave, decision bytes per row
+};
+
+SmallGeo small_geo(const Band &bd) {
+    SmallGeo g;
+    g.lx = bd.lx;
+    g.ly = bd.ly;
+    g.off = bd.off;
+    g.B = bd.B;
+    g.kf = bd.ly - bd.lx + bd.off;
+    g.n = (bd.B + SS - 1) / SS;
+    g.P = 64 / g.n;
+    g.rb = (g.n + 7) / 8 * 8;
+    return g;
+}
+
+struct SLane {
+    float row[SS];
+    float yw[SS + SU - 1];  // yw[q] = y[yj + q]
+    float pen[SS];          // +inf for slots >= B, else 0: max() keeps them out
+    float l;                // last slot of the lane's last row
+    int r, yj;
+    bool first, last;
+};
+
+// One row of the lane; SEL keeps the state of lanes outside [0, lx).
+template <bool SEL>
+__device__ __forceinline__ uint32_t small_step(SLane &L, int u, float x, int lx) {
+    const bool act = !SEL || (unsigned)(L.r + u) < (unsigned)lx;
+    float left = sshr1(L.l);
+    left = L.first ? WBX_INF_F : left;
+    uint32_t pd = 0, pu = 0;
+    const float c0 = small_cell(L.row[1], left, L.row[0], x, L.yw[u], pd, pu);
+    float Uin = sshl1(SEL && !act ? L.row[0] : c0);
+    Uin = L.last ? WBX_INF_F : Uin;
+    left = c0;
+#pragma unroll
+    for (int m = 1; m < SS; ++m) {
+        float c = small_cell(m == SS - 1 ? Uin : L.row[m + 1], left, L.row[m], x, L.yw[u + m], pd,
+                             pu);
+        c = fmaxf(c, L.pen[m]);
+        L.row[m] = SEL ? (act ? c : L.row[m]) : c;
+        left = c;
+    }
+    L.row[0] = SEL ? (act ? c0 : L.row[0]) : c0;
+    L.l = L.row[SS - 1];
+    // slot m at bit m (they were shifted in from the top)
+    return __brev(pd) >> 28 | (__brev(pu) >> 28) << 4;
+}
+
+__device__ __forceinline__ void small_loads(const float *__restrict__ X,
+                                            const float *__restrict__ Y, int xr, int yc, int lx,
+                                            int ly, float (&xo)[SU], float (&yo)[SU]) {
+    const bool in = xr >= 0 && xr + SU <= lx && yc >= 0 && yc + SU <= ly;
+    if (__ballot(!in) == 0) {  // uniform
+#pragma unroll
+        for (int u = 0; u < SU; u += 4) {
+            const f4a a = *(const f4a *)(X + xr + u);
+            const f4a b = *(const f4a *)(Y + yc + u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                xo[u + e] = a[e];
+                yo[u + e] = b[e];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < SU; ++u) {
+            const int i = xr + u;
+            xo[u] = X[i < 0 ? 0 : (i >= lx ? lx - 1 : i)];
+            yo[u] = ldy(Y, yc + u, ly);
+        }
+    }
+}
+
+__global__ __launch_bounds__(64) void k_small_train(PairSpec ps, Series<float> xs,
+                                                    Series<float> ys, SmallGeo g,
+                                                    double *__restrict__ D,
+                                                    float *__restrict__ sq,
+                                                    unsigned char *__restrict__ dec) {
+    const int lane = threadIdx.x;
+    const int gi = lane / g.n;
+    const int q = lane - gi * g.n;
+    const int64_t p = (int64_t)blockIdx.x * g.P + gi;
+    const bool valid = gi < g.P && p < ps.n_pairs;
+    int64_t a = 0, b = 0;
+    if (valid) decode_pair(ps, p, a, b);
+    const float *__restrict__ X = xs.row(a);
+    const float *__restrict__ Y = ys.row(b);
+    const int lx = g.lx, ly = g.ly, k0 = q * SS;
+    constexpr int W = SS + SU - 1;
+
+    SLane L;
+    L.first = q == 0;
+    L.last = q == g.n - 1;
+#pragma unroll
+    for (int m = 0; m < SS; ++m) {
+        L.row[m] = k0 + m == g.off ? 0.0f : WBX_INF_F;
+        L.pen[m] = k0 + m < g.B ? 0.0f : WBX_INF_F;
+    }
+    L.l = L.row[SS - 1];
+    L.r = -q;
+    L.yj = L.r + k0 - g.off;
+#pragma unroll
+    for (int m = 0; m < W; ++m) L.yw[m] = ldy(Y, L.yj + m, ly);
+    // byte of (row, lane); rows outside [0, lx) are never written
+    unsigned char *out = dec + (valid ? p * lx * g.rb + q : 0);
+
+    const int steps = lx + g.n - 1;
+    float xv[SU], yn[SU];
+    small_loads(X, Y, L.r, L.yj + W, lx, ly, xv, yn);
+    auto group = [&](auto edge) {
+        constexpr bool E = decltype(edge)::value;
+        float xb[SU], yb[SU];
+        small_loads(X, Y, L.r + SU, L.yj + W + SU, lx, ly, xb, yb);
+#pragma unroll
+        for (int u = 0; u < SU; ++u) {
+            const uint32_t bits = small_step<E>(L, u, xv[u], lx);
+            const int r = L.r + u;
+            if (valid && (!E || (unsigned)r < (unsigned)lx))
+                out[(int64_t)r * g.rb] = (unsigned char)bits;
+        }
+#pragma unroll
+        for (int m = 0; m < W - SU; ++m) L.yw[m] = L.yw[m + SU];
+#pragma unroll
+        for (int u = 0; u < SU; ++u) {
+            L.yw[W - SU + u] = yn[u];
+            yn[u] = yb[u];
+            xv[u] = xb[u];
+        }
+        L.r += SU;
+        L.yj += SU;
+    };
+    int s = 0;
+    for (; s < g.n - 1; s += SU) group(std::true_type());
+    for (; s + SU <= lx; s += SU) group(std::false_type());
+    for (; s < steps; s += SU) group(std::true_type());
+
+    if (valid && g.kf >= k0 && g.kf < k0 + SS) {
+        float res = WBX_INF_F;
+#pragma unroll
+        for (int m = 0; m < SS; ++m)
+            if (k0 + m == g.kf) res = L.row[m];
+        sq[p] = res;
+        D[p] = sqrt((double)res);
+    }
+}
+
+// Where a pair's gradient rows go: the output itself where it is the only
+// pair of its series, else its row of the per-pair scratch.
+struct SmallGrad {
+    float *gx;    // gx[(one_b ? a : p) * ldgx + i]
+    float *gy;    // gy[(one_a ? b : p) * ldgy + j]
+    int64_t ldgx, ldgy;
+    int one_b, one_a;
+};
+
+// LDS: x (lx), prefix sums of y (ly + 1, float64), the rows' column ranges
+// (lx), the columns' row ranges (ly).
+size_t small_lds(int lx, int ly) { return (size_t)(ly + 1) * 8 + (size_t)(2 * lx + ly) * 4; }
+
+typedef const uint64_t __attribute__((address_space(4))) *cmask;
+
+// NW: 64-bit decision words per row (rb / 8).
+template <int NW>
+__global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float> xs,
+                                                       Series<float> ys, SmallGeo g,
+                                                       const float *__restrict__ sq,
+                                                       const double *__restrict__ G,
+                                                       const unsigned char *__restrict__ dec,
+                                                       SmallGrad out) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    double *pt = (double *)smem;                   // pt[j] = y[0] + ... + y[j - 1]
+    float *lxv = (float *)(pt + g.ly + 1);
+    uint32_t *rows = (uint32_t *)(lxv + g.lx);     // je << 16 | jx
+    uint32_t *cols = rows + g.lx;                  // last row << 16 | first row
+    const int lane = threadIdx.x;
+    const int64_t p = blockIdx.x;
+    int64_t a, b;
+    decode_pair(ps, p, a, b);
+    const float *__restrict__ X = xs.row(a);
+    const float *__restrict__ Y = ys.row(b);
+    const int lx = g.lx, ly = g.ly, off = g.off, B = g.B;
+    for (int i = lane; i < lx; i += 64) lxv[i] = X[i];
+    if (lane == 0) pt[0] = 0.0;
+    double carry = 0.0;
+    for (int j0 = 0; j0 < ly; j0 += 64) {  // the scan of k_prefix_t
+        const int j = j0 + lane;
+        double s = j < ly ? (double)Y[j] : 0.0;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const double o = __shfl_up(s, d);
+            if (lane >= d) s += o;
+        }
+        s += carry;
+        if (j < ly) pt[j + 1] = s;
+        carry = __shfl(s, 63);
+    }
+
+    // the walk, uniform over the wave: RB rows of words are loaded at a time,
+    // the next RB while these are walked
+    constexpr int RB = NW <= 2 ? 8 : 4;
+    const cmask W = (cmask)(dec + p * lx * g.rb);
+    uint64_t cur[RB][NW], nxt[RB][NW];
+    auto load = [&](uint64_t(&w)[RB][NW], int ih) {
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const int i = ih - r < 0 ? 0 : ih - r;
+#pragma unroll
+            for (int e = 0; e < NW; ++e) w[r][e] = W[(int64_t)i * NW + e];
+        }
+    };
+    load(cur, lx - 1);
+    int k = g.kf;
+    for (int ih = lx - 1; ih >= 0; ih -= RB) {
+        load(nxt, ih - RB);
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const int i = ih - r;
+            if (i < 0) break;
+            const int klo = off - i > 0 ? off - i : 0;
+            int khi = ly - 1 - i + off;
+            if (khi > B - 1) khi = B - 1;
+            if (k > khi) k = khi;
+            // exit: the highest slot <= k whose decision is diag or up.  Slot
+            // k is at bit 8 (k / 4 % 8) + k % 4 (diag, 4 above it up) of word
+            // k / 32.
+            const int wk = k >> 5, bk = (k >> 2 & 7) * 8 + (k & 3);
+            int kx = -1;
+            bool isd = false;
+#pragma unroll
+            for (int e = NW - 1; e >= 0; --e) {
+                uint64_t m = (cur[r][e] | cur[r][e] >> 4) & 0x0f0f0f0f0f0f0f0full;
+                if (e > wk) m = 0;
+                if (e == wk) m &= ((uint64_t)2 << bk) - 1;
+                if (kx < 0 && m != 0) {
+                    const int q = 63 - __builtin_clzll(m);
+                    kx = 32 * e + (q >> 3) * 4 + (q & 3);
+                    isd = (cur[r][e] >> q & 1) != 0;
+                }
+            }
+            // Row 0 ends at column 0 (only left moves there); the other two
+            // are unreachable on a finite path and keep the walk in bounds.
+            if (i == 0 || kx < klo) {
+                kx = klo;
+                isd = false;
+            }
+            if (k < kx) k = kx;
+            const int je = i + k - off, jx = i + kx - off;  // in [0, ly)
+            if (lane == 0) rows[i] = (uint32_t)je << 16 | (uint32_t)jx;
+            k = isd ? kx : kx + 1;
+        }
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+#pragma unroll
+            for (int e = 0; e < NW; ++e) cur[r][e] = nxt[r][e];
+    }
+    __syncthreads();
+
+    const double Dp = sqrt((double)sq[p]);
+    const double coefd = Dp > 0.0 ? G[p] / Dp : 0.0;
+    const float coef = (float)coefd;
+    float *__restrict__ gx = out.gx + (out.one_b ? a : p) * out.ldgx;
+    float *__restrict__ gy = out.gy + (out.one_a ? b : p) * out.ldgy;
+    for (int i = lane; i < lx; i += 64) {
+        const uint32_t v = rows[i];
+        const int jx = v & 0xffff, je = v >> 16;
+        const float xi = lxv[i];
+        gx[i] = (float)(coefd * ((double)(je - jx + 1) * (double)xi - (pt[je + 1] - pt[jx])));
+        // Consecutive rows share at most one column (an up step), so a column
+        // has its first row here unless it is the one shared with the row
+        // above, its last unless shared with the row below.
+        const int above = i > 0 ? (int)(rows[i - 1] >> 16) : -1;
+        const int below = i + 1 < lx ? (int)(rows[i + 1] & 0xffff) : ly;
+        for (int j = jx; j <= je; ++j) {
+            if (j > above) ((uint16_t *)cols)[2 * j] = (uint16_t)i;
+            if (j < below) ((uint16_t *)cols)[2 * j + 1] = (uint16_t)i;
+        }
+    }
+    __syncthreads();
+    for (int j = lane; j < ly; j += 64) {
+        const uint32_t v = cols[j];
+        const int i0 = v & 0xffff, i1 = v >> 16;
+        float sx = lxv[i1];
+        for (int i = i1 - 1; i >= i0; --i) sx += lxv[i];
+        const float cnt = (float)(i1 - i0 + 1);
+        gy[j] = coef * cnt * Y[j] - coef * sx;
+    }
+}
+
+// dX[a][i] = sum over b of gxp[(a ny + b) lx + i]: 64 columns per block, the
+// pairs split over the block's 16 waves, then the waves' sums in order.
+__global__ __launch_bounds__(1024) void k_sum_pairs(const float *__restrict__ gxp, int64_t ny,
+                                                    int lx, float *__restrict__ dX, int64_t ldx) {
+    __shared__ float part[16][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + lane;
+    const int64_t a = blockIdx.y;
+    const int64_t per = (ny + 15) / 16, b0 = w * per, b1 = b0 + per < ny ? b0 + per : ny;
+    float s = 0.0f;
+    if (i < lx) {
+        const float *src = gxp + (a * ny) * lx + i;
+#pragma unroll 8
+        for (int64_t b = b0; b < b1; ++b) s += src[b * lx];
+    }
+    part[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && i < lx) {
+#pragma unroll
+        for (int e = 1; e < 16; ++e) s += part[e][lane];
+        dX[a * ldx + i] = s;
+    }
+}
+
+struct SmallScratch {
+    int64_t gx, gw, part, total;
+};
+
+SmallScratch small_scratch(int mode, int64_t nx, int64_t ny, int lx, int ly) {
+    SmallScratch t{};
+    auto al = [](int64_t v) { return (v + 255) / 256 * 256; };
+    if (mode == 0) {
+        t.gw = ny > 1 ? al(nx * ny * lx * 4) : 0;
+        t.part = t.gw + (nx > 1 ? al(nx * ny * ly * 4) : 0);
+        t.total = t.part + (nx > 1 ? al(sum_cols_part_floats(nx, ny, ly) * 4) : 0);
+    }
+    if (t.total == 0) t.total = 256;
+    return t;
+}
+
+}  // namespace
+
+bool small_train_ok(int64_t n_pairs, const Band &bd) {
+    return n_pairs <= kSmallPairs && bd.B <= kSmallMaxB && bd.lx <= kSmallMaxLen &&
+           bd.ly <= kSmallMaxLen;
+}
+
+void small_train_sizes(int mode, int64_t nx, int64_t ny, const Band &bd, int64_t *state_bytes,
+                       int64_t *scratch_bytes) {
+    const SmallGeo g = small_geo(bd);
+    const int64_t np = mode == 0 ? nx * ny : nx;
+    if (state_bytes) *state_bytes = np * bd.lx * g.rb + (np * 4 + 255) / 256 * 256;
+    if (scratch_bytes) *scratch_bytes = small_scratch(mode, nx, ny, bd.lx, bd.ly).total;
+}
+
+int small_train_forward(const PairSpec &ps, Series<float> xs, Series<float> ys, const Band &bd,
+                        double *D, void *state, hipStream_t st) {
+    const SmallGeo g = small_geo(bd);
+    unsigned char *dec = (unsigned char *)state;
+    float *sq = (float *)(dec + ps.n_pairs * bd.lx * g.rb);
+    hipLaunchKernelGGL(k_small_train, dim3((unsigned)((ps.n_pairs + g.P - 1) / g.P)), dim3(64), 0,
+                       st, ps, xs, ys, g, D, sq, dec);
+    WBX_HIP_CHECK(hipGetLastError());
+    return WBX_OK;
+}
+
+int small_train_backward(const PairSpec &ps, Series<float> xs, Series<float> ys, const Band &bd,
+                         int64_t nx, int64_t ny, const double *G, const void *state, float *dX,
+                         int64_t ldx, float *dY, int64_t ldy_, void *scratch, hipStream_t st) {
+    const SmallGeo g = small_geo(bd);
+    const unsigned char *dec = (const unsigned char *)state;
+    const float *sq = (const float *)(dec + ps.n_pairs * bd.lx * g.rb);
+    const int mode = ps.mode == PAIR_GRID ? 0 : 1;
+    const SmallScratch t = small_scratch(mode, nx, ny, bd.lx, bd.ly);
+    char *sc = (char *)scratch;
+    SmallGrad o;
+    o.one_b = mode == 1 || ny == 1;
+    o.one_a = mode == 1 || nx == 1;
+    o.gx = o.one_b ? dX : (float *)(sc + t.gx);
+    o.ldgx = o.one_b ? ldx : bd.lx;
+    o.gy = o.one_a ? dY : (float *)(sc + t.gw);
+    o.ldgy = o.one_a ? ldy_ : bd.ly;
+    const dim3 grid((unsigned)ps.n_pairs);
+    const size_t lds = small_lds(bd.lx, bd.ly);
+    switch (g.rb / 8) {
+#define WBX_SMALL_BWD(N)                                                                        \
+    case N:                                                                                     \
+        hipLaunchKernelGGL(k_small_backward<N>, grid, dim3(64), lds, st, ps, xs, ys, g, sq, G, \
+                           dec, o);                                                             \
+        break;
+        WBX_SMALL_BWD(1) WBX_SMALL_BWD(2) WBX_SMALL_BWD(3) WBX_SMALL_BWD(4)
+#undef WBX_SMALL_BWD
+        default: return fail(WBX_EUNSUPPORTED, "band %d", bd.B);
+    }
+    if (!o.one_b)
+        hipLaunchKernelGGL(k_sum_pairs, dim3((unsigned)((bd.lx + 63) / 64), (unsigned)nx),
+                           dim3(1024), 0, st, o.gx, ny, bd.lx, dX, ldx);
+    if (!o.one_a)
+        launch_sum_cols(o.gy, nx, ny, bd.ly, bd.ly, (float *)(sc + t.part), dY, ldy_, st);
+    WBX_HIP_CHECK(hipGetLastError());
+    return WBX_OK;
+}
+
+}  // namespace wbx
