@@ -2,22 +2,23 @@
 // mean against a cluster's series) and other calls that would leave most of
 // the chip idle with one pair per lane (train.hip).
 //
-//  k_small_train     the forward with n = ceil(B / 4) lanes per pair, four
-//                    band slots each, one row behind the lane before
+//  k_small_train     the forward with n = ceil(B / S) lanes per pair, S = 2 or
+//                    4 band slots each, one row behind the lane before
 //                    (group.hip's schedule).  Every lane writes one byte per
-//                    row: which of its four cells took the diagonal (low
-//                    nibble) and the up (high nibble) predecessor.
-//  k_small_backward  one wave per pair.  The path is walked on the scalar
-//                    unit: a row's decision bytes are scalar loads, the exit
-//                    of a row is a bit scan of the bytes at or below the
-//                    current slot.  The rows' column ranges go to LDS and the
-//                    64 lanes form the gradient terms of rows, then columns,
-//                    with the arithmetic and order of k_lane_backtrack.
+//                    row: which of its cells took the diagonal predecessor
+//                    (low nibble) and the up (high nibble).
+//  k_small_backward  one wave per pair.  Lane k loads the byte of band slot k,
+//                    two compares give the row's decisions as 64-bit masks in
+//                    SGPRs, and the path is walked there: the exit of a row
+//                    is a count of leading zeros.  The rows' column ranges go
+//                    to LDS and the 64 lanes form the gradient terms of rows,
+//                    then columns, with the arithmetic and order of
+//                    k_lane_backtrack.
 //  k_sum_pairs       dX from the per-pair rows.
 //
 // Bound by latency: the chain of cells of a row in the forward, the chain of
 // rows in the walk.  1 x 512 pairs of 256, r = 0.1, against one pair per lane
-// (8 waves): forward 221 -> 26 us, backward 334 -> 51 us.
+// (8 waves): forward 221 -> 36 us, backward 334 -> 65 us.
 #include <type_traits>
 
 #include "train_small.h"
@@ -26,7 +27,6 @@ namespace wbx {
 
 namespace {
 
-constexpr int SS = 4;        // slots per lane
 constexpr int SU = 8;        // steps whose loads are issued together
 constexpr int kSmallMaxB = 112;
 constexpr int kSmallMaxLen = 2048;  // LDS of the backward
@@ -65,54 +65,61 @@ __device__ __forceinline__ float small_cell(float up, float left, float dg, floa
 
 struct SmallGeo {
     int lx, ly, off, B, kf;
-    int n, P, rb;  // lanes per pair, pairs per wave, decision bytes per row
+    int S, n, P;  // slots per lane, lanes per pair (decision bytes per row), pairs per wave
 };
 
-SmallGeo small_geo(const Band &bd) {
+// Two slots per lane while every wave then has a SIMD to itself (the shorter
+// chain), else four.
+SmallGeo small_geo(const Band &bd, int64_t n_pairs) {
     SmallGeo g;
     g.lx = bd.lx;
     g.ly = bd.ly;
     g.off = bd.off;
     g.B = bd.B;
     g.kf = bd.ly - bd.lx + bd.off;
-    g.n = (bd.B + SS - 1) / SS;
+    g.S = 2;
+    g.n = (bd.B + 1) / 2;
     g.P = 64 / g.n;
-    g.rb = (g.n + 7) / 8 * 8;
+    if ((n_pairs + g.P - 1) / g.P > 1024) {
+        g.S = 4;
+        g.n = (bd.B + 3) / 4;
+        g.P = 64 / g.n;
+    }
     return g;
 }
 
+template <int S>
 struct SLane {
-    float row[SS];
-    float yw[SS + SU - 1];  // yw[q] = y[yj + q]
-    float pen[SS];          // +inf for slots >= B, else 0: max() keeps them out
-    float l;                // last slot of the lane's last row
+    float row[S];
+    float yw[S + SU - 1];  // yw[q] = y[yj + q]
+    float l;               // last slot of the lane's last row
     int r, yj;
     bool first, last;
 };
 
-// One row of the lane; SEL keeps the state of lanes outside [0, lx).
-template <bool SEL>
-__device__ __forceinline__ uint32_t small_step(SLane &L, int u, float x, int lx) {
+// One row of the lane; SEL keeps the state of lanes outside [0, lx).  MB: the
+// place of slot B - 1 in the last lane; its up input is +inf, so whatever
+// the slots past the band hold never enters it.
+template <int S, int MB, bool SEL>
+__device__ __forceinline__ uint32_t small_step(SLane<S> &L, int u, float x, int lx) {
     const bool act = !SEL || (unsigned)(L.r + u) < (unsigned)lx;
     float left = sshr1(L.l);
     left = L.first ? WBX_INF_F : left;
     uint32_t pd = 0, pu = 0;
-    const float c0 = small_cell(L.row[1], left, L.row[0], x, L.yw[u], pd, pu);
-    float Uin = sshl1(SEL && !act ? L.row[0] : c0);
-    Uin = L.last ? WBX_INF_F : Uin;
+    auto up_of = [&](int m, float up) { return m == MB && L.last ? WBX_INF_F : up; };
+    const float c0 = small_cell(up_of(0, L.row[1]), left, L.row[0], x, L.yw[u], pd, pu);
+    const float Uin = sshl1(SEL && !act ? L.row[0] : c0);
     left = c0;
 #pragma unroll
-    for (int m = 1; m < SS; ++m) {
-        float c = small_cell(m == SS - 1 ? Uin : L.row[m + 1], left, L.row[m], x, L.yw[u + m], pd,
-                             pu);
-        c = fmaxf(c, L.pen[m]);
+    for (int m = 1; m < S; ++m) {
+        const float c = small_cell(up_of(m, m == S - 1 ? Uin : L.row[m + 1]), left, L.row[m], x,
+                                   L.yw[u + m], pd, pu);
         L.row[m] = SEL ? (act ? c : L.row[m]) : c;
         left = c;
     }
     L.row[0] = SEL ? (act ? c0 : L.row[0]) : c0;
-    L.l = L.row[SS - 1];
-    // slot m at bit m (they were shifted in from the top)
-    return __brev(pd) >> 28 | (__brev(pu) >> 28) << 4;
+    L.l = L.row[S - 1];
+    return pd | pu << 4;  // slot m at bit S - 1 - m of each nibble
 }
 
 __device__ __forceinline__ void small_loads(const float *__restrict__ X,
@@ -140,6 +147,7 @@ __device__ __forceinline__ void small_loads(const float *__restrict__ X,
     }
 }
 
+template <int S, int MB>
 __global__ __launch_bounds__(64) void k_small_train(PairSpec ps, Series<float> xs,
                                                     Series<float> ys, SmallGeo g,
                                                     double *__restrict__ D,
@@ -154,24 +162,23 @@ __global__ __launch_bounds__(64) void k_small_train(PairSpec ps, Series<float> x
     if (valid) decode_pair(ps, p, a, b);
     const float *__restrict__ X = xs.row(a);
     const float *__restrict__ Y = ys.row(b);
-    const int lx = g.lx, ly = g.ly, k0 = q * SS;
-    constexpr int W = SS + SU - 1;
+    const int lx = g.lx, ly = g.ly, k0 = q * S;
+    constexpr int W = S + SU - 1;
 
-    SLane L;
+    SLane<S> L;
     L.first = q == 0;
     L.last = q == g.n - 1;
 #pragma unroll
-    for (int m = 0; m < SS; ++m) {
-        L.row[m] = k0 + m == g.off ? 0.0f : WBX_INF_F;
-        L.pen[m] = k0 + m < g.B ? 0.0f : WBX_INF_F;
-    }
-    L.l = L.row[SS - 1];
+    for (int m = 0; m < S; ++m) L.row[m] = k0 + m == g.off ? 0.0f : WBX_INF_F;
+    L.l = L.row[S - 1];
     L.r = -q;
     L.yj = L.r + k0 - g.off;
 #pragma unroll
     for (int m = 0; m < W; ++m) L.yw[m] = ldy(Y, L.yj + m, ly);
-    // byte of (row, lane); rows outside [0, lx) are never written
-    unsigned char *out = dec + (valid ? p * lx * g.rb + q : 0);
+    // the wave's bytes start at its first pair; the lane's byte of row r is
+    // n r further (at most 32 pairs of 2048 rows of 56 bytes)
+    unsigned char *__restrict__ wout = dec + (int64_t)blockIdx.x * g.P * lx * g.n;
+    uint32_t at = (uint32_t)(gi * lx * g.n + q + L.r * g.n);  // of row L.r
 
     const int steps = lx + g.n - 1;
     float xv[SU], yn[SU];
@@ -182,10 +189,10 @@ __global__ __launch_bounds__(64) void k_small_train(PairSpec ps, Series<float> x
         small_loads(X, Y, L.r + SU, L.yj + W + SU, lx, ly, xb, yb);
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
-            const uint32_t bits = small_step<E>(L, u, xv[u], lx);
-            const int r = L.r + u;
-            if (valid && (!E || (unsigned)r < (unsigned)lx))
-                out[(int64_t)r * g.rb] = (unsigned char)bits;
+            const uint32_t bits = small_step<S, MB, E>(L, u, xv[u], lx);
+            if (valid && (!E || (unsigned)(L.r + u) < (unsigned)lx))
+                wout[at] = (unsigned char)bits;
+            at += (uint32_t)g.n;
         }
 #pragma unroll
         for (int m = 0; m < W - SU; ++m) L.yw[m] = L.yw[m + SU];
@@ -203,10 +210,10 @@ __global__ __launch_bounds__(64) void k_small_train(PairSpec ps, Series<float> x
     for (; s + SU <= lx; s += SU) group(std::false_type());
     for (; s < steps; s += SU) group(std::true_type());
 
-    if (valid && g.kf >= k0 && g.kf < k0 + SS) {
+    if (valid && g.kf >= k0 && g.kf < k0 + S) {
         float res = WBX_INF_F;
 #pragma unroll
-        for (int m = 0; m < SS; ++m)
+        for (int m = 0; m < S; ++m)
             if (k0 + m == g.kf) res = L.row[m];
         sq[p] = res;
         D[p] = sqrt((double)res);
@@ -226,10 +233,8 @@ struct SmallGrad {
 // (lx), the columns' row ranges (ly).
 size_t small_lds(int lx, int ly) { return (size_t)(ly + 1) * 8 + (size_t)(2 * lx + ly) * 4; }
 
-typedef const uint64_t __attribute__((address_space(4))) *cmask;
-
-// NW: 64-bit decision words per row (rb / 8).
-template <int NW>
+// WIDE: bands of 65 .. 112 slots (two masks per row).
+template <bool WIDE>
 __global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float> xs,
                                                        Series<float> ys, SmallGeo g,
                                                        const float *__restrict__ sq,
@@ -247,7 +252,29 @@ __global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float
     decode_pair(ps, p, a, b);
     const float *__restrict__ X = xs.row(a);
     const float *__restrict__ Y = ys.row(b);
-    const int lx = g.lx, ly = g.ly, off = g.off, B = g.B;
+    const int lx = g.lx, ly = g.ly, off = g.off, B = g.B, n = g.n;
+    // the walk's first rows of decisions, RB rows at a time: lane k holds the
+    // byte of slot k (slots past the band read the last lane's; their bits
+    // are above every slot the walk asks about)
+    constexpr int RB = 16, NM = WIDE ? 2 : 1;
+    const unsigned char *__restrict__ drow = dec + p * lx * n;
+    int dq[NM], sh[NM];
+#pragma unroll
+    for (int e = 0; e < NM; ++e) {
+        const int k = lane + 64 * e;
+        dq[e] = k / g.S < n ? k / g.S : n - 1;
+        sh[e] = g.S - 1 - k % g.S;
+    }
+    uint32_t cur[RB][NM], nxt[RB][NM];
+    auto load = [&](uint32_t(&w)[RB][NM], int ih) {
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const int i = ih - r < 0 ? 0 : ih - r;
+#pragma unroll
+            for (int e = 0; e < NM; ++e) w[r][e] = drow[(uint32_t)(i * n) + (uint32_t)dq[e]];
+        }
+    };
+    load(cur, lx - 1);
     for (int i = lane; i < lx; i += 64) lxv[i] = X[i];
     if (lane == 0) pt[0] = 0.0;
     double carry = 0.0;
@@ -264,21 +291,7 @@ __global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float
         carry = __shfl(s, 63);
     }
 
-    // the walk, uniform over the wave: RB rows of words are loaded at a time,
-    // the next RB while these are walked
-    constexpr int RB = NW <= 2 ? 8 : 4;
-    const cmask W = (cmask)(dec + p * lx * g.rb);
-    uint64_t cur[RB][NW], nxt[RB][NW];
-    auto load = [&](uint64_t(&w)[RB][NW], int ih) {
-#pragma unroll
-        for (int r = 0; r < RB; ++r) {
-            const int i = ih - r < 0 ? 0 : ih - r;
-#pragma unroll
-            for (int e = 0; e < NW; ++e) w[r][e] = W[(int64_t)i * NW + e];
-        }
-    };
-    load(cur, lx - 1);
-    int k = g.kf;
+    int k = g.kf;  // the walk is uniform over the wave
     for (int ih = lx - 1; ih >= 0; ih -= RB) {
         load(nxt, ih - RB);
 #pragma unroll
@@ -289,21 +302,31 @@ __global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float
             int khi = ly - 1 - i + off;
             if (khi > B - 1) khi = B - 1;
             if (k > khi) k = khi;
-            // exit: the highest slot <= k whose decision is diag or up.  Slot
-            // k is at bit 8 (k / 4 % 8) + k % 4 (diag, 4 above it up) of word
-            // k / 32.
-            const int wk = k >> 5, bk = (k >> 2 & 7) * 8 + (k & 3);
+            // exit: the highest slot <= k whose decision is diag or up
+            uint64_t mE[NM], mD[NM];
+#pragma unroll
+            for (int e = 0; e < NM; ++e) {
+                const uint32_t v = cur[r][e] >> sh[e];
+                mE[e] = __ballot((v & 0x11) != 0);
+                mD[e] = __ballot((v & 1) != 0);
+            }
             int kx = -1;
             bool isd = false;
-#pragma unroll
-            for (int e = NW - 1; e >= 0; --e) {
-                uint64_t m = (cur[r][e] | cur[r][e] >> 4) & 0x0f0f0f0f0f0f0f0full;
-                if (e > wk) m = 0;
-                if (e == wk) m &= ((uint64_t)2 << bk) - 1;
-                if (kx < 0 && m != 0) {
-                    const int q = 63 - __builtin_clzll(m);
-                    kx = 32 * e + (q >> 3) * 4 + (q & 3);
-                    isd = (cur[r][e] >> q & 1) != 0;
+            if constexpr (WIDE) {
+                const uint64_t hi = k >= 64 ? mE[1] << (127 - k) : 0;
+                const uint64_t lo = k >= 64 ? mE[0] : mE[0] << (63 - k);
+                if (hi) {
+                    kx = k - __builtin_clzll(hi);
+                    isd = (mD[1] >> (kx - 64) & 1) != 0;
+                } else if (lo) {
+                    kx = (k >= 64 ? 63 : k) - __builtin_clzll(lo);
+                    isd = (mD[0] >> kx & 1) != 0;
+                }
+            } else {
+                const uint64_t t = mE[0] << (63 - k);
+                if (t) {
+                    kx = k - __builtin_clzll(t);
+                    isd = (mD[0] >> kx & 1) != 0;
                 }
             }
             // Row 0 ends at column 0 (only left moves there); the other two
@@ -314,13 +337,13 @@ __global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float
             }
             if (k < kx) k = kx;
             const int je = i + k - off, jx = i + kx - off;  // in [0, ly)
-            if (lane == 0) rows[i] = (uint32_t)je << 16 | (uint32_t)jx;
+            rows[i] = (uint32_t)je << 16 | (uint32_t)jx;  // every lane the same
             k = isd ? kx : kx + 1;
         }
 #pragma unroll
         for (int r = 0; r < RB; ++r)
 #pragma unroll
-            for (int e = 0; e < NW; ++e) cur[r][e] = nxt[r][e];
+            for (int e = 0; e < NM; ++e) cur[r][e] = nxt[r][e];
     }
     __syncthreads();
 
@@ -402,21 +425,35 @@ bool small_train_ok(int64_t n_pairs, const Band &bd) {
            bd.ly <= kSmallMaxLen;
 }
 
+static int64_t small_dec_bytes(int64_t n_pairs, const SmallGeo &g) {
+    return (n_pairs * g.lx * g.n + 255) / 256 * 256;
+}
+
 void small_train_sizes(int mode, int64_t nx, int64_t ny, const Band &bd, int64_t *state_bytes,
                        int64_t *scratch_bytes) {
-    const SmallGeo g = small_geo(bd);
     const int64_t np = mode == 0 ? nx * ny : nx;
-    if (state_bytes) *state_bytes = np * bd.lx * g.rb + (np * 4 + 255) / 256 * 256;
+    const SmallGeo g = small_geo(bd, np);
+    if (state_bytes) *state_bytes = small_dec_bytes(np, g) + (np * 4 + 255) / 256 * 256;
     if (scratch_bytes) *scratch_bytes = small_scratch(mode, nx, ny, bd.lx, bd.ly).total;
 }
 
 int small_train_forward(const PairSpec &ps, Series<float> xs, Series<float> ys, const Band &bd,
                         double *D, void *state, hipStream_t st) {
-    const SmallGeo g = small_geo(bd);
+    const SmallGeo g = small_geo(bd, ps.n_pairs);
     unsigned char *dec = (unsigned char *)state;
-    float *sq = (float *)(dec + ps.n_pairs * bd.lx * g.rb);
-    hipLaunchKernelGGL(k_small_train, dim3((unsigned)((ps.n_pairs + g.P - 1) / g.P)), dim3(64), 0,
-                       st, ps, xs, ys, g, D, sq, dec);
+    float *sq = (float *)(dec + small_dec_bytes(ps.n_pairs, g));
+    const dim3 grid((unsigned)((ps.n_pairs + g.P - 1) / g.P));
+#define WBX_SMALL_FWD(SV, MB)                                                                    \
+    case SV * 8 + MB:                                                                            \
+        hipLaunchKernelGGL((k_small_train<SV, MB>), grid, dim3(64), 0, st, ps, xs, ys, g, D, sq, \
+                           dec);                                                                 \
+        break;
+    switch (g.S * 8 + (bd.B - 1) % g.S) {
+        WBX_SMALL_FWD(2, 0) WBX_SMALL_FWD(2, 1) WBX_SMALL_FWD(4, 0) WBX_SMALL_FWD(4, 1)
+        WBX_SMALL_FWD(4, 2) WBX_SMALL_FWD(4, 3)
+        default: return fail(WBX_EUNSUPPORTED, "band %d", bd.B);
+    }
+#undef WBX_SMALL_FWD
     WBX_HIP_CHECK(hipGetLastError());
     return WBX_OK;
 }
@@ -424,9 +461,9 @@ int small_train_forward(const PairSpec &ps, Series<float> xs, Series<float> ys, 
 int small_train_backward(const PairSpec &ps, Series<float> xs, Series<float> ys, const Band &bd,
                          int64_t nx, int64_t ny, const double *G, const void *state, float *dX,
                          int64_t ldx, float *dY, int64_t ldy_, void *scratch, hipStream_t st) {
-    const SmallGeo g = small_geo(bd);
+    const SmallGeo g = small_geo(bd, ps.n_pairs);
     const unsigned char *dec = (const unsigned char *)state;
-    const float *sq = (const float *)(dec + ps.n_pairs * bd.lx * g.rb);
+    const float *sq = (const float *)(dec + small_dec_bytes(ps.n_pairs, g));
     const int mode = ps.mode == PAIR_GRID ? 0 : 1;
     const SmallScratch t = small_scratch(mode, nx, ny, bd.lx, bd.ly);
     char *sc = (char *)scratch;
@@ -439,16 +476,12 @@ int small_train_backward(const PairSpec &ps, Series<float> xs, Series<float> ys,
     o.ldgy = o.one_a ? ldy_ : bd.ly;
     const dim3 grid((unsigned)ps.n_pairs);
     const size_t lds = small_lds(bd.lx, bd.ly);
-    switch (g.rb / 8) {
-#define WBX_SMALL_BWD(N)                                                                        \
-    case N:                                                                                     \
-        hipLaunchKernelGGL(k_small_backward<N>, grid, dim3(64), lds, st, ps, xs, ys, g, sq, G, \
-                           dec, o);                                                             \
-        break;
-        WBX_SMALL_BWD(1) WBX_SMALL_BWD(2) WBX_SMALL_BWD(3) WBX_SMALL_BWD(4)
-#undef WBX_SMALL_BWD
-        default: return fail(WBX_EUNSUPPORTED, "band %d", bd.B);
-    }
+    if (bd.B > 64)
+        hipLaunchKernelGGL(k_small_backward<true>, grid, dim3(64), lds, st, ps, xs, ys, g, sq, G,
+                           dec, o);
+    else
+        hipLaunchKernelGGL(k_small_backward<false>, grid, dim3(64), lds, st, ps, xs, ys, g, sq, G,
+                           dec, o);
     if (!o.one_b)
         hipLaunchKernelGGL(k_sum_pairs, dim3((unsigned)((bd.lx + 63) / 64), (unsigned)nx),
                            dim3(1024), 0, st, o.gx, ny, bd.lx, dX, ldx);
