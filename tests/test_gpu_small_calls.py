@@ -51,3 +51,23 @@ def test_small_singleton_and_paired(n):
     np.testing.assert_array_equal(got, want + want.T)
     p = device.paired(Xd, Yd, metric="dtw", r=0.1, precision="fp64").cpu().numpy()
     np.testing.assert_array_equal(p, np.diag(oracle.pairwise(Y, X, metric="dtw", r=0.1)))
+
+
+@pytest.mark.parametrize("metric", ["dtw", "euclidean"])
+def test_output_in_the_memory_of_an_input(metric):
+    # the distances then wait until every pair has read its series
+    rng = np.random.default_rng(5)
+    X = rng.standard_normal((300, 64)).cumsum(axis=1)
+    Y = rng.standard_normal((64, 64)).cumsum(axis=1)
+    Xd, Yd = torch.from_numpy(X).cuda(), torch.from_numpy(Y).cuda()
+    want = device.pairwise(Xd, Yd, metric=metric, r=0.1, precision="fp64").clone()
+    got = device.pairwise(Xd, Yd, metric=metric, r=0.1, precision="fp64", out=Xd)
+    assert got.data_ptr() == Xd.data_ptr() and torch.equal(got, want)
+    Sd = Yd.clone()
+    want = device.pairwise(Sd, metric=metric, r=0.1, precision="fp64").clone()
+    assert torch.equal(device.pairwise(Sd, metric=metric, r=0.1, precision="fp64", out=Sd), want)
+    Pd = torch.from_numpy(X).cuda()
+    want = device.paired(Pd, Pd.flip(0), metric=metric, r=0.1, precision="fp64").clone()
+    flat = Pd.view(-1)[:300]
+    assert torch.equal(device.paired(Pd, Pd.flip(0), metric=metric, r=0.1, precision="fp64",
+                                     out=flat), want)

@@ -245,7 +245,7 @@ bool lane64_ok(const DeviceCtx *ctx, const void *weights) {
     return !weights || cached_weights_min(ctx, weights) > 0.0;
 }
 
-// Squared costs of the pairs of ps.  m->kind is EUCLIDEAN, DTW, WDTW or ADTW
+// The pairs of ps (squared costs into sq, or distances to ps.out).  m->kind is EUCLIDEAN, DTW, WDTW or ADTW
 // (the derivative kinds arrive here as DTW / WDTW on slopes); w_fixed > 0
 // replaces every pair's band width.
 template <typename T>
@@ -357,12 +357,28 @@ size_t stage_bytes(int dtype, bool want_double, int64_t n, int64_t len) {
         if (_rc) return _rc; \
     } while (0)
 
+// Whether `n_out` doubles at out share memory with n rows of X: the pair
+// kernels then keep their costs apart until every pair has read its series.
+bool overlaps(const double *out, int64_t n_out, const void *X, int64_t n, int64_t len,
+              int64_t stride, int dtype) {
+    if (!X) return false;
+    const char *o0 = (const char *)out, *o1 = o0 + (size_t)n_out * 8;
+    const int64_t last = stride < 0 ? 0 : (n - 1) * stride, first = stride < 0 ? (n - 1) * stride : 0;
+    const int64_t es = dtype == WBX_F64 ? 8 : 4;
+    const char *x0 = (const char *)X + first * es, *x1 = (const char *)X + (last + len) * es;
+    return o0 < x1 && x0 < o1;
+}
+
 // -------------------------------------------------------------- pairwise
 // Workspace of one pairwise call: staged inputs (when the element type is
-// not the compute type) and the squared cost of every pair.
+// not the compute type).
 struct PairwiseLayout {
     PairSpec ps{};
     size_t o_x = 0, o_y = 0, o_sq = 0, total = 0;
+    // with a cost per pair: what the allocation-free entry point counts
+    // against its scratch, and what a call whose output shares memory with
+    // its inputs needs
+    size_t total_costs = 0;
 };
 
 template <typename T>
@@ -382,8 +398,9 @@ PairwiseLayout pairwise_layout(int dtype, int64_t nx, int64_t tx, int64_t ny, in
     Carve cv;
     L.o_x = cv.take(stage_bytes(dtype, dbl, nx, tx));
     L.o_y = singleton ? 0 : cv.take(stage_bytes(dtype, dbl, ny, ty));
-    L.o_sq = cv.take((size_t)L.ps.n_pairs * sizeof(T));
     L.total = cv.total;
+    L.o_sq = cv.take((size_t)L.ps.n_pairs * sizeof(T));
+    L.total_costs = cv.total;
     return L;
 }
 
@@ -392,18 +409,28 @@ PairwiseLayout pairwise_layout(int dtype, int64_t nx, int64_t tx, int64_t ny, in
 template <typename T>
 int pairwise_run(const PairwiseLayout &L, const wbx_metric *m, int dtype, const void *X,
                  int64_t nx, int64_t xstr, int64_t tx, const void *Y, int64_t ystr, int64_t ty,
-                 bool singleton, const T *w, char *ws, double *out, hipStream_t st, int w_fixed) {
+                 bool singleton, const T *w, char *ws, double *out, bool apart, hipStream_t st,
+                 int w_fixed) {
     Staged<T> sx, sy;
     RC(stage<T>(dtype, X, nx, tx, xstr, ws, L.o_x, &sx, st));
     if (singleton)
         sy = sx;
     else
         RC(stage<T>(dtype, Y, L.ps.ny, ty, ystr, ws, L.o_y, &sy, st));
-    T *sq = (T *)(ws + L.o_sq);
-    RC(run_pairs<T>(m, L.ps, series<T>(sx.ptr, sx.stride, tx), series<T>(sy.ptr, sy.stride, ty), w,
+    if (singleton && nx == 1) return launch_fill_f64(out, 1, 0.0, st);  // no pair
+    PairSpec ps = L.ps;
+    T *sq = nullptr;
+    if (apart) {
+        sq = (T *)(ws + L.o_sq);
+    } else {
+        ps.out = out;
+        ps.ld = L.ps.ny;
+    }
+    RC(run_pairs<T>(m, ps, series<T>(sx.ptr, sx.stride, tx), series<T>(sy.ptr, sy.stride, ty), w,
                     sq, st, w_fixed));
+    if (!apart) return WBX_OK;
     if (singleton) RC(launch_fill_f64(out, nx * nx, 0.0, st));
-    return launch_finish<T>(L.ps, sq, out, singleton ? nx : L.ps.ny, st);
+    return launch_finish<T>(L.ps, sq, out, L.ps.ny, st);
 }
 
 template <typename T>
@@ -411,8 +438,11 @@ int pairwise_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *X,
                   int64_t xstr, int64_t tx, const void *Y, int64_t ny, int64_t ystr, int64_t ty,
                   bool singleton, double *out, hipStream_t st, int w_fixed) {
     const PairwiseLayout L = pairwise_layout<T>(dtype, nx, tx, ny, ty, singleton);
+    const int64_t n_out = nx * L.ps.ny;
+    const bool apart = overlaps(out, n_out, X, nx, tx, xstr, dtype) ||
+                       (!singleton && overlaps(out, n_out, Y, ny, ty, ystr, dtype));
     void *wsp = nullptr;
-    RC(ws_reserve(ctx, L.total, &wsp));
+    RC(ws_reserve(ctx, apart ? L.total_costs : L.total, &wsp));
     const T *w = nullptr;
     if (m->kind == WBX_WDTW) {
         const double *w64;
@@ -421,7 +451,7 @@ int pairwise_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *X,
         w = std::is_same<T, double>::value ? (const T *)w64 : (const T *)w32;
     }
     return pairwise_run<T>(L, m, dtype, X, nx, xstr, tx, Y, ystr, ty, singleton, w, (char *)wsp,
-                           out, st, w_fixed);
+                           out, apart, st, w_fixed);
 }
 
 // -------------------------------------------------------------- argmin
@@ -438,7 +468,6 @@ int argmin_pruned(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *X,
     const size_t o_heap = cv.take((size_t)nx * (size_t)k * 16);
     const size_t o_pa = cv.take((size_t)np * 4);
     const size_t o_pb = cv.take((size_t)np * 4);
-    const size_t o_sq = cv.take((size_t)np * 8);
     const size_t o_cnt = cv.take(8);
     void *wsp = nullptr;
     RC(ws_reserve(ctx, cv.total, &wsp));
@@ -451,7 +480,6 @@ int argmin_pruned(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *X,
     if (m->kind == WBX_WDTW) RC(cached_weights(ctx, tx > ty ? tx : ty, m->g, &w64, &w32));
     double *D64 = (double *)(ws + o_d64);
     int32_t *pa = (int32_t *)(ws + o_pa), *pb = (int32_t *)(ws + o_pb);
-    double *sq = (double *)(ws + o_sq);
     unsigned long long *cnt = (unsigned long long *)(ws + o_cnt);
     wbx_metric m64 = *m;
     m64.precision = WBX_FP64;
@@ -466,10 +494,9 @@ int argmin_pruned(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *X,
         WBX_HIP_CHECK(hipStreamSynchronize(st));
         ctx->prune_evaluated += (int64_t)total;
         if (total == 0) continue;
-        PairSpec pl{PAIR_LIST, (int64_t)total, ny, pa, pb};
+        PairSpec pl{PAIR_LIST, (int64_t)total, ny, pa, pb, D64, ny};
         RC(run_pairs<double>(&m64, pl, series<double>(x64.ptr, x64.stride, tx),
-                             series<double>(y64.ptr, y64.stride, ty), w64, sq, st));
-        RC(launch_finish<double>(pl, sq, D64, ny, st));
+                             series<double>(y64.ptr, y64.stride, ty), w64, nullptr, st));
     }
     return launch_argmin_replay(D64, nx, ny, k, lb, ws + o_heap, idx, dist, st);
 }
@@ -489,9 +516,10 @@ int argmin_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *X, i
     Carve cv;
     const size_t o_x64 = cv.take(stage_bytes(dtype, true, nx, tx));
     const size_t o_y64 = cv.take(stage_bytes(dtype, true, ny, ty));
-    const size_t o_sq64 = cv.take((size_t)np * 8);  // certified: of the candidates
+    // the candidates' squared costs, or every pair's distance
+    const size_t o_sq64 = cv.take((size_t)np * 8);
     const size_t o_heap = cv.take((size_t)nx * (size_t)k * 16);
-    size_t o_d64 = 0, o_x32 = 0, o_y32 = 0, o_sq32 = 0, o_cnt = 0, o_off = 0, o_pa = 0, o_pb = 0,
+    size_t o_x32 = 0, o_y32 = 0, o_sq32 = 0, o_cnt = 0, o_off = 0, o_pa = 0, o_pb = 0,
            o_mx = 0, o_words = 0;
     if (certified) {
         o_x32 = cv.take(stage_bytes(dtype, false, nx, tx));
@@ -503,8 +531,6 @@ int argmin_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *X, i
         o_pb = cv.take((size_t)np * 4);
         o_words = cv.take(argmin_words_bytes(nx, ny));
         o_mx = cv.take(16);  // candidate count, then the |x| max
-    } else {
-        o_d64 = cv.take((size_t)np * 8);
     }
     void *wsp = nullptr;
     RC(ws_reserve(ctx, cv.total, &wsp));
@@ -519,12 +545,10 @@ int argmin_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *X, i
     wbx_metric m64 = *m;
     m64.precision = WBX_FP64;
     if (!certified) {
-        PairSpec ps{PAIR_GRID, np, ny, nullptr, nullptr};
-        double *D64 = (double *)(ws + o_d64);
+        PairSpec ps{PAIR_GRID, np, ny, nullptr, nullptr, sq64, ny};
         RC(run_pairs<double>(&m64, ps, series<double>(x64.ptr, x64.stride, tx),
-                             series<double>(y64.ptr, y64.stride, ty), w64, sq64, st));
-        RC(launch_finish<double>(ps, sq64, D64, ny, st));
-        return launch_argmin_replay(D64, nx, ny, k, lb, ws + o_heap, idx, dist, st);
+                             series<double>(y64.ptr, y64.stride, ty), w64, nullptr, st));
+        return launch_argmin_replay(sq64, nx, ny, k, lb, ws + o_heap, idx, dist, st);
     }
     Staged<float> x32, y32;
     RC(stage<float>(dtype, X, nx, tx, xstr, ws, o_x32, &x32, st));
@@ -1266,18 +1290,20 @@ int wbx_dev_pairwise_noalloc(const wbx_metric *metric, int dtype, const void *X,
     const bool dbl = metric->precision == WBX_FP64;
     const PairwiseLayout L = dbl ? pairwise_layout<double>(dtype, nx, tx, ny, ty, singleton)
                                  : pairwise_layout<float>(dtype, nx, tx, ny, ty, singleton);
-    if (L.total > kScratchBytes)
+    if (L.total_costs > kScratchBytes)
         return fail(WBX_EINVAL,
                     "allocation-free pairwise of %lld x %lld series needs %zu bytes of scratch; "
                     "the maximum is %zu (use wbx_dev_pairwise)",
-                    (long long)nx, (long long)ny, L.total, kScratchBytes);
+                    (long long)nx, (long long)ny, L.total_costs, kScratchBytes);
     hipStream_t st = (hipStream_t)stream;
+    const bool apart = overlaps(out, nx * ny, X, nx, tx, x_stride, dtype) ||
+                       (!singleton && overlaps(out, nx * ny, Y, ny, ty, y_stride, dtype));
     g_no_alloc = true;
     const int rc =
         dbl ? pairwise_run<double>(L, metric, dtype, X, nx, x_stride, tx, Y, y_stride, ty,
-                                   singleton, nullptr, (char *)ws, out, st, 0)
+                                   singleton, nullptr, (char *)ws, out, apart, st, 0)
             : pairwise_run<float>(L, metric, dtype, X, nx, x_stride, tx, Y, y_stride, ty, singleton,
-                                  nullptr, (char *)ws, out, st, 0);
+                                  nullptr, (char *)ws, out, apart, st, 0);
     g_no_alloc = false;
     return rc;
 }
@@ -1294,6 +1320,9 @@ int wbx_dev_paired(const wbx_metric *metric, int dtype, const void *X, int64_t x
     RC(begin(ctx, st));
     // _paired_distance binds its rows to the caller's y: out[i] = D(Y[i], X[i]).
     PairSpec ps{PAIR_DIAG, n, n, nullptr, nullptr};
+    const bool apart = overlaps(out, n, X, n, t, x_stride, dtype) ||
+                       overlaps(out, n, Y, n, t, y_stride, dtype);
+    if (!apart) ps.out = out;
     wbx_metric mm = *metric;
     promote_long(&mm, t);
     int rc = acc64_prepare(ctx, &mm, dtype, {{&X, n, t, &x_stride}, {&Y, n, t, &y_stride}}, st);
@@ -1317,7 +1346,7 @@ int wbx_dev_paired(const wbx_metric *metric, int dtype, const void *X, int64_t x
     Carve cv;
     const size_t o_x = cv.take(stage_bytes(dtype, dbl, n, t));
     const size_t o_y = cv.take(stage_bytes(dtype, dbl, n, t));
-    const size_t o_sq = cv.take((size_t)n * 8);
+    const size_t o_sq = cv.take(apart ? (size_t)n * 8 : 0);
     void *wsp = nullptr;
     rc = ws_reserve(ctx, cv.total, &wsp);
     if (!rc) {
@@ -1333,7 +1362,7 @@ int wbx_dev_paired(const wbx_metric *metric, int dtype, const void *X, int64_t x
                 rc = run_pairs<double>(metric, ps, series<double>(sy.ptr, sy.stride, t),
                                        series<double>(sx.ptr, sx.stride, t), w64,
                                        (double *)(ws + o_sq), st, w_fixed);
-            if (!rc) rc = launch_finish<double>(ps, (double *)(ws + o_sq), out, n, st);
+            if (!rc && apart) rc = launch_finish<double>(ps, (double *)(ws + o_sq), out, n, st);
         } else if (!rc) {
             Staged<float> sx, sy;
             rc = stage<float>(dtype, X, n, t, x_stride, ws, o_x, &sx, st);
@@ -1342,7 +1371,7 @@ int wbx_dev_paired(const wbx_metric *metric, int dtype, const void *X, int64_t x
                 rc = run_pairs<float>(metric, ps, series<float>(sy.ptr, sy.stride, t),
                                       series<float>(sx.ptr, sx.stride, t), w32,
                                       (float *)(ws + o_sq), st, w_fixed);
-            if (!rc) rc = launch_finish<float>(ps, (float *)(ws + o_sq), out, n, st);
+            if (!rc && apart) rc = launch_finish<float>(ps, (float *)(ws + o_sq), out, n, st);
         }
     }
     int rc2 = end(ctx, st);

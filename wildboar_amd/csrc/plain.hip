@@ -38,7 +38,7 @@ __global__ __launch_bounds__(64) void k_plain_dtw(PairSpec ps, Series<T> xs,
     const int w = w_fixed > 0 ? w_fixed : band_w(lx, ly, rr);
     const T res = block_dtw<T, AD>(xs.row(a), lx, ys.row(b), ly, w, weights, buf, buf + cap,
                                    buf + 2 * cap, pen);
-    if (threadIdx.x == 0) sq[p] = res;
+    if (threadIdx.x == 0) put_cost(ps, p, a, b, res, sq);
 }
 
 // A measurement baseline, selected only by the batch plan's policy 2: the
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(64) void k_plain_dtw_padded(PairSpec ps, Series<T> 
         d1 = d0;
         d0 = t;
     }
-    if (tid == 0) sq[p] = res;
+    if (tid == 0) put_cost(ps, p, a, b, res, sq);
 }
 
 template <typename T>
@@ -172,7 +172,7 @@ __device__ __forceinline__ void euclid_acc(float &acc, float v) { acc = __builti
 __device__ __forceinline__ void euclid_acc(double &acc, double v) { acc += v * v; }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_euclid_grid(Series<T> xs, int64_t nx,
+__global__ __launch_bounds__(256) void k_euclid_grid(PairSpec ps, Series<T> xs, int64_t nx,
                                                      Series<T> ys, int64_t ny,
                                                      int t, T *__restrict__ sq) {
     // rows padded to EK + 2: even, so a pair of timesteps is one aligned
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void k_euclid_grid(Series<T> xs, int64_t nx,
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int64_t b = b0 + tx + 16 * j;
-            if (b < ny) sq[a * ny + b] = acc[i][j];
+            if (b < ny) put_cost(ps, a * ny + b, a, b, acc[i][j], sq);
         }
     }
 }
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void k_euclid_pairs(PairSpec ps, Series<T> xs,
         }
         if (dist < min_dist) min_dist = dist;
     }
-    sq[p] = min_dist;
+    put_cost(ps, p, a, b, min_dist, sq);
 }
 
 template <typename T>
@@ -291,7 +291,7 @@ int launch_euclid_pairs(const PairSpec &ps, Series<T> xs, Series<T> ys, T *sq,
         const int64_t nx = ps.n_pairs / ps.ny, ny = ps.ny;
         dim3 grid((unsigned)((ny + EB - 1) / EB), (unsigned)((nx + EB - 1) / EB));
         if (grid.y > 65535) return fail(WBX_EUNSUPPORTED, "too many rows for euclidean tiles");
-        hipLaunchKernelGGL(k_euclid_grid<T>, grid, dim3(256), 0, st, xs, nx, ys, ny, xs.len, sq);
+        hipLaunchKernelGGL(k_euclid_grid<T>, grid, dim3(256), 0, st, ps, xs, nx, ys, ny, xs.len, sq);
     } else {
         dim3 grid((unsigned)((ps.n_pairs + 255) / 256));
         hipLaunchKernelGGL(k_euclid_pairs<T>, grid, dim3(256), 0, st, ps, xs, ys, sq);

@@ -99,6 +99,12 @@ struct PairSpec {
     int64_t n_pairs;
     int64_t ny;  // GRID: columns; TRIANGLE: n
     const int32_t *pa, *pb;
+    // Where the distances go, in the driver's layout (NULL: the kernels leave
+    // squared costs in pair order): rows of ld values, GRID and DIAG in pair
+    // order, LIST at (a, b), TRIANGLE at both (a, b) and (b, a) with the
+    // diagonal.
+    double *out = nullptr;
+    int64_t ld = 0;
 };
 
 __host__ __device__ inline void decode_pair(const PairSpec &ps, int64_t p,
@@ -127,6 +133,31 @@ __host__ __device__ inline void decode_pair(const PairSpec &ps, int64_t p,
             a = ps.pa[p];
             b = ps.pb[p];
             break;
+    }
+}
+
+// The result of pair p = (a, b): its squared cost, or its distance in place.
+// The pair kernels end with it: a separate pass over the costs would cost
+// another launch and, on large matrices, reading them back.
+template <typename T>
+__device__ __forceinline__ void put_cost(const PairSpec &ps, int64_t p, int64_t a, int64_t b, T c,
+                                         T *__restrict__ sq) {
+    if (!ps.out) {
+        sq[p] = c;
+        return;
+    }
+    const double v = sqrt((double)c);
+    if (ps.mode == PAIR_TRIANGLE) {
+        ps.out[a * ps.ld + b] = v;
+        ps.out[b * ps.ld + a] = v;
+        if (b == a + 1) {
+            ps.out[a * ps.ld + a] = 0.0;
+            if (b == ps.ny - 1) ps.out[b * ps.ld + b] = 0.0;
+        }
+    } else if (ps.mode == PAIR_LIST) {
+        ps.out[a * ps.ld + b] = v;
+    } else {
+        ps.out[p] = v;
     }
 }
 
