@@ -997,7 +997,7 @@ int scaled_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void *S,
     Carve cv;
     const size_t o_x = cv.take(stage_bytes(dtype, true, n, t));
     const size_t o_s = cv.take(stage_bytes(dtype, true, 1, total));
-    const size_t o_k = cv.take(scaled_ws_bytes(mm.kind, hl.data(), n_s, total, n, t));
+    const size_t o_k = cv.take(scaled_ws_bytes(mm.kind, mm.r, hl.data(), n_s, total, n, t));
     void *wsp = nullptr;
     RC(ws_reserve(ctx, cv.total, &wsp));
     char *ws = (char *)wsp;

@@ -10,7 +10,7 @@
 // std of a running scan, ex += x[k], ex2 += x[k]^2 and, after window I,
 // ex -= x[I], ex2 -= x[I]^2; mean = ex / L, std = sqrt(ex2 / L - mean^2)
 // (1.0 when that is <= 0).  The rounding of those sums depends on every
-// earlier step, so k_window_stats_all replays the scan, one thread per
+// earlier step, so k_window_sums_all replays the scan, one thread per
 // (series, pattern length).
 //
 // Cascade.  Per window the reference computes, in this order, LB_Kim
@@ -175,20 +175,20 @@ __global__ __launch_bounds__(64) void k_scaled_euclid(ScaledTask a) {
 }
 
 // LB_Kim of the reference (constant_lower_bound), in full, on the
-// normalised window zx[k * 64] (the same quotients the reference forms);
-// L >= 3.
-__device__ double scaled_kim(const double *__restrict__ z, const double *__restrict__ zx, int L) {
-    const double tx0 = zx[0], ty0 = zx[(int64_t)(L - 1) * 64];
+// normalised window zx(k) (the same quotients the reference forms); L >= 3.
+template <typename Z>
+__device__ __forceinline__ double scaled_kim(const double *__restrict__ z, Z zx, int L) {
+    const double tx0 = zx(0), ty0 = zx(L - 1);
     const double sx0 = z[0], sy0 = z[L - 1];
     double d = sqd(tx0, sx0) + sqd(ty0, sy0);
-    const double tx1 = zx[64], sx1 = z[1];
+    const double tx1 = zx(1), sx1 = z[1];
     d += dmin(dmin(sqd(tx1, sx0), sqd(tx0, sx1)), sqd(tx1, sx1));
-    const double ty1 = zx[(int64_t)(L - 2) * 64], sy1 = z[L - 2];
+    const double ty1 = zx(L - 2), sy1 = z[L - 2];
     d += dmin(dmin(sqd(ty1, sy1), sqd(ty0, sy1)), sqd(ty1, sy1));
-    const double tx2 = zx[128], sx2 = z[2];
+    const double tx2 = zx(2), sx2 = z[2];
     d += dmin(dmin(dmin(sqd(tx0, sx2), dmin(sqd(tx1, sx2), sqd(tx2, sx2))), sqd(tx2, sx1)),
               sqd(tx2, sx0));
-    const double ty2 = zx[(int64_t)(L - 3) * 64], sy2 = z[L - 3];
+    const double ty2 = zx(L - 3), sy2 = z[L - 3];
     d += dmin(dmin(dmin(sqd(ty0, sy2), dmin(sqd(ty1, sy2), sqd(ty2, sy2))), sqd(ty2, sy1)),
               sqd(ty2, sy0));
     return d;
@@ -243,7 +243,8 @@ __device__ double scaled_bounds(const ScaledTask &a, const double *__restrict__ 
             cb[(int64_t)(m0 - u) * 64] = acc;
         }
     }
-    const double T = L >= 3 ? scaled_kim(z, zx, L) : 0.0;
+    const double T =
+        L >= 3 ? scaled_kim(z, [&](int k) { return zx[(int64_t)k * 64]; }, L) : 0.0;
     return dmax(dmax(T, lk), lk2);
 }
 
@@ -293,8 +294,9 @@ __device__ __forceinline__ double srow(double (&row)[BP], const double *yw, doub
 // Banded DTW (|i - j| <= rw) of z (rows) against the normalised window
 // (columns) in registers; D = cell (L-1, L-1), M = max over rows i with
 // i + rw < L - 1 of v_i = rowmin_i + cb[i * 64], A = the first v_i >= th
-// (the value the reference's abandoned DTW returns), else D.
-template <int BP, int U>
+// (the value the reference's abandoned DTW returns), else D; without TH no
+// threshold is looked at (A = D) and the rows have no branch between them.
+template <int BP, int U, bool TH>
 __device__ __forceinline__ void scaled_cost(const double *__restrict__ z, int L,
                                             const double *__restrict__ zx, int rw, int B,
                                             const double *__restrict__ cb, double th, double &D,
@@ -309,27 +311,38 @@ __device__ __forceinline__ void scaled_cost(const double *__restrict__ z, int L,
     for (int q = 0; q < 8; ++q) pen[q] = (BP - 8 + q >= B) ? WBX_INF_D : -WBX_INF_D;
     double yw[W];
 #pragma unroll
-    for (int m = 0; m < W; ++m) yw[m] = ldz(zx, m - off, L);
+    for (int m = 0; m < W; ++m) {
+        yw[m] = ldz(zx, m - off, L);
+        // four loads at a time: an address pair each while they are in flight
+        if ((m & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     const int last = L - 1 - rw;  // rows i < last are checked against cb
     M = -WBX_INF_D;
     bool ab = false;
     A = WBX_INF_D;
-    auto check = [&](double v) {
-        M = dmax(M, v);
-        if (!ab && v >= th) {
-            ab = true;
-            A = v;
+    auto check = [&](int i, double v) {
+        if constexpr (TH) {
+            if (i < last) {
+                M = dmax(M, v);
+                if (!ab && v >= th) {
+                    ab = true;
+                    A = v;
+                }
+            }
+        } else {
+            M = dmax(M, i < last ? v : -WBX_INF_D);
         }
     };
     double rm = srow<BP>(row, yw, z[0], pen);
-    if (0 < last) check(rm + cb[0]);
+    check(0, rm + (0 < last ? cb[0] : 0.0));
 #pragma unroll
     for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
     yw[W - 1] = ldz(zx, 1 - off + W - 1, L);
     const int rem = (L - 1) % U;
     for (int i = 1; i <= rem; ++i) {
         rm = srow<BP>(row, yw, z[i], pen);
-        if (i < last) check(rm + cb[(int64_t)i * 64]);
+        check(i, rm + (i < last ? cb[(int64_t)i * 64] : 0.0));
 #pragma unroll
         for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
         yw[W - 1] = ldz(zx, i + 1 - off + W - 1, L);
@@ -345,7 +358,7 @@ __device__ __forceinline__ void scaled_cost(const double *__restrict__ z, int L,
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             rm = srow<BP>(row, yw + u, zv[u], pen);
-            if (i0 + u < last) check(rm + cv[u]);
+            check(i0 + u, rm + cv[u]);
         }
 #pragma unroll
         for (int m = 0; m < W - U; ++m) yw[m] = yw[m + U];
@@ -416,7 +429,7 @@ __global__ __launch_bounds__(64) void k_scaled_dtw(ScaledTask a, ScaledItems it,
                                        a.X + ii * a.xstride + sc, a.elo + ii * a.t + sc,
                                        a.eup + ii * a.t + sc, mu, sd, cb, zx);
         double D, M, A;
-        scaled_cost<BP, U>(a.zs + so, L, zx, a.rw, a.B, cb, a.th, D, M, A);
+        scaled_cost<BP, U, true>(a.zs + so, L, zx, a.rw, a.B, cb, a.th, D, M, A);
         scaled_store(a, it, q, ii, s, nwin, T, M, D, A, T);
     }
 }
@@ -502,6 +515,342 @@ __global__ __launch_bounds__(64) void k_scaled_accept(ScaledTask a, ScaledItems 
     }
 }
 
+// ------------------------------------------------ pruned search
+// One wave per (series, pattern).  The acceptance rule needs T(I) < best, and
+// after any window J was considered best <= T(J) (an accepted window sets it
+// to D <= T, a rejected one has T >= best).  So a window I whose bound
+// max(LK, LK2) <= T(I) reaches an upper bound of some earlier window's T is
+// rejected by the reference, and its DTW is not needed.  Nor are LK, LK2 and
+// the abandon values M of the others: each is at most D up to the rounding of
+// sums of L terms (LB_Keogh against an envelope as wide as the band, a row
+// minimum plus the terms of columns the path has still to visit), so with
+// D+ = D (1 + 1e-9) + 1e-9 a window is rejected if D >= best or K >= best and
+// accepted if D+ < best (K, the LB_Kim as the reference writes it, may exceed
+// D and is computed exactly); max(K, D+) bounds T from above.  A window
+// between the two sends its whole task to k_scaled_search_exact, which
+// computes T itself.  The wave
+//   - computes (K, D) of 64 windows spread over the series,
+//   - goes through the others 64 at a time with the two LB_Keogh sums (one
+//     product per value instead of a division, a relative and absolute 1e-9
+//     taken off for it) and collects those below the smallest spread T before
+//     them and the best so far,
+//   - computes (K, D) of 64 collected windows together, stops them when every
+//     row minimum has reached its window's bound, and replays the acceptance
+//     over these and the spread ones in window order.
+// Of random-walk windows 29 % pass the bounds and 7 % have D below the spread
+// T.  Bound by float64 VALU: 32 patterns of 64 .. 128 over 200 series of 1024,
+// r = 0.1, 3.7 ms a call, 16.8 ms with every window's T.
+struct SearchPattern {
+    int64_t goff;  // offset of its length's window statistics
+    int64_t eoff;  // offset of its warp width's series envelopes
+    int32_t j, L, rw;
+};
+
+struct SearchArgs {
+    ScaledTask a;  // X, xstride, t, c0, cn, zs / zl / zu, n_s, dist, idx
+    const SearchPattern *pats;
+    int64_t n_tasks;  // patterns of the launch times cn
+    const double *wmean, *wstd, *elo, *eup;
+    const int64_t *s_off;
+    int *undecided;  // per task: left to k_scaled_search_exact
+};
+
+// The search proper over one task's windows, shared by the two kernels.
+// eval(s, thr, T, D): the values of window s per lane, T an upper bound of
+// the reference's T, D its DTW, or anything >= thr in both once the DTW is
+// known to reach thr.  accept(T, D, best): 1 accepted, 0 rejected, -1 not
+// decided.  Returns false where accept could not decide.
+template <typename Eval, typename Accept>
+__device__ __forceinline__ bool search_task(const ScaledTask &a, int *queue,
+                                            const double *__restrict__ z,
+                                            const double *__restrict__ zl,
+                                            const double *__restrict__ zu,
+                                            const double *__restrict__ x,
+                                            const double *__restrict__ el,
+                                            const double *__restrict__ eu,
+                                            const double *__restrict__ wm,
+                                            const double *__restrict__ wsd, Eval eval,
+                                            Accept decide, double &best, int &bi) {
+    const int lane = threadIdx.x, L = a.L, nwin = a.t - L + 1;
+    // the spread windows lane * step; upre = the smallest T up to the lane's
+    const int step = (nwin + 63) / 64, sw = lane * step;
+    double sT = WBX_INF_D, sD = WBX_INF_D, upre = WBX_INF_D;
+    best = WBX_INF_D;
+    bi = -1;
+    int next_spread = 0, nq = 0, b0 = 0;
+    bool ok = true;
+    auto accept = [&](double T, double D, int s) {
+        const int v = decide(T, D, best);
+        if (v < 0) ok = false;
+        if (v > 0) {
+            best = D;
+            bi = s;
+        }
+    };
+    // spread windows before window s, in order
+    auto accept_spread = [&](int s) {
+        while (next_spread < 64 && next_spread * step < s && next_spread * step < nwin) {
+            accept(__shfl(sT, next_spread), __shfl(sD, next_spread), next_spread * step);
+            ++next_spread;
+        }
+    };
+    for (bool first = true;; first = false) {
+        int s = sw < nwin ? sw : 0;
+        double lim = WBX_INF_D;
+        if (!first) {
+            while (nq < 64 && b0 < nwin) {
+                const int sb = b0 + lane;
+                const int sc = sb < nwin ? sb : nwin - 1;
+                const bool want = sb < nwin && sb % step != 0;  // not a spread one
+                // the spread windows before sb are those of lanes up to
+                // (sb - 1) / step
+                const double thr = dmin(__shfl(upre, sc > 0 ? (sc - 1) / step : 0), best);
+                const double mu = wm[sc], inv = 1.0 / wsd[sc];
+                double lk = 0.0, lk2 = 0.0;
+                bool below = want;
+                for (int k0 = 0; k0 < L; k0 += 16) {
+                    const int k1 = k0 + 16 < L ? k0 + 16 : L;
+#pragma unroll 4
+                    for (int k = k0; k < k1; ++k) {
+                        const double v = (x[sc + k] - mu) * inv;
+                        const double d = dmax(dmax(v - zu[k], zl[k] - v), 0.0);
+                        lk += d * d;
+                        const double us = (eu[sc + k] - mu) * inv, ls = (el[sc + k] - mu) * inv;
+                        const double d2 = dmax(dmax(z[k] - us, ls - z[k]), 0.0);
+                        lk2 += d2 * d2;
+                    }
+                    below = want && !(dmax(lk, lk2) * (1.0 - 1e-9) - 1e-9 >= thr);
+                    if (__ballot(below) == 0) break;  // no window of the 64 is left
+                }
+                const uint64_t keep = __ballot(below);
+                if (below) queue[nq + __popcll(keep & (((uint64_t)1 << lane) - 1))] = sb;
+                nq += __popcll(keep);
+                b0 += 64;
+                __syncthreads();
+            }
+            if (nq == 0) break;
+            s = queue[lane < nq ? lane : 0];
+            lim = dmin(__shfl(upre, s > 0 ? (s - 1) / step : 0), best);
+        }
+        double T, D;
+        eval(s, lim, T, D);
+        if (first) {
+            if (sw < nwin) {
+                sT = T;
+                sD = D;
+            }
+            upre = sT;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const double o = __shfl_up(upre, d);
+                if (lane >= d) upre = dmin(upre, o);
+            }
+            continue;
+        }
+        const int count = nq < 64 ? nq : 64;
+        // only windows below the bound at their place can be accepted
+        uint64_t cand = __ballot(lane < count && D < best);
+        while (cand) {
+            const int l = __builtin_ctzll(cand);
+            cand &= cand - 1;
+            const int sl = __shfl(s, l);
+            accept_spread(sl);
+            accept(__shfl(T, l), __shfl(D, l), sl);
+        }
+        if (!ok) return false;
+        const int rest = queue[64 + lane];
+        __syncthreads();
+        queue[lane] = rest;
+        nq -= count;
+        __syncthreads();
+    }
+    accept_spread(nwin);
+    return ok;
+}
+
+// Banded DTW (|i - j| <= rw, B = 2 rw + 1) of z against the window x of L
+// values, each (x[j] - mu) / sd normalised as it enters the band, in
+// registers: the values scaled_cost computes, without scratch.  +inf once
+// every lane's row minimum has reached its lim (row minima only grow).
+template <int BP, int U>
+__device__ __forceinline__ double window_cost(const double *__restrict__ z, int L,
+                                              const double *__restrict__ x, double mu, double sd,
+                                              int rw, int B, double lim) {
+    constexpr int W = BP + U - 1;
+    const int off = rw;
+    auto ld = [&](int j) { return x[j < 0 ? 0 : (j >= L ? L - 1 : j)]; };
+    auto norm = [&](double v, int j) {
+        const double q = (v - mu) / sd;
+        return (unsigned)j < (unsigned)L ? q : WBX_INF_D;
+    };
+    double row[BP];
+#pragma unroll
+    for (int k = 0; k < BP; ++k) row[k] = (k == off) ? 0.0 : WBX_INF_D;
+    double pen[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) pen[q] = (BP - 8 + q >= B) ? WBX_INF_D : -WBX_INF_D;
+    double yw[W];
+#pragma unroll
+    for (int m = 0; m < W; ++m) {
+        yw[m] = norm(ld(m - off), m - off);
+        if (m & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    auto cells = [&](const double *y, double xi) {
+        double left = WBX_INF_D;
+#pragma unroll
+        for (int k = 0; k < BP; ++k) {
+            const double up = (k + 1 < BP) ? row[k + 1] : WBX_INF_D;
+            const double m = dmin(dmin(up, left), row[k]);
+            const double v = xi - y[k];
+            const double c = m + v * v;
+            row[k] = c;
+            left = c;
+        }
+#pragma unroll
+        for (int q = 1; q < 8; ++q) row[BP - 8 + q] = fmax(row[BP - 8 + q], pen[q]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int rem = L % U;
+    for (int i = 0; i < rem; ++i) {
+        cells(yw, z[i]);
+#pragma unroll
+        for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
+        yw[W - 1] = norm(ld(i + 1 - off + W - 1), i + 1 - off + W - 1);
+    }
+    double xn[U];  // raw values of the next group's window entries
+#pragma unroll
+    for (int u = 0; u < U; ++u) xn[u] = ld(rem - off + W + u);
+    for (int i0 = rem; i0 < L; i0 += U) {
+        const int jn = i0 - off + W;
+        double yn[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            yn[u] = norm(xn[u], jn + u);
+            xn[u] = ld(jn + U + u);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) cells(yw + u, z[i0 + u]);
+#pragma unroll
+        for (int m = 0; m < W - U; ++m) yw[m] = yw[m + U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) yw[W - U + u] = yn[u];
+        if (((i0 - rem) / U & 3) == 3) {  // every fourth group
+            double rm = row[0];
+#pragma unroll
+            for (int k = 1; k < BP; ++k) rm = dmin(rm, row[k]);
+            if (__ballot(!(rm >= lim)) == 0) return WBX_INF_D;
+        }
+    }
+    double res = WBX_INF_D;
+#pragma unroll
+    for (int k = 0; k < BP; ++k)
+        if (k == off) res = row[k];
+    return res;
+}
+
+// A task's pointers, from its index.
+struct SearchView {
+    ScaledTask a;
+    int j;
+    int64_t ii;
+    const double *z, *zl, *zu, *x, *el, *eu, *wm, *wsd;
+};
+
+__device__ __forceinline__ SearchView search_view(const SearchArgs &g, int64_t task) {
+    SearchView v;
+    const int64_t pi = task / g.a.cn;
+    v.ii = task - pi * g.a.cn;
+    const SearchPattern sp = g.pats[pi];
+    v.a = g.a;
+    v.a.L = sp.L;
+    v.a.rw = sp.rw;
+    v.j = sp.j;
+    const int64_t so = g.s_off[sp.j], nwin = g.a.t - sp.L + 1;
+    v.z = g.a.zs + so;
+    v.zl = g.a.zl + so;
+    v.zu = g.a.zu + so;
+    v.x = g.a.X + v.ii * g.a.xstride;
+    v.el = g.elo + sp.eoff + v.ii * g.a.t;
+    v.eu = g.eup + sp.eoff + v.ii * g.a.t;
+    v.wm = g.wmean + sp.goff + v.ii * nwin;
+    v.wsd = g.wstd + sp.goff + v.ii * nwin;
+    return v;
+}
+
+__device__ __forceinline__ void search_result(const SearchArgs &g, const SearchView &v,
+                                              double best, int bi) {
+    if (threadIdx.x == 0) {
+        const int64_t o = (g.a.c0 + v.ii) * g.a.n_s + v.j;
+        g.a.dist[o] = sqrt(best);
+        g.a.idx[o] = bi >= 0 ? bi : 0;
+    }
+}
+
+// Waves per SIMD the registers are held to (float64 row and window).
+constexpr int search_waves(int BP) { return BP <= 8 ? 4 : BP <= 16 ? 3 : BP <= 40 ? 2 : 1; }
+
+template <int BP, int U>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(search_waves(BP)))) void
+k_scaled_search(SearchArgs g) {
+    __shared__ int queue[128];
+    for (int64_t task = blockIdx.x; task < g.n_tasks; task += gridDim.x) {
+        const SearchView v = search_view(g, task);
+        const int L = v.a.L, rw = v.a.rw;
+        auto eval = [&](int s, double lim, double &T, double &D) {
+            const double mu = v.wm[s], sd = v.wsd[s];
+            const double *__restrict__ xw = v.x + s;
+            D = window_cost<BP, U>(v.z, L, xw, mu, sd, rw, 2 * rw + 1, lim);
+            const double K =
+                L >= 3 ? scaled_kim(v.z, [&](int k) { return (xw[k] - mu) / sd; }, L) : 0.0;
+            T = dmax(K, D * (1.0 + 1e-9) + 1e-9);
+        };
+        auto decide = [&](double T, double D, double best) {
+            // T = max(K, D+): below best it is accepted, whatever LK, LK2, M
+            if (!(D < best)) return 0;
+            if (T < best || best == WBX_INF_D) return 1;
+            // K >= best rejects; D+ >= best does not tell
+            return D * (1.0 + 1e-9) + 1e-9 < best ? 0 : -1;
+        };
+        double best;
+        int bi;
+        const bool ok = search_task(v.a, queue, v.z, v.zl, v.zu, v.x, v.el, v.eu, v.wm, v.wsd, eval,
+                                    decide, best, bi);
+        if (ok) search_result(g, v, best, bi);
+        if (threadIdx.x == 0) g.undecided[task] = ok ? 0 : 1;
+        __syncthreads();  // the queue is reused
+    }
+}
+
+// The tasks the search left undecided, with T itself.
+template <int BP, int U>
+__global__ __launch_bounds__(64) void k_scaled_search_exact(SearchArgs g,
+                                                            double *__restrict__ scratch,
+                                                            int64_t per_lane) {
+    __shared__ int queue[128];
+    double *__restrict__ cb = scratch + (int64_t)blockIdx.x * per_lane * 64 + threadIdx.x;
+    for (int64_t task = blockIdx.x; task < g.n_tasks; task += gridDim.x) {
+        if (g.undecided[task] == 0) continue;  // uniform
+        const SearchView v = search_view(g, task);
+        const int L = v.a.L, rw = v.a.rw;
+        double *__restrict__ zx = cb + (int64_t)2 * (L - rw - 1) * 64;
+        auto eval = [&](int s, double, double &T, double &D) {
+            double M, A;
+            T = scaled_bounds(v.a, v.z, v.zl, v.zu, v.x + s, v.el + s, v.eu + s, v.wm[s], v.wsd[s],
+                              cb, zx);
+            scaled_cost<BP, U, false>(v.z, L, zx, rw, 2 * rw + 1, cb, WBX_INF_D, D, M, A);
+            T = dmax(dmax(T, M), D);
+        };
+        auto decide = [&](double T, double, double best) { return T < best ? 1 : 0; };
+        double best;
+        int bi;
+        search_task(v.a, queue, v.z, v.zl, v.zu, v.x, v.el, v.eu, v.wm, v.wsd, eval, decide, best,
+                    bi);
+        search_result(g, v, best, bi);
+        __syncthreads();  // the queue is reused
+    }
+}
+
 // ------------------------------------------------ wrapped metrics
 // ScaledSubsequenceMetricWrap (_cdistance.pyx:470-567) around WeightedDtw-,
 // DerivativeDtw-, WeightedDerivativeDtw- and AmercingDtwMetric: every window
@@ -555,7 +904,7 @@ __device__ void incstats_row(const double *__restrict__ x, int t, int L, double 
     }
 }
 
-// One thread per (group, series), laid out as k_window_stats_all.
+// One thread per (group, series), laid out as k_window_sums_all.
 __global__ __launch_bounds__(64) void k_incstats_all(const double *__restrict__ X, int64_t cn,
                                                      int64_t stride, int t, int n_groups,
                                                      const int *__restrict__ lens,
@@ -685,15 +1034,19 @@ __global__ __launch_bounds__(64) void k_scaled_wrap(ScaledTask a, ScaledItems it
     }
 }
 
-// Window statistics of every pattern length at once: thread (g, i) replays
-// the scan of series i for length lens[g] into mean / sdev + goff[g]
-// (rows of t - lens[g] + 1).
-__global__ __launch_bounds__(64) void k_window_stats_all(const double *__restrict__ X, int64_t cn,
-                                                         int64_t stride, int t, int n_groups,
-                                                         const int *__restrict__ lens,
-                                                         const int64_t *__restrict__ goff,
-                                                         double *__restrict__ mean,
-                                                         double *__restrict__ sdev) {
+// Window statistics of every pattern length at once.  The running sums are a
+// chain of additions whose rounding depends on every earlier step: thread
+// (g, i) replays it for series i and length lens[g] and leaves the sums of
+// each window in mean / sdev + goff[g] (rows of t - lens[g] + 1); the
+// quotients and square roots follow in a pass of their own over all windows
+// (25 lengths of 200 series of 1024: 335 us in one kernel, 192 us in two).
+// The loads of 8 steps are issued together.
+__global__ __launch_bounds__(64) void k_window_sums_all(const double *__restrict__ X, int64_t cn,
+                                                        int64_t stride, int t, int n_groups,
+                                                        const int *__restrict__ lens,
+                                                        const int64_t *__restrict__ goff,
+                                                        double *__restrict__ mean,
+                                                        double *__restrict__ sdev) {
     const int64_t id = (int64_t)blockIdx.x * 64 + threadIdx.x;
     if (id >= cn * n_groups) return;
     const int64_t g = id / cn, i = id - g * cn;
@@ -702,22 +1055,56 @@ __global__ __launch_bounds__(64) void k_window_stats_all(const double *__restric
     const double *__restrict__ x = X + i * stride;
     double *__restrict__ mo = mean + goff[g] + i * nwin;
     double *__restrict__ so = sdev + goff[g] + i * nwin;
-    const double dl = (double)L;
     double ex = 0.0, ex2 = 0.0;
-    for (int k = 0; k < t; ++k) {
-        const double v = x[k];
-        ex += v;
-        ex2 += v * v;
-        if (k >= L - 1) {
-            const int I = k - (L - 1);
-            const double mu = ex / dl;
-            const double tmp = ex2 / dl - mu * mu;
-            mo[I] = mu;
-            so[I] = tmp > 0.0 ? sqrt(tmp) : 1.0;
-            const double u = x[I];
-            ex -= u;
-            ex2 -= u * u;
+    constexpr int KB = 8;
+    for (int k0 = 0; k0 < L - 1; k0 += KB) {
+        double v[KB];
+#pragma unroll
+        for (int u = 0; u < KB; ++u) v[u] = x[k0 + u < L - 1 ? k0 + u : 0];
+#pragma unroll
+        for (int u = 0; u < KB; ++u)
+            if (k0 + u < L - 1) {
+                ex += v[u];
+                ex2 += v[u] * v[u];
+            }
+    }
+    for (int I0 = 0; I0 < nwin; I0 += KB) {
+        double v[KB], w[KB];
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+            const int I = I0 + u < nwin ? I0 + u : nwin - 1;
+            v[u] = x[I + L - 1];
+            w[u] = x[I];
         }
+#pragma unroll
+        for (int u = 0; u < KB; ++u)
+            if (I0 + u < nwin) {
+                ex += v[u];
+                ex2 += v[u] * v[u];
+                mo[I0 + u] = ex;
+                so[I0 + u] = ex2;
+                ex -= w[u];
+                ex2 -= w[u] * w[u];
+            }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_window_stats_all(int64_t cn, int t, int n_groups,
+                                                          const int *__restrict__ lens,
+                                                          const int64_t *__restrict__ goff,
+                                                          double *__restrict__ mean,
+                                                          double *__restrict__ sdev) {
+    const int g = blockIdx.y;
+    const int L = lens[g];
+    const int64_t n = cn * (t - L + 1);
+    const double dl = (double)L;
+    double *__restrict__ mo = mean + goff[g];
+    double *__restrict__ so = sdev + goff[g];
+    for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < n; q += (int64_t)gridDim.x * 256) {
+        const double mu = mo[q] / dl;
+        const double tmp = so[q] / dl - mu * mu;
+        mo[q] = mu;
+        so[q] = tmp > 0.0 ? sqrt(tmp) : 1.0;
     }
 }
 
@@ -806,6 +1193,9 @@ constexpr size_t kScratchCap = (size_t)512 << 20;  // DTW scratch rows
 constexpr size_t kChunkCap = (size_t)512 << 20;    // window statistics + envelopes
 constexpr size_t kTDCap = (size_t)256 << 20;       // per-window (T, D)
 constexpr int64_t kMaxWaves = 8192;
+// Smallest class (series times patterns) for the pruned search: a task is one
+// wave's 0.3 ms in turn, every window of 256 tasks in parallel takes that too.
+constexpr int64_t kSearchTasks = 256;
 
 size_t scratch_bytes(int64_t max_len) {
     const size_t one = (size_t)64 * 8 * (size_t)(4 * max_len);  // at least one wave
@@ -844,8 +1234,19 @@ Groups make_groups(const int64_t *hl, int64_t n_s, int64_t t) {
     return G;
 }
 
-int64_t chunk_rows(int kind, int64_t n, int64_t t, int64_t win_total) {
-    const int64_t per = win_total * 16 + (kind == WBX_DTW ? t * 16 : 0);
+// Distinct warp widths of the groups, ascending (r: the band fraction).
+std::vector<int> warp_widths(const Groups &G, double r) {
+    std::vector<int> w;
+    for (int L : G.len) {
+        const int rw = warp_width(L, r);
+        if (w.empty() || w.back() != rw) w.push_back(rw);
+    }
+    return w;
+}
+
+// env: sets of series envelopes kept (0: none).
+int64_t chunk_rows(int64_t n, int64_t t, int64_t win_total, int64_t env) {
+    const int64_t per = win_total * 16 + env * t * 16;
     int64_t c = (int64_t)(kChunkCap / (size_t)per);
     if (c < 1) c = 1;
     return c < n ? c : n;
@@ -853,11 +1254,12 @@ int64_t chunk_rows(int kind, int64_t n, int64_t t, int64_t win_total) {
 
 }  // namespace
 
-size_t scaled_ws_bytes(int kind, const int64_t *hl, int64_t n_s, int64_t total, int64_t n,
-                       int64_t t) {
+size_t scaled_ws_bytes(int kind, double r, const int64_t *hl, int64_t n_s, int64_t total,
+                       int64_t n, int64_t t) {
     const Groups G = make_groups(hl, n_s, t);
     int64_t max_len = G.len.back();
-    const int64_t cn = chunk_rows(kind, n, t, G.win_total);
+    const int64_t env = kind == WBX_DTW ? (int64_t)warp_widths(G, r).size() : 0;
+    const int64_t cn = chunk_rows(n, t, G.win_total, env);
     size_t b = 0;
     auto take = [&](size_t bytes) { b += (bytes + 255) & ~(size_t)255; };
     take((size_t)total * 8);                                // zs
@@ -867,7 +1269,8 @@ size_t scaled_ws_bytes(int kind, const int64_t *hl, int64_t n_s, int64_t total, 
     take(G.len.size() * 16);                                // group offsets, lengths
     take((size_t)cn * (size_t)G.win_total * 16);            // window mean / std
     if (kind == WBX_DTW) {
-        take((size_t)cn * (size_t)t * 16);                  // series envelopes
+        take((size_t)n_s * sizeof(SearchPattern));
+        take((size_t)env * (size_t)cn * (size_t)t * 16);    // series envelopes
         take(scratch_bytes(max_len));
         take(kTDCap > (size_t)cn * (size_t)t * 16 ? kTDCap : (size_t)cn * (size_t)t * 16);
     }
@@ -885,7 +1288,9 @@ int launch_scaled_subseq(int kind, double r, const double *S, const int64_t *s_o
     const Groups G = make_groups(hl, n_s, t);
     const int n_groups = (int)G.len.size();
     const int64_t max_len = G.len.back();
-    const int64_t cn_max = chunk_rows(kind, n, t, G.win_total);
+    const std::vector<int> widths = dtw ? warp_widths(G, r) : std::vector<int>();
+    const int64_t n_env = (int64_t)widths.size();
+    const int64_t cn_max = chunk_rows(n, t, G.win_total, n_env);
     std::vector<int64_t> goff((size_t)n_groups);
     for (int64_t g = 0, w = 0; g < n_groups; ++g) {
         goff[g] = w * cn_max;
@@ -907,11 +1312,32 @@ int launch_scaled_subseq(int kind, double r, const double *S, const int64_t *s_o
     double *wmean = (double *)take((size_t)cn_max * (size_t)G.win_total * 16);
     double *wstd = wmean + cn_max * G.win_total;
     double *elo = nullptr, *eup = nullptr, *scratch = nullptr, *Tb = nullptr;
+    // the patterns by register class of their band, longest first in each
+    std::vector<SearchPattern> pats;
+    std::vector<int64_t> cls_beg(kMaxBPS / 8 + 2, 0);
+    SearchPattern *d_pats = nullptr;
     const size_t sbytes = scratch_bytes(max_len);
     size_t td_bytes = 0;
     if (dtw) {
-        elo = (double *)take((size_t)cn_max * (size_t)t * 16);
-        eup = elo + cn_max * t;
+        for (int c = 1; c <= kMaxBPS / 8; ++c) {
+            cls_beg[c] = (int64_t)pats.size();
+            for (int g = n_groups - 1; g >= 0; --g) {
+                const int rw = warp_width(G.len[g], r);
+                if ((2 * rw + 8) / 8 != c) continue;  // (2 rw + 1 rounded up) / 8
+                const int64_t set =
+                    std::lower_bound(widths.begin(), widths.end(), rw) - widths.begin();
+                for (int64_t k = G.start[g]; k < G.start[g + 1]; ++k)
+                    pats.push_back({goff[g], set * cn_max * t, (int32_t)G.order[k], G.len[g],
+                                    rw});
+            }
+        }
+        cls_beg[kMaxBPS / 8 + 1] = (int64_t)pats.size();
+        d_pats = (SearchPattern *)take((size_t)n_s * sizeof(SearchPattern));
+        if (!pats.empty())
+            WBX_HIP_CHECK(hipMemcpyAsync(d_pats, pats.data(), sizeof(SearchPattern) * pats.size(),
+                                         hipMemcpyHostToDevice, st));
+        elo = (double *)take((size_t)n_env * (size_t)cn_max * (size_t)t * 16);
+        eup = elo + n_env * cn_max * t;
         scratch = (double *)take(sbytes);
         td_bytes = kTDCap > (size_t)cn_max * (size_t)t * 16 ? kTDCap : (size_t)cn_max * (size_t)t * 16;
         Tb = (double *)take(td_bytes);
@@ -930,10 +1356,73 @@ int launch_scaled_subseq(int kind, double r, const double *S, const int64_t *s_o
         const int64_t cn = n - c0 < cn_max ? n - c0 : cn_max;
         const double *xc = X + c0 * xstride;
         const int64_t nst = cn * n_groups;
-        hipLaunchKernelGGL(k_window_stats_all, dim3((unsigned)((nst + 63) / 64)), dim3(64), 0, st,
+        hipLaunchKernelGGL(k_window_sums_all, dim3((unsigned)((nst + 63) / 64)), dim3(64), 0, st,
                            xc, cn, xstride, (int)t, n_groups, d_glen, d_goff, wmean, wstd);
+        for (int g0 = 0; g0 < n_groups; g0 += 65535) {
+            const int gn = std::min(n_groups - g0, 65535);
+            const int64_t nb = (cn * (t - G.len[g0] + 1) + 1023) / 1024;
+            hipLaunchKernelGGL(k_window_stats_all, dim3((unsigned)std::min<int64_t>(nb, 4096),
+                                                        (unsigned)gn),
+                               dim3(256), 0, st, cn, (int)t, gn, d_glen + g0, d_goff + g0, wmean,
+                               wstd);
+        }
         WBX_HIP_CHECK(hipGetLastError());
-        int env_w = -1;
+        for (int64_t e = 0; e < n_env; ++e) {
+            const int rc = launch_envelope(xc, cn, xstride, (int)t, widths[e], elo + e * cn_max * t,
+                                           eup + e * cn_max * t, st);
+            if (rc) return rc;
+        }
+        // Classes with enough (series, pattern) tasks take the pruned search;
+        // fewer run every window of every task in parallel instead.
+        std::vector<char> searched(kMaxBPS / 8 + 1, 0);
+        for (int c = 1; dtw && !wide_only && c <= kMaxBPS / 8; ++c) {
+            const int64_t np = cls_beg[c + 1] - cls_beg[c];
+            if (np == 0 || np * cn < kSearchTasks) continue;
+            searched[c] = 1;
+            SearchArgs sa{};
+            sa.a.X = xc;
+            sa.a.xstride = xstride;
+            sa.a.t = (int)t;
+            sa.a.c0 = c0;
+            sa.a.cn = cn;
+            sa.a.zs = zs;
+            sa.a.zl = zl;
+            sa.a.zu = zu;
+            sa.a.n_s = n_s;
+            sa.a.dist = dist;
+            sa.a.idx = idx;
+            sa.wmean = wmean;
+            sa.wstd = wstd;
+            sa.elo = elo;
+            sa.eup = eup;
+            sa.s_off = s_off;
+            sa.undecided = (int *)Tb;
+            // as many patterns at a time as have their flags in the buffer
+            const int64_t step = std::max<int64_t>(1, (int64_t)(td_bytes / 4) / cn);
+            for (int64_t k0 = cls_beg[c]; k0 < cls_beg[c + 1]; k0 += step) {
+                const int64_t k1 = std::min(cls_beg[c + 1], k0 + step);
+                sa.pats = d_pats + k0;
+                sa.n_tasks = (k1 - k0) * cn;
+                int64_t per_lane = 0;
+                for (int64_t k = k0; k < k1; ++k)
+                    per_lane = std::max(per_lane, per_lane_doubles(pats[k].L, pats[k].rw, false));
+                const dim3 grid((unsigned)std::min(sa.n_tasks, kMaxWaves));
+                const dim3 gridx((unsigned)group_waves(std::min<int64_t>(sa.n_tasks, 1024), sbytes,
+                                                       per_lane));
+#define WBX_SEARCH_LAUNCH(C)                                                                  \
+    case C:                                                                                   \
+        hipLaunchKernelGGL((k_scaled_search<C, 4>), grid, dim3(64), 0, st, sa);               \
+        hipLaunchKernelGGL((k_scaled_search_exact<C, 4>), gridx, dim3(64), 0, st, sa, scratch, \
+                           per_lane);                                                         \
+        break;
+                switch (8 * c) {
+                    WBX_SCALED_CLASSES(WBX_SEARCH_LAUNCH)
+                    default: return fail(WBX_EUNSUPPORTED, "scaled dtw: class %d", 8 * c);
+                }
+#undef WBX_SEARCH_LAUNCH
+                WBX_HIP_CHECK(hipGetLastError());
+            }
+        }
         for (int g = 0; g < n_groups; ++g) {
             const int L = G.len[g];
             const int nwin = (int)(t - L + 1);
@@ -963,17 +1452,14 @@ int launch_scaled_subseq(int kind, double r, const double *S, const int64_t *s_o
                 continue;
             }
             const int rw = warp_width(L, r);
-            if (rw != env_w) {
-                const int rc = launch_envelope(xc, cn, xstride, (int)t, rw, elo, eup, st);
-                if (rc) return rc;
-                env_w = rw;
-            }
-            a.elo = elo;
-            a.eup = eup;
+            const int64_t set = std::lower_bound(widths.begin(), widths.end(), rw) - widths.begin();
+            a.elo = elo + set * cn_max * t;
+            a.eup = eup + set * cn_max * t;
             a.rw = rw;
             a.B = 2 * rw + 1;
             const int BP = (a.B + 7) / 8 * 8;
             const bool wide = wide_only || BP > kMaxBPS;
+            if (!wide && searched[BP / 8]) continue;
             const int64_t per_lane = per_lane_doubles(L, rw, wide);
             // patterns of the group in batches whose (T, D) fit the buffer
             int64_t bsz = (int64_t)(td_bytes / ((size_t)cn * (size_t)nwin * 16));
@@ -1016,7 +1502,7 @@ size_t scaled_wrap_ws_bytes(const int64_t *hl, int64_t n_s, int64_t total, int64
                             int64_t t) {
     const Groups G = make_groups(hl, n_s, t);
     const int64_t max_len = G.len.back();
-    const int64_t cn = chunk_rows(WBX_EUCLIDEAN, n, t, G.win_total);
+    const int64_t cn = chunk_rows(n, t, G.win_total, 0);
     size_t b = 0;
     auto take = [&](size_t bytes) { b += (bytes + 255) & ~(size_t)255; };
     take((size_t)total * 8);                      // zs
@@ -1039,7 +1525,7 @@ int launch_scaled_wrap(int kind, double r, const double *weights, double penalty
     const Groups G = make_groups(hl, n_s, t);
     const int n_groups = (int)G.len.size();
     const int64_t max_len = G.len.back();
-    const int64_t cn_max = chunk_rows(WBX_EUCLIDEAN, n, t, G.win_total);
+    const int64_t cn_max = chunk_rows(n, t, G.win_total, 0);
     std::vector<int64_t> goff((size_t)n_groups);
     for (int64_t g = 0, w = 0; g < n_groups; ++g) {
         goff[g] = w * cn_max;

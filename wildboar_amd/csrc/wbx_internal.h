@@ -369,8 +369,8 @@ int launch_subseq_exact(int kind, double r, Shapelets sh, int max_len, Series<T>
 // host lengths, total = packed length), pattern mean / std (device), float64
 // series X (n rows of length t, stride xstride).  ws holds scaled_ws_bytes.
 // wide_only: the DTW band in scratch memory for every width.
-size_t scaled_ws_bytes(int kind, const int64_t *hl, int64_t n_s, int64_t total, int64_t n,
-                       int64_t t);
+size_t scaled_ws_bytes(int kind, double r, const int64_t *hl, int64_t n_s, int64_t total,
+                       int64_t n, int64_t t);
 int launch_scaled_subseq(int kind, double r, const double *S, const int64_t *s_off,
                          const int64_t *s_len, const int64_t *hl, int64_t n_s, int64_t total,
                          const double *s_mean, const double *s_std, const double *X,
