@@ -1,0 +1,49 @@
+"""The pruned float32 subsequence DTW scan: distances and indices are the
+reference's exactly, whatever windows its bounds leave out.  Window counts
+around 64 (the spread windows), 256 (a round of bounds) and its trial length,
+shapelets shorter than a bound's four terms, every kind of band, equal windows
+(which overflow the candidate list) and data on which no bound prunes."""
+
+import numpy as np
+import pytest
+
+import oracle
+from wildboar_amd import distance as wd
+
+pytestmark = pytest.mark.gpu
+
+
+def _data(kind, n, t, lens, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "integers":
+        return (rng.integers(0, 3, (n, t)).astype(np.float64),
+                [rng.integers(0, 3, L).astype(np.float64) for L in lens])
+    if kind == "constant":
+        X = np.full((n, t), 2.0)
+        X[1:, t // 2:] = 0.5
+        return X, [np.full(L, 1.0) for L in lens]
+    if kind == "noise":  # the envelope covers nearly everything
+        return rng.standard_normal((n, t)) * 0.01, [rng.standard_normal(L) * 5.0 for L in lens]
+    X = rng.standard_normal((n, t)).cumsum(axis=1)
+    S = [X[i % n, (t - L) // 2:][:L] + rng.standard_normal(L) * 0.1 for i, L in enumerate(lens)]
+    return X, S
+
+
+@pytest.mark.parametrize("kind", ["walks", "integers", "constant", "noise"])
+@pytest.mark.parametrize("t,lens,r", [
+    (40, (3, 5, 40, 37), 0.3),
+    (83, (20, 20, 19, 21), 0.2),       # 63, 64 and 65 windows
+    (300, (45, 46, 44), 0.1),          # 255, 256 and 257 windows
+    (700, (64, 101, 128), 0.1),
+    (900, (60, 128), 0.24),            # bands to 59 slots
+    (600, (40, 33), 0.05),             # one-slot bands
+    (400, (47, 50), 1.0),
+])
+def test_pruned_scan_is_exact(t, lens, r, kind):
+    X, S = _data(kind, 4, t, lens, t + len(lens))
+    for x in (X, X.astype(np.float32).astype(np.float64)):
+        d, i = wd.pairwise_subsequence_distance(S, x, metric="dtw", metric_params={"r": r},
+                                                return_index=True, precision="fp32")
+        od, oi = oracle.subsequence(S, x, metric="dtw", r=r)
+        np.testing.assert_array_equal(d, od)
+        np.testing.assert_array_equal(i, oi)

@@ -28,8 +28,14 @@ struct TaskMap {
 
 struct SubCand {
     int32_t count;             // number of candidates (> kMaxCand: overflow)
-    int32_t win[kMaxCand];     // window starts, increasing
+    int32_t win[kMaxCand];     // window starts
     float best32;
+};
+
+// The candidates of a launch: the task of each (a task's are together).
+struct CandOut {
+    uint32_t *list;
+    int *n;
 };
 
 struct SubGeo {
@@ -41,12 +47,16 @@ struct SubGeo {
     int T;
     double r;
     float rho, A;       // certification: tau(c) = rho (c + A) + A
+    const float *lo, *hi;  // the shapelets' envelopes, packed like S (DTW)
 };
 
+int launch_subseq_envelope(const float *S, const int64_t *off, const int64_t *len, int64_t n_s,
+                           double r, float *lo, float *hi, hipStream_t st);
+
 int launch_subseq_fast(int kind, int B, TaskMap tasks, int64_t n_tasks, SubGeo sg,
-                       SubCand *cands, hipStream_t st);
+                       SubCand *cands, CandOut co, hipStream_t st);
 int launch_subseq_exact_cands(int kind, int B, TaskMap tasks, const SubCand *cands,
-                              int64_t n_tasks, const double *S64, const int64_t *soff,
+                              CandOut co, int64_t n_tasks, const double *S64, const int64_t *soff,
                               const int64_t *slen, const double *X64, int64_t xstride, int T,
                               double r, double *cost64, hipStream_t st);
 int launch_subseq_select(TaskMap tasks, const SubCand *cands, int64_t n_tasks,

@@ -6,17 +6,23 @@
 // euclidean_distance, distance/_metric.pyx:654-683), the first window that
 // attains it, and sqrt of that minimum.
 //
-// Pass 1 (FP32): one (sample, shapelet) task per 64-lane wave, lane l scans
-//   window ws = 64 b + l of block b.  For DTW each lane runs the register-band
-//   recursion of lane.hip on its window (all lanes share the shapelet, so the
-//   geometry is uniform); for euclidean each lane sums (x - s)^2 over its
-//   window.  A window is a candidate when its FP32 cost c satisfies
+// Pass 1 (FP32): one (sample, shapelet) task per 64-lane wave.  For DTW each
+//   lane runs the register-band recursion of lane.hip on a window (all lanes
+//   share the shapelet, so the geometry is uniform); for euclidean each lane
+//   sums (x - s)^2 over its windows.  A window is a candidate when its FP32 cost c satisfies
 //   c <= tau(c*) = rho (c* + A) + A, c* the smallest FP32 cost so far: by the
 //   bound in rerank.hip no other window can hold the float64 minimum.  The
 //   wave keeps up to 64 candidates with their costs in LDS and drops those
 //   that fail tau of the current best when the list fills; at the end the
 //   ones within tau(final best) are stored (at most kMaxCand, else the task
-//   is marked as overflowed).
+//   is marked as overflowed).  The order in which windows are looked at does
+//   not change the candidates, so DTW takes 64 windows spread over the series
+//   first and then only those whose LB_Keogh sum (the window against the
+//   shapelet's envelope of the band's radius, four FP32 instructions a value
+//   against three per band slot) does not exceed tau of the best so far.  Sum
+//   and cost carry the same kind of rounding: with K = 2 L + 2 roundings each
+//   way the sum is at most rho times the window's FP32 cost, so a sum above
+//   rho^2 tau leaves the cost above tau.
 // Pass 2 (FP64): one candidate per lane, evaluated with the reference's exact
 //   arithmetic (DTW: min(min(up, left), diag) + v*v, no FMA; euclidean: the
 //   sequential sum), then per task the first strictly smallest candidate wins.
@@ -86,7 +92,8 @@ __device__ __forceinline__ void cand_push(CandList &cl, int *s_win, float *s_cos
 // else the task is marked for the exact rescan (count kMaxCand + 1).
 __device__ __forceinline__ void cand_finish(const CandList &cl, const int *s_win,
                                             const float *s_cost, float tau, float best,
-                                            SubCand *__restrict__ out) {
+                                            int64_t task, SubCand *__restrict__ out,
+                                            CandOut co) {
     const int lane = threadIdx.x;
     __syncthreads();
     const bool has = !cl.overflow && lane < cl.count;
@@ -96,139 +103,16 @@ __device__ __forceinline__ void cand_finish(const CandList &cl, const int *s_win
     const uint64_t km = __ballot(keep);
     const int n = (int)__popcll(km);
     const bool ovf = cl.overflow || n > kMaxCand;
-    if (!ovf && keep) out->win[__popcll(km & ((1ull << lane) - 1ull))] = w;
+    const int pos = (int)__popcll(km & ((1ull << lane) - 1ull));
+    if (!ovf && keep) out->win[pos] = w;
+    unsigned base = 0;
     if (lane == 0) {
         out->count = ovf ? kMaxCand + 1 : n;
         out->best32 = best;
+        if (!ovf) base = atomicAdd((unsigned *)co.n, (unsigned)n);
     }
-}
-
-// Waves per SIMD the register allocation is held to, by band class: left
-// alone the allocator spreads the window-batch set-up over up to 230
-// registers (two or three waves); 13 and 15 fit four waves and 17 .. 23
-// three without spills (wider classes would spill).
-constexpr int subseq_dtw32_waves(int BP) {
-    return BP <= 11 ? 1 : BP <= 15 ? 4 : BP <= 23 ? 3 : 1;
-}
-
-template <int BP, int U>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(subseq_dtw32_waves(BP)))) void
-k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands) {
-    static_assert(U % 4 == 0, "groups of whole 16-byte loads");
-    constexpr int W = BP + U - 1;
-    const int lane = threadIdx.x;
-    const SubTask tk = tasks.at(blockIdx.x);
-    // the shapelet is the same for every lane and is not written by the
-    // launch: read through the constant address space, its values are scalar
-    // loads into SGPRs
-    const float *__restrict__ S = sg.S + sg.off[tk.shapelet];
-    const __attribute__((address_space(4))) float *Sc =
-        (const __attribute__((address_space(4))) float *)S;
-    const int L = (int)sg.len[tk.shapelet];
-    const int off = band_w(L, L, sg.r) - 1;  // the band has 2 w - 1 == BP slots
-    const int nwin = sg.T - L + 1;
-    const float *__restrict__ Xrow = sg.X + (int64_t)tk.sample * sg.xstride;
-    SubCand *cout = cands + blockIdx.x;
-    __shared__ int s_win[kCap];
-    __shared__ float s_cost[kCap];
-    CandList cl{0, false};
-    float best = WBX_INF_F;
-    for (int b0 = 0; b0 < nwin; b0 += 64) {
-        const int ws = b0 + lane;
-        const bool active = ws < nwin;
-        const float *__restrict__ Y = Xrow + (active ? ws : nwin - 1);
-        float row[BP];
-#pragma unroll
-        for (int k = 0; k < BP; ++k) row[k] = (k == off) ? 0.0f : WBX_INF_F;
-        float yw[W];
-        if (b0 >= off && W - off <= L) {
-            // uniform: every lane's columns -off .. W - off - 1 are inside the
-            // series row (ws >= off) and end inside the window; the first off
-            // are left of it (+inf)
-            const float *__restrict__ Yb = Y - off;
-#pragma unroll
-            for (int q = 0; q < W; q += 4) {
-                if (q + 4 <= W) {
-                    const f4a v = *(const f4a *)(Yb + q);
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) yw[q + u] = v[u];
-                } else {
-#pragma unroll
-                    for (int u = 0; q + u < W; ++u) yw[q + u] = Yb[q + u];
-                }
-            }
-#pragma unroll
-            for (int m = 0; m < W; ++m) yw[m] = m < off ? WBX_INF_F : yw[m];
-        } else {
-#pragma unroll
-            for (int m = 0; m < W; ++m) yw[m] = ldy(Y, m - off, L);
-        }
-        const int rem = L % U;
-        for (int i = 0; i < rem; ++i) {
-            const float xi = S[i];
-            float left = WBX_INF_F;
-#pragma unroll
-            for (int k = 0; k < BP; ++k) {
-                const float up = (k + 1 < BP) ? row[k + 1] : WBX_INF_F;
-                const float mn = fminf(fminf(up, left), row[k]);
-                const float d = xi - yw[k];
-                const float c = __builtin_fmaf(d, d, mn);
-                row[k] = c;
-                left = c;
-            }
-#pragma unroll
-            for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
-            yw[W - 1] = ldy(Y, i + 1 - off + W - 1, L);
-        }
-        for (int i0 = rem; i0 < L; i0 += U) {
-            // This group's new window entries, columns jn .. jn + U - 1
-            // (jn >= 0).  Every lane has the same shapelet and row, so when
-            // they lie inside the window (the usual case) they are plain
-            // vector loads, waited for only at the window shift.  The
-            // shapelet values are scalar loads (the shapelet stays in the
-            // scalar cache).
-            float yn[U];
-            const int jn = i0 - off + W;
-            if (jn + U <= L) {
-#pragma unroll
-                for (int u = 0; u < U; u += 4) {
-                    const f4a b = *(const f4a *)(Y + jn + u);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) yn[u + q] = b[q];
-                }
-            } else {
-#pragma unroll
-                for (int u = 0; u < U; ++u) yn[u] = ldy(Y, jn + u, L);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const float xi = Sc[i0 + u];
-                float left = WBX_INF_F;
-#pragma unroll
-                for (int k = 0; k < BP; ++k) {
-                    const float up = (k + 1 < BP) ? row[k + 1] : WBX_INF_F;
-                    const float mn = fminf(fminf(up, left), row[k]);
-                    const float d = xi - yw[k + u];
-                    const float c = __builtin_fmaf(d, d, mn);
-                    row[k] = c;
-                    left = c;
-                }
-            }
-#pragma unroll
-            for (int m = 0; m < W - U; ++m) yw[m] = yw[m + U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) yw[W - U + u] = yn[u];
-        }
-        float c = WBX_INF_F;
-#pragma unroll
-        for (int k = 0; k < BP; ++k)
-            if (k == off) c = row[k];
-        if (!active) c = WBX_INF_F;
-        best = fminf(best, wave_min(c));
-        const float tau = sg.rho * (best + sg.A) + sg.A;
-        cand_push(cl, s_win, s_cost, active && c <= tau, ws, c, tau);
-    }
-    cand_finish(cl, s_win, s_cost, sg.rho * (best + sg.A) + sg.A, best, cout);
+    base = (unsigned)__shfl((int)base, 0);
+    if (!ovf && keep) co.list[(size_t)base + pos] = (uint32_t)task;
 }
 
 // Four consecutive floats of a row of length T starting at e (e >= 0): one
@@ -243,13 +127,262 @@ __device__ __forceinline__ f4u row4(const float *__restrict__ row, int e, int T)
     return v;
 }
 
+// FP32 cost of the window at Y of every lane against the shapelet S (scalar
+// loads through Sc), band of BP = 2 off + 1 slots; sw: the lane's window
+// start (columns left of it are read when every lane has off of them).  +inf
+// once every lane's row minimum is above lim (row minima only grow).
+template <int BP, int U>
+__device__ __forceinline__ float window_cost32(const float *__restrict__ S,
+                                               const __attribute__((address_space(4))) float *Sc,
+                                               int L, int off, const float *__restrict__ Y, int sw,
+                                               float lim) {
+    static_assert(U % 4 == 0, "groups of whole 16-byte loads");
+    constexpr int W = BP + U - 1;
+    float row[BP];
+#pragma unroll
+    for (int k = 0; k < BP; ++k) row[k] = (k == off) ? 0.0f : WBX_INF_F;
+    float yw[W];
+    if (__ballot(sw < off) == 0 && W - off <= L) {
+        // uniform: every lane's columns -off .. W - off - 1 are inside the
+        // series row and end inside the window; the first off are left of it
+        // (+inf)
+        const float *__restrict__ Yb = Y - off;
+#pragma unroll
+        for (int q = 0; q < W; q += 4) {
+            if (q + 4 <= W) {
+                const f4a v = *(const f4a *)(Yb + q);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) yw[q + u] = v[u];
+            } else {
+#pragma unroll
+                for (int u = 0; q + u < W; ++u) yw[q + u] = Yb[q + u];
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < W; ++m) yw[m] = m < off ? WBX_INF_F : yw[m];
+    } else {
+#pragma unroll
+        for (int m = 0; m < W; ++m) yw[m] = ldy(Y, m - off, L);
+    }
+    auto cells = [&](const float *y, float xi) {
+        float left = WBX_INF_F;
+#pragma unroll
+        for (int k = 0; k < BP; ++k) {
+            const float up = (k + 1 < BP) ? row[k + 1] : WBX_INF_F;
+            const float mn = fminf(fminf(up, left), row[k]);
+            const float d = xi - y[k];
+            const float c = __builtin_fmaf(d, d, mn);
+            row[k] = c;
+            left = c;
+        }
+    };
+    const int rem = L % U;
+    for (int i = 0; i < rem; ++i) {
+        cells(yw, S[i]);
+#pragma unroll
+        for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
+        yw[W - 1] = ldy(Y, i + 1 - off + W - 1, L);
+    }
+    for (int i0 = rem; i0 < L; i0 += U) {
+        // This group's new window entries, columns jn .. jn + U - 1 (jn >=
+        // 0).  Every lane has the same shapelet and row, so when they lie
+        // inside the window (the usual case) they are plain vector loads,
+        // waited for only at the window shift.  The shapelet values are
+        // scalar loads (the shapelet stays in the scalar cache).
+        float yn[U];
+        const int jn = i0 - off + W;
+        if (jn + U <= L) {
+#pragma unroll
+            for (int u = 0; u < U; u += 4) {
+                const f4a b = *(const f4a *)(Y + jn + u);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) yn[u + q] = b[q];
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) yn[u] = ldy(Y, jn + u, L);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) cells(yw + u, Sc[i0 + u]);
+#pragma unroll
+        for (int m = 0; m < W - U; ++m) yw[m] = yw[m + U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) yw[W - U + u] = yn[u];
+        if (BP > 3 && ((i0 - rem) / U & 3) == 3) {  // every fourth group
+            float rm = row[0];
+#pragma unroll
+            for (int k = 1; k < BP; ++k) rm = fminf(rm, row[k]);
+            if (__ballot(!(rm > lim)) == 0) return WBX_INF_F;
+        }
+    }
+    float c = WBX_INF_F;
+#pragma unroll
+    for (int k = 0; k < BP; ++k)
+        if (k == off) c = row[k];
+    return c;
+}
+
+// Waves per SIMD the register allocation is held to, by band class: left
+// alone the allocator spreads the window-batch set-up over many registers;
+// 13 and 15 fit four waves and 17 .. 23 three without spills (wider classes
+// would spill).
+constexpr int subseq_dtw32_waves(int BP) {
+    return BP <= 11 ? 1 : BP <= 15 ? 4 : BP <= 23 ? 3 : 1;
+}
+
+// Windows whose LB_Keogh sums were formed before the scan decides whether
+// they are worth forming: with more than three quarters of them left, the
+// rest of the task's windows go straight to the DTW.
+constexpr int kLbTrial = 512;
+
+// 256 shapelets of 16 .. 128 over 500 series of 1024, r = 0.1: 3.4 ms for
+// all classes, 7.9 ms when every window's DTW was computed.
+template <int BP, int U>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(subseq_dtw32_waves(BP)))) void
+k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands, CandOut co) {
+    const int lane = threadIdx.x;
+    const SubTask tk = tasks.at(blockIdx.x);
+    // the shapelet is the same for every lane and is not written by the
+    // launch: read through the constant address space, its values are scalar
+    // loads into SGPRs
+    typedef const __attribute__((address_space(4))) float *cfp;
+    const int64_t so = sg.off[tk.shapelet];
+    const float *__restrict__ S = sg.S + so;
+    const cfp Sc = (cfp)S, lo = (cfp)(sg.lo + so), hi = (cfp)(sg.hi + so);
+    const int L = (int)sg.len[tk.shapelet];
+    const int off = band_w(L, L, sg.r) - 1;  // the band has 2 w - 1 == BP slots
+    const int T = sg.T, nwin = T - L + 1;
+    const float *__restrict__ Xrow = sg.X + (int64_t)tk.sample * sg.xstride;
+    __shared__ int s_win[kCap];
+    __shared__ float s_cost[kCap];
+    __shared__ int queue[64 + 256];
+    CandList cl{0, false};
+    float best = WBX_INF_F, tau = WBX_INF_F;
+    if constexpr (BP <= 3) {
+        // a row costs about what its LB_Keogh terms would: every window, in
+        // order (B = 1: 36 us so, 82 us pruned; B = 3: 111 and 149; B = 5:
+        // 181 and 163)
+        for (int b0 = 0; b0 < nwin; b0 += 64) {
+            const int ws = b0 + lane;
+            const bool active = ws < nwin;
+            const int wc = active ? ws : nwin - 1;
+            float c = window_cost32<BP, U>(S, Sc, L, off, Xrow + wc, wc, WBX_INF_F);
+            if (!active) c = WBX_INF_F;
+            best = fminf(best, wave_min(c));
+            tau = sg.rho * (best + sg.A) + sg.A;
+            cand_push(cl, s_win, s_cost, active && c <= tau, ws, c, tau);
+        }
+        cand_finish(cl, s_win, s_cost, tau, best, blockIdx.x, cands + blockIdx.x, co);
+        return;
+    }
+    const int step = (nwin + 63) / 64;  // the spread windows are lane * step
+    int nq = 0, b0 = 0, tested = 0, left = 0;
+    for (bool first = true;; first = false) {
+        int ws = lane * step;
+        bool active = ws < nwin;
+        if (!first) {
+            const bool bound = tested < kLbTrial || left * 4 <= tested * 3;
+            while (nq < 64 && b0 < nwin) {
+                // lane l forms the sums of the windows w0 .. w0 + 3
+                const int w0 = b0 + 4 * lane;
+                const float lim = tau * sg.rho * sg.rho * 1.000001f;
+                float lb[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (bound) {
+                    float xw[8];
+                    const f4u a = row4(Xrow, w0 < T ? w0 : T - 1, T),
+                              b = row4(Xrow, w0 + 4 < T ? w0 + 4 : T - 1, T);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        xw[q] = a[q];
+                        xw[4 + q] = b[q];
+                    }
+                    // the last L % 4 terms are left out
+                    for (int j0 = 0; j0 + 4 <= L; j0 += 4) {
+                        const f4u nx = row4(Xrow, w0 + j0 + 8 < T ? w0 + j0 + 8 : T - 1, T);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const float h = hi[j0 + u], l = lo[j0 + u];
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) {
+                                const float d =
+                                    fmaxf(fmaxf(xw[q + u] - h, l - xw[q + u]), 0.0f);
+                                lb[q] = __builtin_fmaf(d, d, lb[q]);
+                            }
+                        }
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            xw[q] = xw[4 + q];
+                            xw[4 + q] = nx[q];
+                        }
+                        if ((j0 & 12) == 12) {
+                            const float m = fminf(fminf(lb[0], lb[1]), fminf(lb[2], lb[3]));
+                            if (__ballot(!(m > lim)) == 0) break;
+                        }
+                    }
+                }
+                int kept = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int s = w0 + q;
+                    const bool keep = s < nwin && s % step != 0 && !(lb[q] > lim);
+                    const uint64_t km = __ballot(keep);
+                    if (keep) queue[nq + kept + (int)__popcll(km & ((1ull << lane) - 1ull))] = s;
+                    kept += (int)__popcll(km);
+                }
+                nq += kept;
+                if (bound) {
+                    tested += 256;
+                    left += kept;
+                }
+                b0 += 256;
+                __syncthreads();
+            }
+            if (nq == 0) break;
+            active = lane < nq;
+            // the newest 64 of the queue
+            ws = queue[active ? (nq < 64 ? lane : nq - 64 + lane) : 0];
+            nq = nq < 64 ? 0 : nq - 64;
+            __syncthreads();
+        }
+        const int wc = active ? ws : (first ? 0 : ws);
+        float c = window_cost32<BP, U>(S, Sc, L, off, Xrow + wc, wc, tau);
+        if (!active) c = WBX_INF_F;
+        best = fminf(best, wave_min(c));
+        tau = sg.rho * (best + sg.A) + sg.A;
+        cand_push(cl, s_win, s_cost, active && c <= tau, ws, c, tau);
+    }
+    cand_finish(cl, s_win, s_cost, tau, best, blockIdx.x, cands + blockIdx.x, co);
+}
+
+// Envelope of each packed shapelet over the band's columns, |k - j| < w.
+__global__ __launch_bounds__(64) void k_subseq_envelope(const float *__restrict__ S,
+                                                        const int64_t *__restrict__ off,
+                                                        const int64_t *__restrict__ len, double r,
+                                                        float *__restrict__ lo,
+                                                        float *__restrict__ hi) {
+    const int64_t j = blockIdx.x;
+    const int L = (int)len[j];
+    const int rad = band_w(L, L, r) - 1;
+    const float *__restrict__ s = S + off[j];
+    for (int k = threadIdx.x; k < L; k += 64) {
+        const int a = k - rad > 0 ? k - rad : 0, b = k + rad < L - 1 ? k + rad : L - 1;
+        float l = s[a], h = s[a];
+        for (int q = a + 1; q <= b; ++q) {
+            l = fminf(l, s[q]);
+            h = fmaxf(h, s[q]);
+        }
+        lo[off[j] + k] = l;
+        hi[off[j] + k] = h;
+    }
+}
+
 // Lane l owns the U = 4 consecutive windows w0 .. w0 + 3 (w0 = b0 + 4 l) and
 // keeps x[w0 + j .. w0 + j + 8) in registers: four steps of j use static
 // indices (window q at step u reads xw[q + u]), then the window moves by four
 // with one 16-byte load.  Each window's sum runs over j in order.
 template <int U>
 __global__ __launch_bounds__(64) void k_subseq_euclid32(TaskMap tasks, SubGeo sg,
-                                                        SubCand *__restrict__ cands) {
+                                                        SubCand *__restrict__ cands, CandOut co) {
     static_assert(U == 4, "four windows per lane");
     const int lane = threadIdx.x;
     const SubTask tk = tasks.at(blockIdx.x);
@@ -258,7 +391,6 @@ __global__ __launch_bounds__(64) void k_subseq_euclid32(TaskMap tasks, SubGeo sg
     const int T = sg.T;
     const int nwin = T - L + 1;
     const float *__restrict__ Xrow = sg.X + (int64_t)tk.sample * sg.xstride;
-    SubCand *cout = cands + blockIdx.x;
     __shared__ int s_win[kCap];
     __shared__ float s_cost[kCap];
     CandList cl{0, false};
@@ -317,51 +449,55 @@ __global__ __launch_bounds__(64) void k_subseq_euclid32(TaskMap tasks, SubGeo sg
             cand_push(cl, s_win, s_cost, active && c <= tau, ws, c, tau);
         }
     }
-    cand_finish(cl, s_win, s_cost, sg.rho * (best + sg.A) + sg.A, best, cout);
+    cand_finish(cl, s_win, s_cost, sg.rho * (best + sg.A) + sg.A, best, blockIdx.x,
+                cands + blockIdx.x, co);
 }
 
 // ------------------------------------------------------------------ exact
 // Float64 cost of one candidate window per lane; per-lane geometry (all lanes
 // of a launch share BP).  Same arithmetic as dtw_distance: rows of S against
-// the window, cost = min(min(up, left), diag) + v * v.
+// the window, cost = min(min(up, left), diag) + v * v.  The lanes go over the
+// launch's candidate list (most tasks have one or two of the kMaxCand; a lane
+// for each place left seven of eight idle).
 template <int BP>
 __global__ __launch_bounds__(64) void k_subseq_cand64(TaskMap tasks,
                                                       const SubCand *__restrict__ cands,
-                                                      int64_t n_tasks, const double *__restrict__ S64,
+                                                      CandOut co, const double *__restrict__ S64,
                                                       const int64_t *__restrict__ soff,
                                                       const int64_t *__restrict__ slen,
                                                       const double *__restrict__ X64,
                                                       int64_t xstride, int T, double r, int kind,
                                                       double *__restrict__ cost64) {
-    const int64_t q = (int64_t)blockIdx.x * 64 + threadIdx.x;
-    const int64_t t = q / kMaxCand;
-    const int slot = (int)(q - t * kMaxCand);
-    if (t >= n_tasks) return;
-    const SubCand &cd = cands[t];
-    if (cd.count > kMaxCand || slot >= cd.count) return;
-    const SubTask tk = tasks.at(t);
-    const double *S = S64 + soff[tk.shapelet];
-    const int L = (int)slen[tk.shapelet];
-    const double *Y = X64 + (int64_t)tk.sample * xstride + cd.win[slot];
-    double res;
-    if (kind == WBX_EUCLIDEAN) {
-        double dist = 0.0;
-        for (int j = 0; j < L; ++j) {
-            double v = Y[j];
-            v -= S[j];
-            dist += v * v;
+    const int64_t n = (int64_t)(unsigned)*co.n;
+    for (int64_t q = (int64_t)blockIdx.x * 64 + threadIdx.x; q < n; q += (int64_t)gridDim.x * 64) {
+        const int64_t t = co.list[q];
+        int slot = 0;  // a task's entries are together, in the order of its places
+        while (slot < kMaxCand - 1 && q - 1 - slot >= 0 && co.list[q - 1 - slot] == (uint32_t)t)
+            ++slot;
+        const SubTask tk = tasks.at(t);
+        const double *S = S64 + soff[tk.shapelet];
+        const int L = (int)slen[tk.shapelet];
+        const double *Y = X64 + (int64_t)tk.sample * xstride + cands[t].win[slot];
+        double res;
+        if (kind == WBX_EUCLIDEAN) {
+            double dist = 0.0;
+            for (int j = 0; j < L; ++j) {
+                double v = Y[j];
+                v -= S[j];
+                dist += v * v;
+            }
+            res = dist;
+        } else {
+            // the band row in registers with a sliding window of the
+            // candidate's values (the float64 lane kernels' cell arithmetic,
+            // bit for bit); a launch holds one band class, B in (BP - 8, BP),
+            // whose padding slot B the routine resets every row
+            const int w = band_w(L, L, r);
+            res = lane64_cost<BP, 4, false, false, true>(S, L, Y, L, w - 1, 2 * w - 1, w - 1,
+                                                         nullptr, L);
         }
-        res = dist;
-    } else {
-        // the band row in registers with a sliding window of the candidate's
-        // values (the float64 lane kernels' cell arithmetic, bit for bit);
-        // a launch holds one band class, B in (BP - 8, BP), whose padding
-        // slot B the routine resets every row
-        const int w = band_w(L, L, r);
-        res = lane64_cost<BP, 4, false, false, true>(S, L, Y, L, w - 1, 2 * w - 1, w - 1, nullptr,
-                                                    L);
+        cost64[t * kMaxCand + slot] = res;
     }
-    cost64[q] = res;
 }
 
 // Per task: first strictly smallest exact cost among the candidates (window
@@ -478,17 +614,30 @@ int launch_subseq_rescan(TaskMap tasks, const int32_t *list, const int *n_list_d
                 X(59, 4) X(61, 4) X(63, 4)
 #define SUB_DTW_CASES(X) X(8, 8) X(16, 8) X(24, 8) X(32, 8) X(40, 8) X(48, 8) X(56, 8) X(64, 8)
 
+int launch_subseq_envelope(const float *S, const int64_t *off, const int64_t *len, int64_t n_s,
+                           double r, float *lo, float *hi, hipStream_t st) {
+    if (n_s <= 0) return WBX_OK;
+    hipLaunchKernelGGL(k_subseq_envelope, dim3((unsigned)n_s), dim3(64), 0, st, S, off, len, r, lo,
+                       hi);
+    WBX_HIP_CHECK(hipGetLastError());
+    return WBX_OK;
+}
+
 int launch_subseq_fast(int kind, int B, TaskMap tasks, int64_t n_tasks, SubGeo sg,
-                       SubCand *cands, hipStream_t st) {
+                       SubCand *cands, CandOut co, hipStream_t st) {
     if (n_tasks <= 0) return WBX_OK;
     if (n_tasks > 0x7fffffff) return fail(WBX_EUNSUPPORTED, "too many subsequence tasks");
     const dim3 grid((unsigned)n_tasks);
     if (kind == WBX_EUCLIDEAN) {
-        hipLaunchKernelGGL(k_subseq_euclid32<4>, grid, dim3(64), 0, st, tasks, sg, cands);
+        hipLaunchKernelGGL(k_subseq_euclid32<4>, grid, dim3(64), 0, st, tasks, sg, cands,
+                           co);
     } else {
         switch (B) {
 #define SD_CASE(B_, U_) \
-    case B_: hipLaunchKernelGGL((k_subseq_dtw32<B_, U_>), grid, dim3(64), 0, st, tasks, sg, cands); break;
+    case B_:                                                                                  \
+        hipLaunchKernelGGL((k_subseq_dtw32<B_, U_>), grid, dim3(64), 0, st, tasks, sg, cands, \
+                           co);                                                               \
+        break;
             SUB_SCAN_CASES(SD_CASE)
 #undef SD_CASE
             default: return fail(WBX_EUNSUPPORTED, "subsequence band %d", B);
@@ -499,16 +648,18 @@ int launch_subseq_fast(int kind, int B, TaskMap tasks, int64_t n_tasks, SubGeo s
 }
 
 int launch_subseq_exact_cands(int kind, int B, TaskMap tasks, const SubCand *cands,
-                              int64_t n_tasks, const double *S64, const int64_t *soff,
+                              CandOut co, int64_t n_tasks, const double *S64, const int64_t *soff,
                               const int64_t *slen, const double *X64, int64_t xstride, int T,
                               double r, double *cost64, hipStream_t st) {
     if (n_tasks <= 0) return WBX_OK;
-    const int64_t nl = n_tasks * kMaxCand;
-    const dim3 grid((unsigned)((nl + 63) / 64));
+    // the list's length stays on the device: a grid for two candidates a task
+    // at most, each block going on by the grid's width
+    const int64_t nb = (n_tasks * 2 + 63) / 64;
+    const dim3 grid((unsigned)(nb < 65536 ? nb : 65536));
     switch (kind == WBX_EUCLIDEAN ? 8 : (B + 7) / 8 * 8) {
 #define C_CASE(B_, U_)                                                                            \
     case B_:                                                                                      \
-        hipLaunchKernelGGL(k_subseq_cand64<B_>, grid, dim3(64), 0, st, tasks, cands, n_tasks, S64, \
+        hipLaunchKernelGGL(k_subseq_cand64<B_>, grid, dim3(64), 0, st, tasks, cands, co, S64,      \
                            soff, slen, X64, xstride, T, r, kind, cost64);                         \
         break;
         SUB_DTW_CASES(C_CASE)
