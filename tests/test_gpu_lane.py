@@ -1,5 +1,5 @@
 """The exact-band float32 lane kernels with a shared x series per wave (matrix
-rows cut into waves of 64 columns) against the group kernel, which computes
+rows cut into waves of 64 columns), with and without weights in SGPRs, against the group kernel, which computes
 the same cells in the same order: bit-identical.  Column counts on both sides
 of whole waves, series shorter than a group of rows, remainders of 8 rows,
 unequal lengths, the narrowest and widest bands; and against the oracle."""
@@ -27,15 +27,17 @@ CASES = [  # nx, ny, tx, ty, r -> band
 ]
 
 
+@pytest.mark.parametrize("metric", ["dtw", "wdtw"])
 @pytest.mark.parametrize("nx,ny,tx,ty,r", CASES)
-def test_shared_x_waves_match_group_kernel(nx, ny, tx, ty, r):
+def test_shared_x_waves_match_group_kernel(nx, ny, tx, ty, r, metric):
     rng = np.random.default_rng(nx * ny + tx)
     X = rng.standard_normal((nx, tx)).cumsum(axis=1)
     Y = rng.standard_normal((ny, ty)).cumsum(axis=1)
     # many rows of x, so that the matrix fills the chip and the lanes run it
     reps = -(-140000 // (nx * ny))
     X = np.tile(X, (reps, 1))
-    call = lambda: wd.pairwise_distance(X, Y, metric="dtw", metric_params={"r": r},
+    params = {"r": r} if metric == "dtw" else {"r": r, "g": 0.1}
+    call = lambda: wd.pairwise_distance(X, Y, metric=metric, metric_params=params,
                                         precision="fp32")
     got = call()
     _lib.set_policy(2)
@@ -44,7 +46,7 @@ def test_shared_x_waves_match_group_kernel(nx, ny, tx, ty, r):
     finally:
         _lib.set_policy(0)
     np.testing.assert_array_equal(got, want)
-    ref = oracle.pairwise(X[:nx], Y, metric="dtw", r=r)
+    ref = oracle.pairwise(X[:nx], Y, metric=metric, r=r, g=0.1)
     # (1 + u)^(lx + ly) and the rounding of the inputs
     tol = (tx + ty + 8) * 2.0**-24 * (1 + np.abs(X).max() ** 2)
     np.testing.assert_allclose(got[:nx], ref, rtol=1e-5, atol=tol)

@@ -300,6 +300,18 @@ int run_pairs(const wbx_metric *m, const PairSpec &ps, Series<T> xs, Series<T> y
         double group_ns = 0.0;
         const bool group =
             !pen && group_plan(B, bd.lx, ps.n_pairs, dbl, wt, &gg, &group_ns);
+        if constexpr (!dbl) {
+            // WDTW matrices of equal lengths: every wave shares its x series
+            // and the weights are scalar, 7 ns a slot alone and 4.3 shared
+            const int64_t ww = wt && policy != 2 ? lane_exact_w_waves(ps, xs.len, ys.len, B) : 0;
+            const double wns = pair_launch_ns(ww, bd.lx, 20.0 + 7.0 * B, 4.3 * B);
+            if (ww && (!lane || wns < lane_ns) && (!group || wns < group_ns)) {
+                ProfScope pf(st, KERN_LANE);
+                return launch_lane_exact_w(
+                    ps, xs, ys, LaneGeo{bd.lx, bd.ly, bd.off, B, bd.ly - bd.lx + bd.off}, weights,
+                    sq, st);
+            }
+        }
         if (group && group_ns < lane_ns) lane = false;
         if (policy == 2 && group) lane = false;  // group kernel wherever it applies
         if (lane) {

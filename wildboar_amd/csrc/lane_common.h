@@ -17,6 +17,12 @@ bool lane_exact_supported(int B);
 int launch_lane_exact(const PairSpec &ps, Series<float> xs, Series<float> ys, const LaneGeo &g,
                       float *sq, hipStream_t st);
 
+// WDTW matrices of series of equal length on such a band (lane_exact_w.hip);
+// the waves of the launch, 0 where it does not apply.
+int64_t lane_exact_w_waves(const PairSpec &ps, int lx, int ly, int B);
+int launch_lane_exact_w(const PairSpec &ps, Series<float> xs, Series<float> ys, const LaneGeo &g,
+                        const float *weights, float *sq, hipStream_t st);
+
 // Four floats at a 4-byte aligned address (one 16-byte load).
 typedef float f4a __attribute__((ext_vector_type(4), aligned(4)));
 

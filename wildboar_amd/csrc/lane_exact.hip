@@ -23,10 +23,10 @@ void launch_exact(const PairSpec &ps, Series<float> xs, Series<float> ys, const 
         ps.mode == PAIR_GRID ? ps.n_pairs / ps.ny * ((ps.ny + 63) / 64) : INT64_MAX;
     if (waves_xu <= waves + waves / 16 && waves_xu <= INT32_MAX)
         hipLaunchKernelGGL((k_lane_dtw_exact<B, U, true>), dim3((unsigned)waves_xu), dim3(64), 0,
-                           st, ps, xs, ys, g, sq);
+                           st, ps, xs, ys, g, nullptr, sq);
     else
         hipLaunchKernelGGL((k_lane_dtw_exact<B, U1, false>), dim3((unsigned)waves), dim3(64), 0, st,
-                           ps, xs, ys, g, sq);
+                           ps, xs, ys, g, nullptr, sq);
 }
 
 }  // namespace

@@ -254,6 +254,39 @@ __device__ __forceinline__ void exact_row(float (&row)[B], const float *yw, floa
     }
 }
 
+// The same for WDTW between series of equal length: slot k weighs w[|k - off|]
+// with off = (B - 1) / 2, the same for every lane and row, so the (B + 1) / 2
+// weights sit in SGPRs and the cell is c = fma(w, d * d, m), four VALU
+// instructions.  ROW0: the prefix sum's weights, w[j - 1] at column j > 0,
+// w[0] at column 0 (columns below 0 are +inf whatever their weight).
+template <int B, bool ROW0>
+__device__ __forceinline__ void exact_row_w(float (&row)[B], const float *yw, float xi,
+                                            const float (&w)[(B + 1) / 2]) {
+    constexpr int off = (B - 1) / 2;
+    float left = WBX_INF_F;
+#pragma unroll
+    for (int k = 0; k < B; ++k) {
+        constexpr int top = (B + 1) / 2 - 1;
+        const int a = k < off ? off - k : k - off;
+        const int e = !ROW0 ? a : (k > off ? a - 1 : 0);
+        const float wk = w[e < top ? e : top];
+        float d = xi - yw[k];
+        if (k == 0)
+            asm("v_min_f32 %0, %2, %0\n\tv_mul_f32 %1, %1, %1\n\tv_fmac_f32 %0, %3, %1"
+                : "+v"(row[k]), "+v"(d)
+                : "v"(row[1]), "s"(wk));
+        else if (k + 1 < B)
+            asm("v_min3_f32 %0, %2, %3, %0\n\tv_mul_f32 %1, %1, %1\n\tv_fmac_f32 %0, %4, %1"
+                : "+v"(row[k]), "+v"(d)
+                : "v"(row[k + 1]), "v"(left), "s"(wk));
+        else
+            asm("v_min_f32 %0, %2, %0\n\tv_mul_f32 %1, %1, %1\n\tv_fmac_f32 %0, %3, %1"
+                : "+v"(row[k]), "+v"(d)
+                : "v"(left), "s"(wk));
+        left = row[k];
+    }
+}
+
 // x of a wave that shares one series: constant address space, so the loads
 // are scalar.
 typedef const float __attribute__((address_space(4))) *cfloat;
@@ -267,9 +300,12 @@ typedef const float __attribute__((address_space(4))) *cfloat;
 // B = 101), longer groups gain nothing.  2000 x 2000 x 512 on one box, x per
 // lane -> XU: B = 23 2.92 -> 2.67 ms, B = 49 5.52 -> 5.23, B = 75 8.83 -> 8.10,
 // B = 101 12.02 -> 10.73, B = 111 13.05 -> 11.70.
-template <int B, int U, bool XU>
+// WT: WDTW (equal lengths, XU; weights: at least (B + 1) / 2 values).  1000 x
+// 1000 x 256, B = 49: 1205 us on the group kernel, 873 us.
+template <int B, int U, bool XU, bool WT = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_lane_dtw_exact(
-    PairSpec ps, Series<float> xs, Series<float> ys, LaneGeo g, float *__restrict__ sq) {
+    PairSpec ps, Series<float> xs, Series<float> ys, LaneGeo g,
+    const float *__restrict__ weights, float *__restrict__ sq) {
     constexpr int W = B + U - 1;
     static_assert(U % 4 == 0, "groups of whole 16-byte loads");
     const int lane = threadIdx.x;
@@ -306,10 +342,31 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         if ((m & 7) == 7) __builtin_amdgcn_sched_barrier(0);
     }
     __builtin_amdgcn_sched_barrier(0);
+    float w[WT ? (B + 1) / 2 : 1];
+    if constexpr (WT) {
+        const cfloat ws = (cfloat)weights;
+#pragma unroll
+        for (int q = 0; q < (B + 1) / 2; ++q) w[q] = ws[q];
+    }
+    auto one_row = [&](const float *y, float xi, auto row0) {
+        if constexpr (WT)
+            exact_row_w<B, decltype(row0)::value>(row, y, xi, w);
+        else
+            exact_row<B>(row, y, xi);
+    };
     // leading rows one at a time so the rest is a whole number of groups
-    const int rem = lx % U;
-    for (int i = 0; i < rem; ++i) {
-        exact_row<B>(row, yw, X[i]);
+    // (WDTW: row 0 among them, its weights differ)
+    int i_begin = 0;
+    if constexpr (WT) {
+        one_row(yw, X[0], std::true_type());
+#pragma unroll
+        for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
+        yw[W - 1] = ldy(Y, 1 - off + W - 1, ly);
+        i_begin = 1;
+    }
+    const int rem = i_begin + (lx - i_begin) % U;
+    for (int i = i_begin; i < rem; ++i) {
+        one_row(yw, X[i], std::false_type());
 #pragma unroll
         for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
         yw[W - 1] = ldy(Y, i + 1 - off + W - 1, ly);
@@ -351,7 +408,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
             }
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) exact_row<B>(row, yw + u, xv[u]);
+        for (int u = 0; u < U; ++u) one_row(yw + u, xv[u], std::false_type());
 #pragma unroll
         for (int m = 0; m < W - U; ++m) yw[m] = yw[m + U];
 #pragma unroll
