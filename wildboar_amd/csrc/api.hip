@@ -267,7 +267,7 @@ int run_pairs(const wbx_metric *m, const PairSpec &ps, Series<T> xs, Series<T> y
         // columns, no slot outside the matrix
         FullGeo fg{};
         if (!wt && !pen && bd.w >= (xs.len < ys.len ? xs.len : ys.len) && policy != 2 &&
-            full_plan(xs.len, ys.len, !std::is_same<T, float>::value, &fg)) {
+            full_plan(xs.len, ys.len, ps.n_pairs, !std::is_same<T, float>::value, &fg)) {
             ProfScope pf(st, KERN_FULL);
             return launch_full_dtw<T>(ps, xs, ys, sq, st);
         }

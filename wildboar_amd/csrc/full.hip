@@ -23,6 +23,8 @@
 // (bit-exact: _elastic.pyx:893-940 with w = 1).
 #pragma clang fp contract(off)
 
+#include <type_traits>
+
 #include "wbx_internal.h"
 
 namespace wbx {
@@ -100,11 +102,11 @@ __device__ __forceinline__ T fldx(const T *__restrict__ X, int i, int lx) {
     return X[i < 0 ? 0 : (i >= lx ? lx - 1 : i)];
 }
 
-// Waves per SIMD the register allocation is held to: float64 lanes of 24
+// Waves per SIMD the register allocation is held to: float64 lanes of 21 to 24
 // columns fit three waves' 168 registers without spills (184 otherwise).
 template <typename T, int S>
 constexpr int full_waves() {
-    return sizeof(T) == 8 && S == 24 ? 3 : 1;
+    return sizeof(T) == 8 && S >= 21 && S <= 24 ? 3 : 1;
 }
 
 template <typename T, int S, int U>
@@ -134,28 +136,38 @@ k_full_dtw(PairSpec ps, Series<T> xs, Series<T> ys, FullGeo g, T *__restrict__ s
     L.dg = q == 0 ? (T)0 : finf<T>();  // D(-1, -1) = 0
     L.l = finf<T>();
     L.r = -q;
-    // fill: steps [0, n - 1) (lanes before row 0 keep their state)
-    const int fill = g.n - 1;
-    for (int s = 0; s < fill; ++s) fstep<T, S, true>(L, fldx(X, L.r, lx), lx);
-    // steady: steps [n - 1, lx), every lane inside rows [0, lx)
-    const int steady = lx - fill > 0 ? lx - fill : 0;
-    const int rem = steady % U;
-    for (int s = 0; s < rem; ++s) fstep<T, S, false>(L, fldx(X, L.r, lx), lx);
+    // Steps go in groups of U, the next group's x values loaded during the
+    // current one; steps with a lane outside its rows (the first n - 1 and
+    // those past row lx - 1 of lane 0) keep that lane's state through selects.
+    // They go in groups too, except in the float64 lanes held to three waves
+    // (whose registers that would spill): one at a time.
+    constexpr bool kEdgeGroups = full_waves<T, S>() == 1;
+    const int steps = lx + g.n - 1;
+    int s = 0;
+    if constexpr (!kEdgeGroups) {
+        for (; s < g.n - 1; ++s) fstep<T, S, true>(L, fldx(X, L.r, lx), lx);
+        const int rem = s < lx ? (lx - s) % U : 0;
+        for (int e = 0; e < rem; ++e, ++s) fstep<T, S, false>(L, fldx(X, L.r, lx), lx);
+    }
     T xv[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) xv[u] = fldx(X, L.r + u, lx);
-    for (int s = rem; s < steady; s += U) {
+    auto group = [&](auto edge) {
         T xn[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) xn[u] = fldx(X, L.r + U + u, lx);
 #pragma unroll
-        for (int u = 0; u < U; ++u) fstep<T, S, false>(L, xv[u], lx);
+        for (int u = 0; u < U; ++u) fstep<T, S, decltype(edge)::value>(L, xv[u], lx);
 #pragma unroll
         for (int u = 0; u < U; ++u) xv[u] = xn[u];
-    }
-    // drain: up to step lx + n - 2 (lanes past row lx - 1 keep it)
-    const int drain = lx + g.n - 1 - fill - steady;
-    for (int s = 0; s < drain; ++s) fstep<T, S, true>(L, fldx(X, L.r, lx), lx);
+    };
+    if constexpr (kEdgeGroups)
+        for (; s < g.n - 1; s += U) group(std::true_type());
+    for (; s + U <= lx; s += U) group(std::false_type());
+    if constexpr (kEdgeGroups)
+        for (; s < steps; s += U) group(std::true_type());
+    else
+        for (; s < steps; ++s) fstep<T, S, true>(L, fldx(X, L.r, lx), lx);
 
     const int jf = ly - 1;
     if (valid && jf >= c0 && jf < c0 + S) {
@@ -167,36 +179,42 @@ k_full_dtw(PairSpec ps, Series<T> xs, Series<T> ys, FullGeo g, T *__restrict__ s
     }
 }
 
-constexpr int kFullS32[] = {4, 8, 12, 16, 24, 32};
-constexpr int kFullS64[] = {4, 8, 12, 16, 24};
+constexpr int kFullS32[] = {4,  6,  8,  10, 12, 14, 15, 16, 17, 18, 19, 20,
+                            21, 22, 23, 24, 25, 26, 27, 28, 30, 32};
+constexpr int kFullS64[] = {4,  6,  8,  10, 12, 14, 15, 16, 17, 18, 19,
+                            20, 21, 22, 23, 24, 25, 26, 27, 28};
 
 template <typename T, int S>
 void launch_full_one(const PairSpec &ps, Series<T> xs, Series<T> ys, const FullGeo &g, T *sq,
                      hipStream_t st) {
     const dim3 grid((unsigned)((ps.n_pairs + g.P - 1) / g.P));
-    hipLaunchKernelGGL((k_full_dtw<T, S, 4>), grid, dim3(64), 0, st, ps, xs, ys, g, sq);
+    hipLaunchKernelGGL((k_full_dtw<T, S, (S <= 8 ? 8 : 4)>), grid, dim3(64), 0, st, ps, xs, ys, g, sq);
 }
 
 }  // namespace
 
 // Columns per lane S and lanes per pair n = ceil(ly / S) <= 64: the compiled S
-// with the most matrix cells per VALU instruction of a wave step, counting
-// the 64 / n pairs a wave holds, k S + 4 instructions per lane step (cells,
-// the DPP move, its group-edge select, loop) and the fill and drain steps.
-bool full_plan(int lx, int ly, bool fp64, FullGeo *g) {
+// with the smallest time for n_pairs pairs.  Large calls want the cells of a
+// wave step to be matrix cells (64 / n pairs a wave, n S columns for ly, n - 1
+// steps of fill and drain), small ones few columns in turn.  The figures are
+// the group kernel's kind (pair_launch_ns), measured on series of 275: 50
+// pairs float64 81 us at S = 24, 36 us at S = 6; 400000 pairs of 100, 844 us
+// at S = 24, 707 us at S = 26.
+bool full_plan(int lx, int ly, int64_t n_pairs, bool fp64, FullGeo *g) {
     const int *tab = fp64 ? kFullS64 : kFullS32;
     const int nt = fp64 ? (int)(sizeof(kFullS64) / sizeof(int))
                         : (int)(sizeof(kFullS32) / sizeof(int));
-    const double k = fp64 ? 5.0 : 3.0;
-    double best = -1.0;
+    double best = 0.0;
     for (int t = 0; t < nt; ++t) {
         const int S = tab[t];
         const int n = (ly + S - 1) / S;
         if (n > 64) continue;
         const int P = 64 / n;
-        const double score = (double)P * ly / (k * S + 4.0) * lx / (double)(lx + n - 1);
-        if (score > best) {
-            best = score;
+        const double time =
+            pair_launch_ns((n_pairs + P - 1) / P, lx + n - 1, fp64 ? 35.0 + 10.0 * S : 30.0 + 5.2 * S,
+                           fp64 ? 22.0 + 9.5 * S : 17.0 + 3.25 * S);
+        if (best == 0.0 || time < best) {
+            best = time;
             g->S = S;
             g->n = n;
             g->P = P;
@@ -213,17 +231,22 @@ int launch_full_dtw(const PairSpec &ps, Series<T> xs, Series<T> ys, T *sq, hipSt
     if (xs.lens || ys.lens) return fail(WBX_EUNSUPPORTED, "full kernel: needs one geometry");
     FullGeo g{};
     const bool dbl = std::is_same<T, double>::value;
-    if (!full_plan(xs.len, ys.len, dbl, &g))
+    if (!full_plan(xs.len, ys.len, ps.n_pairs, dbl, &g))
         return fail(WBX_EUNSUPPORTED, "full kernel: %d columns", ys.len);
     switch (g.S) {
-        case 4: launch_full_one<T, 4>(ps, xs, ys, g, sq, st); break;
-        case 8: launch_full_one<T, 8>(ps, xs, ys, g, sq, st); break;
-        case 12: launch_full_one<T, 12>(ps, xs, ys, g, sq, st); break;
-        case 16: launch_full_one<T, 16>(ps, xs, ys, g, sq, st); break;
-        case 24: launch_full_one<T, 24>(ps, xs, ys, g, sq, st); break;
+#define WBX_F(SV) \
+    case SV: launch_full_one<T, SV>(ps, xs, ys, g, sq, st); break;
+        WBX_F(4) WBX_F(6) WBX_F(8) WBX_F(10) WBX_F(12) WBX_F(14) WBX_F(15) WBX_F(16) WBX_F(17)
+        WBX_F(18) WBX_F(19) WBX_F(20) WBX_F(21) WBX_F(22) WBX_F(23) WBX_F(24) WBX_F(25) WBX_F(26)
+        WBX_F(27) WBX_F(28)
+#undef WBX_F
+        case 30:
         case 32:
             if constexpr (!std::is_same<T, double>::value) {
-                launch_full_one<T, 32>(ps, xs, ys, g, sq, st);
+                if (g.S == 30)
+                    launch_full_one<T, 30>(ps, xs, ys, g, sq, st);
+                else
+                    launch_full_one<T, 32>(ps, xs, ys, g, sq, st);
                 break;
             }
             [[fallthrough]];

@@ -286,7 +286,7 @@ struct FullGeo {
     int lx, ly;
     int n, P, S;  // lanes per pair, pairs per wave, columns per lane
 };
-bool full_plan(int lx, int ly, bool fp64, FullGeo *g);
+bool full_plan(int lx, int ly, int64_t n_pairs, bool fp64, FullGeo *g);
 template <typename T>
 int launch_full_dtw(const PairSpec &ps, Series<T> xs, Series<T> ys, T *sq, hipStream_t st);
 template <typename T>
