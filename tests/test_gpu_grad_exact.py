@@ -1,0 +1,56 @@
+"""Differentiable DTW on exact-band lanes, with x from SGPRs (grids of whole
+waves) and from VGPRs (lists of pairs): bands on both sides of the 32-slot
+decision words and the narrowest and widest exact ones.  D is homogeneous of
+degree 1 in (x, y) jointly, so <dD/dx, x> + <dD/dy, y> = D, which holds only
+when the walked path has the cost the recurrence found."""
+
+import numpy as np
+import pytest
+import torch
+
+from wildboar_amd.dtw import dtw, paired_dtw
+
+pytestmark = pytest.mark.gpu
+
+
+def _grads(fn, X, Y, G, r):
+    X, Y = X.clone().requires_grad_(True), Y.clone().requires_grad_(True)
+    D = fn(X, Y, r)
+    gx, gy = torch.autograd.grad((D * G).sum(), (X, Y))
+    return D.detach(), gx, gy
+
+
+@pytest.mark.parametrize("data", ["walks", "integers"])
+@pytest.mark.parametrize("slots", [9, 31, 33, 49, 63, 65, 97, 111])
+def test_exact_forms(slots, data):
+    rng = np.random.default_rng(slots)
+    nx, ny, t = 260, 64, 131  # more pairs than the few-pairs form takes
+    r = (slots - 1) / 2 / t + 1e-6
+
+    def series(n):
+        if data == "integers":
+            return rng.integers(-2, 3, (n, t))
+        return rng.standard_normal((n, t)).cumsum(axis=1)
+
+    X = torch.from_numpy(series(nx).astype(np.float32)).cuda()
+    Y = torch.from_numpy(series(ny).astype(np.float32)).cuda()
+    G = torch.from_numpy(rng.uniform(0.5, 2.0, (nx, ny))).cuda()
+    D, gx, gy = _grads(dtw, X, Y, G, r)
+    Xp, Yp, Gp = X.repeat_interleave(ny, 0), Y.repeat(nx, 1), G.reshape(-1)
+    Dp, px, py = _grads(paired_dtw, Xp, Yp, Gp, r)
+    assert torch.equal(D.reshape(-1), Dp)
+
+    # sums of m float32 terms are within m u of the sum of their magnitudes
+    u = 2.0**-24
+    qx, qy = px.double().reshape(nx, ny, t), py.double().reshape(nx, ny, t)
+    assert ((gx.double() - qx.sum(1)).abs() <= ny * u * qx.abs().sum(1) + 1e-30).all()
+    assert ((gy.double() - qy.sum(0)).abs() <= nx * u * qy.abs().sum(0) + 1e-30).all()
+
+    # a path has at most 2 t cells; each adds terms of at most G/D |x|max (|x| +
+    # |y|)max to the products, rounded a few times in sums of at most t terms;
+    # D^2 is a float32 sum of at most 2 t squares
+    pos = Dp > 0
+    hom = (px.double() * Xp.double()).sum(1) + (py.double() * Yp.double()).sum(1)
+    big = torch.maximum(Xp.abs().amax(1), Yp.abs().amax(1)).double()
+    bound = 2 * t * u * (Gp * Dp + 2 * t * Gp / Dp.clamp(min=1e-30) * 4 * big**2)
+    assert ((hom - Gp * Dp).abs() <= bound)[pos].all()

@@ -24,139 +24,10 @@
 //                    row's and the column's sums.
 //  k_sum_*           fixed-order sums of per-pair gradients into dX, dY
 //                    (the backward is bitwise deterministic).
-#include "lane_common.h"
+#include "lane_train.h"
 #include "train_small.h"
 
 namespace wbx {
-
-// One cell after m = min3(up, left, dg):
-//   bd = (m == dg), bu = (m == up)          two compares into SGPR masks
-//   c  = m + (x - y)^2                      sub + fmac
-//   pd = 2 pd + bd, pu = 2 pu + bu          add-with-carry shifts each bit in
-// Each mask is read three VALU instructions after it is written, which covers
-// the wait states gfx950 requires between a VALU mask write and a VALU carry
-// read, so the block needs no s_nop.  Seven VALU instructions per cell.
-__device__ __forceinline__ float train_cell(float m, float dg, float up, float x, float y,
-                                            uint32_t &pd, uint32_t &pu) {
-    float c = m, d;
-    uint64_t sa, sb;
-    asm("v_cmp_eq_f32_e64 %[sa], %[c], %[dg]\n\t"
-        "v_cmp_eq_f32_e64 %[sb], %[c], %[up]\n\t"
-        "v_sub_f32_e32 %[d], %[x], %[y]\n\t"
-        "v_fmac_f32_e32 %[c], %[d], %[d]\n\t"
-        "v_addc_co_u32_e64 %[pd], %[sa], %[pd], %[pd], %[sa]\n\t"
-        "v_addc_co_u32_e64 %[pu], %[sb], %[pu], %[pu], %[sb]"
-        : [c] "+v"(c), [pd] "+v"(pd), [pu] "+v"(pu), [d] "=&v"(d), [sa] "=&s"(sa),
-          [sb] "=&s"(sb)
-        : [dg] "v"(dg), [up] "v"(up), [x] "v"(x), [y] "v"(y));
-    return c;
-}
-
-template <int BP>
-__device__ __forceinline__ void train_row(float (&row)[BP], const float *yw, float xi,
-                                          const float (&pen)[8], uint32_t *pd, uint32_t *pu) {
-    float left = WBX_INF_F;
-#pragma unroll
-    for (int k = 0; k < BP; ++k) {
-        const float up = (k + 1 < BP) ? row[k + 1] : WBX_INF_F;
-        const float dg = row[k];
-        const float m = fminf(fminf(up, left), dg);
-        const float c = train_cell(m, dg, up, xi, yw[k], pd[k >> 5], pu[k >> 5]);
-        row[k] = c;
-        left = c;
-    }
-#pragma unroll
-    for (int q = 1; q < 8; ++q) row[BP - 8 + q] = fmaxf(row[BP - 8 + q], pen[q]);
-}
-
-// Plane words of wave v, row i, lane l: 2 NW words starting at
-// dirs[((v * lx + i) * 64 + l) * 2 NW], as (diag word w, up word w) pairs, so a
-// lane's row is one contiguous piece and a wave's row is 64 of them in a row.
-__device__ __forceinline__ int64_t plane_base(int64_t wave, int lx, int i, int nw2, int lane) {
-    return (((int64_t)wave * lx + i) * 64 + lane) * nw2;
-}
-
-template <int BP>
-__device__ __forceinline__ void store_planes(uint32_t *__restrict__ dirs, int64_t wave, int lane,
-                                             int lx, int i, uint32_t (&pd)[(BP + 31) / 32],
-                                             uint32_t (&pu)[(BP + 31) / 32]) {
-    constexpr int NW = (BP + 31) / 32;
-    uint2 *d = (uint2 *)(dirs + plane_base(wave, lx, i, 2 * NW, lane));
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-        d[w] = make_uint2(pd[w], pu[w]);
-        pd[w] = 0u;
-        pu[w] = 0u;
-    }
-}
-
-template <int BP, int U>
-__global__ __launch_bounds__(64) void k_lane_train(PairSpec ps, Series<float> xs, Series<float> ys,
-                                                   LaneGeo g, float *__restrict__ sq,
-                                                   uint32_t *__restrict__ dirs) {
-    constexpr int W = BP + U - 1;
-    constexpr int NW = (BP + 31) / 32;
-    const int lane = threadIdx.x;
-    const int64_t wave = blockIdx.x;
-    const int64_t p0 = wave * 64 + lane;
-    const int64_t p = p0 < ps.n_pairs ? p0 : ps.n_pairs - 1;
-    int64_t a, b;
-    decode_pair(ps, p, a, b);
-    const float *__restrict__ X = xs.row(a);
-    const float *__restrict__ Y = ys.row(b);
-    const int lx = g.lx, ly = g.ly, off = g.off, B = g.B;
-
-    float row[BP];
-#pragma unroll
-    for (int k = 0; k < BP; ++k) row[k] = (k == off) ? 0.0f : WBX_INF_F;
-    float pen[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) pen[q] = (BP - 8 + q == B) ? WBX_INF_F : -WBX_INF_F;
-    uint32_t pd[NW], pu[NW];
-#pragma unroll
-    for (int w = 0; w < NW; ++w) pd[w] = pu[w] = 0u;
-    float yw[W];
-#pragma unroll
-    for (int m = 0; m < W; ++m) yw[m] = ldy(Y, m - off, ly);
-
-    const int rem = lx % U;
-    for (int i = 0; i < rem; ++i) {
-        train_row<BP>(row, yw, X[i], pen, pd, pu);
-        store_planes<BP>(dirs, wave, lane, lx, i, pd, pu);
-#pragma unroll
-        for (int m = 0; m < W - 1; ++m) yw[m] = yw[m + 1];
-        yw[W - 1] = ldy(Y, i + 1 - off + W - 1, ly);
-    }
-    float xv[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) xv[u] = X[rem + u < lx ? rem + u : lx - 1];
-    for (int i0 = rem; i0 < lx; i0 += U) {
-        float xn[U], yn[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int inext = i0 + U + u;
-            xn[u] = X[inext < lx ? inext : lx - 1];
-            yn[u] = ldy(Y, i0 + U - off + W - U + u, ly);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            train_row<BP>(row, yw + u, xv[u], pen, pd, pu);
-            store_planes<BP>(dirs, wave, lane, lx, i0 + u, pd, pu);
-        }
-#pragma unroll
-        for (int m = 0; m < W - U; ++m) yw[m] = yw[m + U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            yw[W - U + u] = yn[u];
-            xv[u] = xn[u];
-        }
-    }
-    float res = WBX_INF_F;
-#pragma unroll
-    for (int k = 0; k < BP; ++k)
-        if (k == g.kf) res = row[k];
-    if (p0 < ps.n_pairs) sq[p0] = res;
-}
 
 // Sum over the 64 lanes in a fixed order: a running sum within each row of 16
 // lanes (DPP row_shr 1, 2, 4, 8), then rows folded in with row_bcast 15 and
@@ -245,15 +116,15 @@ __global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ src
 }
 
 // Bit of slot k in its plane word: slots are shifted in from the low end, so
-// slot k of word w sits at bit (count_w - 1 - (k - 32 w)).
+// slot k of word w sits at bit (count_w - 1 - (k - 32 w)); the last word holds
+// the lastc slots that the forward computed past the others.
 template <int BP>
 __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
                                                        const float *__restrict__ sq,
                                                        const double *__restrict__ G,
                                                        const uint32_t *__restrict__ dirs,
-                                                       GradOut go) {
+                                                       int lastc, GradOut go) {
     constexpr int NW = (BP + 31) / 32;
-    constexpr int LASTC = BP - 32 * (NW - 1);
     const int lane = threadIdx.x;
     const int64_t wave = blockIdx.x;
     const int64_t p0 = wave * 64 + lane;
@@ -341,7 +212,7 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
             bool isd = false;
 #pragma unroll
             for (int w = NW - 1; w >= 0; --w) {
-                const int cnt_w = (w == NW - 1) ? LASTC : 32;
+                const int cnt_w = (w == NW - 1) ? lastc : 32;
                 uint32_t msk = wd[r][w] | wu[r][w];
                 if (w > wk) msk = 0u;
                 if (w == wk) msk &= ~0u << (cnt_w - 1 - (k - 32 * w));
@@ -506,15 +377,16 @@ static int train_bp(int B) { return (B + 7) / 8 * 8; }
 template <int BP, int U>
 static void train_fwd_one(const PairSpec &ps, Series<float> xs, Series<float> ys, LaneGeo g,
                           float *sq, uint32_t *dirs, hipStream_t st) {
-    hipLaunchKernelGGL((k_lane_train<BP, U>), dim3((unsigned)((ps.n_pairs + 63) / 64)), dim3(64), 0,
+    hipLaunchKernelGGL((k_lane_train<BP, U, false, false>), dim3((unsigned)((ps.n_pairs + 63) / 64)), dim3(64), 0,
                        st, ps, xs, ys, g, sq, dirs);
 }
 
 template <int BP>
 static void train_bwd_one(const PairSpec &ps, LaneGeo g, const float *sq, const double *G,
                           const uint32_t *dirs, GradOut go, hipStream_t st) {
+    const int slots = lane_exact_supported(g.B) ? g.B : BP;  // as the forward computed
     hipLaunchKernelGGL((k_lane_backtrack<BP>), dim3((unsigned)((ps.n_pairs + 63) / 64)), dim3(64), 0,
-                       st, ps, g, sq, G, dirs, go);
+                       st, ps, g, sq, G, dirs, slots - 32 * ((BP + 31) / 32 - 1), go);
 }
 
 #define TRAIN_CASES(X)                                                                          \
@@ -666,6 +538,10 @@ int wbx_dev_dtw_train_forward(const wbx_metric *metric, int mode, const float *X
     Series<float> xs{X, x_stride, (int)tx, nullptr}, ys{Y, y_stride, (int)ty, nullptr};
     const Band bd = make_band((int)tx, (int)ty, metric->r);
     if (small_train_ok(ps.n_pairs, bd)) return small_train_forward(ps, xs, ys, bd, D, state, st);
+    if (lane_exact_supported(tg.g.B)) {
+        RCT(launch_lane_train_exact(ps, xs, ys, tg.g, sq, dirs, st));
+        return launch_finish<float>(ps, sq, D, ny, st);
+    }
     switch (tg.BP) {
 #define FWD_CASE(BPV, UV) \
     case BPV: train_fwd_one<BPV, UV>(ps, xs, ys, tg.g, sq, dirs, st); break;

@@ -21,6 +21,7 @@
 // (8 waves): forward 221 -> 36 us, backward 334 -> 65 us.
 #include <type_traits>
 
+#include "lane_train.h"
 #include "train_small.h"
 
 namespace wbx {
@@ -45,22 +46,11 @@ __device__ __forceinline__ float sshl1(float v) {
 }
 
 // c = min3(up, left, dg) + (x - y)^2 with the two decision bits shifted into
-// pd (min came from diag) and pu (from up); see train_cell in train.hip.
+// pd (clear: the minimum came from diag) and pu (from up); see train_cell.
 __device__ __forceinline__ float small_cell(float up, float left, float dg, float x, float y,
                                             uint32_t &pd, uint32_t &pu) {
-    const float m = fminf(fminf(up, left), dg);
-    float c = m, d;
-    uint64_t sa, sb;
-    asm("v_cmp_eq_f32_e64 %[sa], %[c], %[dg]\n\t"
-        "v_cmp_eq_f32_e64 %[sb], %[c], %[up]\n\t"
-        "v_sub_f32_e32 %[d], %[x], %[y]\n\t"
-        "v_fmac_f32_e32 %[c], %[d], %[d]\n\t"
-        "v_addc_co_u32_e64 %[pd], %[sa], %[pd], %[pd], %[sa]\n\t"
-        "v_addc_co_u32_e64 %[pu], %[sb], %[pu], %[pu], %[sb]"
-        : [c] "+v"(c), [pd] "+v"(pd), [pu] "+v"(pu), [d] "=&v"(d), [sa] "=&s"(sa),
-          [sb] "=&s"(sb)
-        : [dg] "v"(dg), [up] "v"(up), [x] "v"(x), [y] "v"(y));
-    return c;
+    train_cell<false>(dg, up, left, x, y, pd, pu);
+    return dg;
 }
 
 struct SmallGeo {
@@ -119,7 +109,8 @@ __device__ __forceinline__ uint32_t small_step(SLane<S> &L, int u, float x, int 
     }
     L.row[0] = SEL ? (act ? c0 : L.row[0]) : c0;
     L.l = L.row[S - 1];
-    return pd | pu << 4;  // slot m at bit S - 1 - m of each nibble
+    // slot m at bit S - 1 - m of each nibble, set where the minimum came from
+    return (pd | pu << 4) ^ ((1u << S) - 1u) * 0x11u;
 }
 
 __device__ __forceinline__ void small_loads(const float *__restrict__ X,
