@@ -2,7 +2,8 @@
 waves) and from VGPRs (lists of pairs): bands on both sides of the 32-slot
 decision words and the narrowest and widest exact ones.  D is homogeneous of
 degree 1 in (x, y) jointly, so <dD/dx, x> + <dD/dy, y> = D, which holds only
-when the walked path has the cost the recurrence found."""
+when the walked path has the cost the recurrence found.  Grids of one and of
+several waves per x series and of waves across series."""
 
 import numpy as np
 import pytest
@@ -21,10 +22,11 @@ def _grads(fn, X, Y, G, r):
 
 
 @pytest.mark.parametrize("data", ["walks", "integers"])
+@pytest.mark.parametrize("nx,ny", [(260, 64), (130, 128), (237, 70)])  # more than few pairs
 @pytest.mark.parametrize("slots", [9, 31, 33, 49, 63, 65, 97, 111])
-def test_exact_forms(slots, data):
+def test_exact_forms(slots, nx, ny, data):
     rng = np.random.default_rng(slots)
-    nx, ny, t = 260, 64, 131  # more pairs than the few-pairs form takes
+    t = 131
     r = (slots - 1) / 2 / t + 1e-6
 
     def series(n):

@@ -19,9 +19,10 @@
 //                    enters at slot k and moves left until the first cell
 //                    whose decision is diag or up; that exit is a bit scan of
 //                    (diag | up) over the row's words, which sit at addresses
-//                    independent of the path and are fetched one row ahead.
-//                    The cells of the segment add (x_i - y_j) G / D to the
-//                    row's and the column's sums.
+//                    independent of the path and are fetched rows ahead.
+//                    The row's sum of (x_i - y_j) G / D comes from prefix
+//                    sums of y at once, a column's from prefix sums of x as
+//                    soon as no lane's path can reach it any more.
 //  k_sum_*           fixed-order sums of per-pair gradients into dX, dY
 //                    (the backward is bitwise deterministic).
 #include "lane_train.h"
@@ -45,11 +46,9 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 #undef WBX_DPP
 
-// Where the per-pair gradients go.  For column j of pair (a, b) the walk keeps
-// u = coef * (number of path cells in column j) and v = coef * (sum of x_i
-// over those cells) and writes the one term dD/dy_j = y_j u - v when the
-// column's 8-column window is complete; the window's 8 y values are fetched
-// one window ahead from YP, so the walk never waits on them.
+// Where the per-pair gradients go.  Column j of pair (a, b) has the one term
+// dD/dy_j = y_j u - v, u = coef * (number of path cells in column j) and
+// v = coef * (sum of x_i over those cells), written 8 columns at a time.
 struct GradOut {
     int mode;          // 0: GRID pairs, 1: DIAG (paired) pairs
     int xred;          // GRID with ny % 64 == 0: a wave's lanes share one x row
@@ -66,20 +65,35 @@ struct GradOut {
     // lanes of a wave hold neighbouring pairs, so their loads coalesce
     const float *XT;
     const double *PT;
+    // prefix sums of X, PX[i * pxi + a * pxa]: rows of one series where the
+    // lanes of a wave share it, else transposed like PT
+    const double *PX;
+    int64_t pxi, pxa;
 };
 
-// PT[j * ny + b] = sum of y_b[0 .. j) in float64; one wave per series, 64
-// columns at a time with a shuffle scan (the sum order is fixed: the result
-// is deterministic).
-// YP[b * lyp + j] = y_b[j], zero for ly <= j < lyp.
-__global__ __launch_bounds__(64) void k_prefix_t(const float *__restrict__ Y, int64_t ny, int ly,
-                                                 int64_t stride, double *__restrict__ PT,
+// Prefix sums P_b[j] = y_b[0] + ... + y_b[j - 1] in float64, j in [0, ly]; one
+// wave per series, 64 columns at a time with a shuffle scan (the sum order is
+// fixed: the result is deterministic).  ROWS: out[b * (ly + 1) + j]; else
+// transposed, out[j * n + b], through an LDS tile so that a block's 16 series
+// write whole lines (a scattered store per sum took 116 us longer for twice
+// 65,536 series of 64).
+// YP[b * lyp + j] = y_b[j], zero for ly <= j < lyp (lyp 0: not wanted).
+template <bool ROWS>
+__global__ __launch_bounds__(1024) void k_prefix(const float *__restrict__ Y, int64_t n, int ly,
+                                                 int64_t stride, double *__restrict__ out,
                                                  float *__restrict__ YP, int lyp) {
-    const int64_t b = blockIdx.x;
-    const int lane = threadIdx.x;
-    const float *y = Y + b * stride;
-    if (lane == 0) PT[b] = 0.0;
-    for (int j = lane; j < lyp; j += 64) YP[b * lyp + j] = j < ly ? y[j] : 0.0f;
+    __shared__ double tile[16][65];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t b0 = (int64_t)blockIdx.x * 16, b = b0 + w;
+    const bool mine = b < n;
+    const float *y = Y + (mine ? b : n - 1) * stride;
+    if (ROWS) {
+        if (mine && lane == 0) out[b * (ly + 1)] = 0.0;
+    } else if (threadIdx.x < 16 && b0 + threadIdx.x < n) {
+        out[b0 + threadIdx.x] = 0.0;
+    }
+    if (mine)
+        for (int j = lane; j < lyp; j += 64) YP[b * lyp + j] = j < ly ? y[j] : 0.0f;
     double carry = 0.0;
     for (int j0 = 0; j0 < ly; j0 += 64) {
         const int j = j0 + lane;
@@ -90,8 +104,16 @@ __global__ __launch_bounds__(64) void k_prefix_t(const float *__restrict__ Y, in
             if (lane >= d) s += o;
         }
         s += carry;
-        if (j < ly) PT[(int64_t)(j + 1) * ny + b] = s;
         carry = __shfl(s, 63);
+        if (ROWS) {
+            if (mine && j < ly) out[b * (ly + 1) + j + 1] = s;
+        } else {
+            tile[w][lane] = s;
+            __syncthreads();
+            const int q = threadIdx.x & 15, c = threadIdx.x >> 4;
+            if (b0 + q < n && j0 + c < ly) out[(j0 + c + 1) * n + b0 + q] = tile[q][c];
+            __syncthreads();
+        }
     }
 }
 
@@ -139,42 +161,66 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
     const double D = sqrt((double)sq[p]);
     const double coefd = (active && D > 0.0) ? G[p] / D : 0.0;
     const float coef = (float)coefd;
-    // Columns are finished in decreasing order, each exactly once: their
-    // terms go to the lane's CW-column window in LDS (slot col % CW) and out
-    // as one vector store per CW columns when column col % CW == 0 completes
-    // it (columns >= ly of the top window stay the zeros written first).  A
-    // column costs two LDS writes, not a shift of two register windows, in a
-    // loop every lane of the wave runs as often as its busiest lane.
-    constexpr int CW = 8;
-    typedef float fcw __attribute__((ext_vector_type(CW)));
-    __shared__ float wbuf[2][CW][64];  // u, v of column slot e, lane
-#pragma unroll
-    for (int e = 0; e < CW; ++e) wbuf[0][e][lane] = wbuf[1][e][lane] = 0.0f;
-    fcw *__restrict__ gww = (fcw *)(go.gw + p * go.lyp);
-    const fcw *__restrict__ ypw = (const fcw *)(go.YP + b * go.lyp);
-    fcw yv_ = ypw[(ly - 1) / CW];  // y of the first window to complete
-    auto finish = [&](int col, float u, float v) {
-        const int e = col & (CW - 1);
-        wbuf[0][e][lane] = u;
-        wbuf[1][e][lane] = v;
-        if (e == 0) {  // columns col .. col + CW - 1 are complete
-            fcw wu, wv;
-#pragma unroll
-            for (int q = 0; q < CW; ++q) {
-                wu[q] = wbuf[0][q][lane];
-                wv[q] = wbuf[1][q][lane];
-            }
-            if (active) gww[col / CW] = wu * yv_ - wv;
-            yv_ = ypw[col >= CW ? col / CW - 1 : 0];  // the next window down
-        }
-    };
-
+    // A column's terms need its first and last path row.  The walk of a row
+    // notes, at the column where the row ends, its exit and entry slots (one
+    // LDS write; of several rows ending in a column the topmost stays), and
+    // columns that no later row can reach are finished by all lanes together,
+    // CG at a time from the right: rows of a column are contiguous and one
+    // row's columns too, so the last note seen gives both rows, and the sum of
+    // x over them is a difference of prefix sums.  Finishing each row's
+    // columns as the row leaves them runs every wave as long as the longest
+    // horizontal run among its 64 paths, row after row: 953 us at 262,144
+    // pairs of 256, B = 49, 769 us this way.
+    constexpr int CG = 8;
     // Rows are taken RB at a time: first the path through the RB rows (bits
     // only, already in registers) while every x and prefix load those rows need
     // is issued, then the sums; the next RB rows' bits are fetched in between.
-    // RB is as many rows as keep the kernel within 128 registers (four waves
-    // per SIMD): more rows per batch are fewer memory round trips per pair.
-    constexpr int RB = BP <= 32 ? 7 : BP <= 64 ? 6 : BP <= 96 ? 5 : 4;
+    // More rows per batch are fewer memory round trips per pair: 8 rows in 168
+    // registers (three waves per SIMD) 769 us, 4 rows in 125 (four) 838 us.
+    constexpr int RB = BP <= 64 ? 8 : 4;
+    // columns with notes at a time: the band, a batch of rows, a partial group
+    constexpr int W = BP + RB + CG - 2;
+    __shared__ uint16_t note[W][64];  // column mod W: 1, exit slot, entry slot (1 + 7 + 7 bits)
+#pragma unroll
+    for (int e = 0; e < W; ++e) note[e][lane] = 0;
+    typedef float fcg __attribute__((ext_vector_type(CG)));
+    fcg *__restrict__ gww = (fcg *)(go.gw + p * go.lyp);
+    const fcg *__restrict__ ypw = (const fcg *)(go.YP + b * go.lyp);
+    const double *__restrict__ PX = go.PX + a * go.pxa;
+    const int64_t pxi = go.pxi;
+    int jg = (ly - 1) / CG * CG;  // the next group of columns
+    int sg = jg % W;
+    int is = lx - 1, js = 0;  // topmost row of the last column done, its first column
+    auto finish_group = [&]() {
+        double hi[CG], lo[CG];
+        float cnt[CG];
+        const fcg yv_ = ypw[jg / CG];
+#pragma unroll
+        for (int e = CG - 1; e >= 0; --e) {
+            const int j = jg + e;
+            const int sl = sg + e < W ? sg + e : sg + e - W;
+            const uint32_t v = note[sl][lane];
+            note[sl][lane] = 0;
+            const int last = js > j ? is - 1 : is;  // entered by a diagonal step
+            if (v) {
+                is = j + off - (int)(v >> 7 & 127u);
+                js = is + (int)(v & 127u) - off;
+            }
+            cnt[e] = (float)(last - is + 1);
+            hi[e] = PX[(last + 1) * pxi];
+            lo[e] = PX[is * pxi];
+        }
+        fcg o;
+#pragma unroll
+        for (int e = 0; e < CG; ++e) {
+            const float c = jg + e < ly ? coef : 0.0f;  // zeros past the series
+            o[e] = __builtin_fmaf(c * cnt[e], yv_[e], -(c * (float)(hi[e] - lo[e])));
+        }
+        if (active) gww[jg / CG] = o;
+        jg -= CG;
+        sg = sg >= CG ? sg - CG : sg - CG + W;
+    };
+
     uint32_t wd[RB][NW], wu[RB][NW];
     auto load_bits = [&](int ih) {
 #pragma unroll
@@ -191,9 +237,8 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
     };
     load_bits(lx - 1);
     int k = g.kf;
-    int cj = ly - 1;   // column being accumulated
-    float cnt = 0.0f;  // its number of path cells
-    float sxc = 0.0f;  // and the sum of their x
+    int sb = (lx - 1 - off) % W;  // slot 0 of the row, as a note's place
+    if (sb < 0) sb += W;
     for (int ih = lx - 1; ih >= 0; ih -= RB) {
         int jer[RB], jxr[RB];
         float xr[RB];
@@ -230,6 +275,9 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
             }
             if (k < kx) k = kx;  // likewise unreachable; keeps je >= jx
             const int je = i + k - off, jx = i + kx - off;  // in [0, ly)
+            const int sl = sb + k;
+            note[sl < W ? sl : sl - W][lane] = (uint16_t)(1u << 14 | k << 7 | kx);
+            sb = sb == 0 ? W - 1 : sb - 1;
             jer[r] = je;
             jxr[r] = jx;
             xr[r] = XT[(int64_t)i * nxs];
@@ -244,22 +292,6 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
             if (i < 0) break;  // uniform
             const float xi = xr[r];
             const int je = jer[r], jx = jxr[r];
-            // The open column cj takes this row's cell when the row enters
-            // there (an up step; a diagonal step enters at cj - 1).  Columns
-            // cj down to jx + 1 are then finished: cj with its sums, the rest
-            // with this row's single cell; jx becomes the open column.
-            if (je == cj) {
-                cnt += 1.0f;
-                sxc += xi;
-            }
-            const int nfin = cj - jx;
-            for (int t = 0; t < nfin; ++t)
-                finish(cj - t, t == 0 ? coef * cnt : coef, t == 0 ? coef * sxc : coef * xi);
-            if (nfin > 0) {
-                cj = jx;
-                cnt = 1.0f;
-                sxc = xi;
-            }
             // dD/dx_i: coef * sum over the row's cells of (x_i - y_j)
             const float gx = (float)(coefd * ((double)(je - jx + 1) * (double)xi - (ph[r] - pl[r])));
             if (go.mode == 1) {
@@ -277,8 +309,9 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
                 go.gxp[(wave * lx + i) * 64 + lane] = gx;
             }
         }
+        // rows up to ih - RB reach columns below ih - RB + B - off
+        while (jg >= 0 && (ih < RB || jg >= ih - RB + B - off)) finish_group();
     }
-    finish(cj, coef * cnt, coef * sxc);  // column 0 completes the last window
 }
 
 __device__ __forceinline__ int64_t pair_slot(int64_t p, int len, int idx) {
@@ -448,7 +481,7 @@ static int train_geo(const wbx_metric *m, int64_t tx, int64_t ty, TrainGeo *out)
 // the column partials.
 struct TrainScratch {
     bool xred;
-    int64_t nbc, xt, pt, gw, yp, gx, xpart, part, total;  // byte offsets / sizes
+    int64_t nbc, xt, pt, px, gw, yp, gx, xpart, part, total;  // byte offsets / sizes
 };
 
 static TrainScratch train_scratch(int mode, int64_t nx, int64_t ny, int64_t tx, int64_t ty) {
@@ -460,6 +493,8 @@ static TrainScratch train_scratch(int mode, int64_t nx, int64_t ny, int64_t tx, 
     o += al(nx * tx * 4);
     t.pt = o;
     o += al((ty + 1) * ny * 8);
+    t.px = o;
+    o += al((tx + 1) * nx * 8);
     const int64_t lyp = (ty + 7) / 8 * 8;
     t.gw = o;
     o += al(np * lyp * 4);
@@ -604,8 +639,15 @@ int wbx_dev_dtw_train_backward(const wbx_metric *metric, int mode, const float *
     double *pt = (double *)(sc + ts.pt);
     hipLaunchKernelGGL(k_transpose, dim3((unsigned)((tx + 31) / 32), (unsigned)((nx + 31) / 32)),
                        dim3(256), 0, st, X, nx, (int)tx, x_stride, xt);
-    hipLaunchKernelGGL(k_prefix_t, dim3((unsigned)ny), dim3(64), 0, st, Y, ny, (int)ty, y_stride,
-                       pt, yp, go.lyp);
+    hipLaunchKernelGGL(k_prefix<false>, dim3((unsigned)((ny + 15) / 16)), dim3(1024), 0, st, Y, ny,
+                       (int)ty, y_stride, pt, yp, go.lyp);
+    double *px = (double *)(sc + ts.px);
+    go.pxi = ts.xred ? 1 : nx;
+    go.pxa = ts.xred ? tx + 1 : 1;
+    go.PX = px;
+    hipLaunchKernelGGL(ts.xred ? k_prefix<true> : k_prefix<false>,
+                       dim3((unsigned)((nx + 15) / 16)), dim3(1024), 0, st, X, nx, (int)tx,
+                       x_stride, px, (float *)nullptr, 0);
     go.XT = xt;
     go.PT = pt;
     switch (tg.BP) {

@@ -12,13 +12,13 @@
 //                    SGPRs, and the path is walked there: the exit of a row
 //                    is a count of leading zeros.  The rows' column ranges go
 //                    to LDS and the 64 lanes form the gradient terms of rows,
-//                    then columns, with the arithmetic and order of
-//                    k_lane_backtrack.
+//                    then columns (prefix sums of y, then of x, in
+//                    LDS), with the arithmetic of k_lane_backtrack.
 //  k_sum_pairs       dX from the per-pair rows.
 //
 // Bound by latency: the chain of cells of a row in the forward, the chain of
 // rows in the walk.  1 x 512 pairs of 256, r = 0.1, against one pair per lane
-// (8 waves): forward 221 -> 36 us, backward 334 -> 65 us.
+// (8 waves): forward 221 -> 36 us, backward 334 -> 59 us.
 #include <type_traits>
 
 #include "lane_train.h"
@@ -222,7 +222,9 @@ struct SmallGrad {
 
 // LDS: x (lx), prefix sums of y (ly + 1, float64), the rows' column ranges
 // (lx), the columns' row ranges (ly).
-size_t small_lds(int lx, int ly) { return (size_t)(ly + 1) * 8 + (size_t)(2 * lx + ly) * 4; }
+size_t small_lds(int lx, int ly) {
+    return (size_t)((lx > ly ? lx : ly) + 1) * 8 + (size_t)(lx + ly) * 4;
+}
 
 // WIDE: bands of 65 .. 112 slots (two masks per row).
 template <bool WIDE>
@@ -233,9 +235,8 @@ __global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float
                                                        const unsigned char *__restrict__ dec,
                                                        SmallGrad out) {
     extern __shared__ __align__(16) unsigned char smem[];
-    double *pt = (double *)smem;                   // pt[j] = y[0] + ... + y[j - 1]
-    float *lxv = (float *)(pt + g.ly + 1);
-    uint32_t *rows = (uint32_t *)(lxv + g.lx);     // je << 16 | jx
+    double *pt = (double *)smem;  // pt[j] = y[0] + ... + y[j - 1], later of x
+    uint32_t *rows = (uint32_t *)(pt + (g.lx > g.ly ? g.lx : g.ly) + 1);  // je << 16 | jx
     uint32_t *cols = rows + g.lx;                  // last row << 16 | first row
     const int lane = threadIdx.x;
     const int64_t p = blockIdx.x;
@@ -266,21 +267,23 @@ __global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float
         }
     };
     load(cur, lx - 1);
-    for (int i = lane; i < lx; i += 64) lxv[i] = X[i];
-    if (lane == 0) pt[0] = 0.0;
-    double carry = 0.0;
-    for (int j0 = 0; j0 < ly; j0 += 64) {  // the scan of k_prefix_t
-        const int j = j0 + lane;
-        double s = j < ly ? (double)Y[j] : 0.0;
+    auto prefix = [&](const float *__restrict__ v, int len) {  // the scan of k_prefix
+        if (lane == 0) pt[0] = 0.0;
+        double carry = 0.0;
+        for (int j0 = 0; j0 < len; j0 += 64) {
+            const int j = j0 + lane;
+            double s = j < len ? (double)v[j] : 0.0;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const double o = __shfl_up(s, d);
-            if (lane >= d) s += o;
+            for (int d = 1; d < 64; d <<= 1) {
+                const double o = __shfl_up(s, d);
+                if (lane >= d) s += o;
+            }
+            s += carry;
+            if (j < len) pt[j + 1] = s;
+            carry = __shfl(s, 63);
         }
-        s += carry;
-        if (j < ly) pt[j + 1] = s;
-        carry = __shfl(s, 63);
-    }
+    };
+    prefix(Y, ly);
 
     int k = g.kf;  // the walk is uniform over the wave
     for (int ih = lx - 1; ih >= 0; ih -= RB) {
@@ -346,7 +349,7 @@ __global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float
     for (int i = lane; i < lx; i += 64) {
         const uint32_t v = rows[i];
         const int jx = v & 0xffff, je = v >> 16;
-        const float xi = lxv[i];
+        const float xi = X[i];
         gx[i] = (float)(coefd * ((double)(je - jx + 1) * (double)xi - (pt[je + 1] - pt[jx])));
         // Consecutive rows share at most one column (an up step), so a column
         // has its first row here unless it is the one shared with the row
@@ -359,13 +362,13 @@ __global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float
         }
     }
     __syncthreads();
+    prefix(X, lx);
+    __syncthreads();
     for (int j = lane; j < ly; j += 64) {
         const uint32_t v = cols[j];
         const int i0 = v & 0xffff, i1 = v >> 16;
-        float sx = lxv[i1];
-        for (int i = i1 - 1; i >= i0; --i) sx += lxv[i];
         const float cnt = (float)(i1 - i0 + 1);
-        gy[j] = coef * cnt * Y[j] - coef * sx;
+        gy[j] = __builtin_fmaf(coef * cnt, Y[j], -(coef * (float)(pt[i1 + 1] - pt[i0])));
     }
 }
 
