@@ -56,3 +56,32 @@ def test_exact_forms(slots, nx, ny, data):
     big = torch.maximum(Xp.abs().amax(1), Yp.abs().amax(1)).double()
     bound = 2 * t * u * (Gp * Dp + 2 * t * Gp / Dp.clamp(min=1e-30) * 4 * big**2)
     assert ((hom - Gp * Dp).abs() <= bound)[pos].all()
+
+
+@pytest.mark.parametrize("nx,ny,t,r", [
+    (3073, 64, 20, 0.1),   # 385 blocks of 8 series, the last with one; band 5 (padded to 8)
+    (1540, 128, 45, 0.45), # two waves per x series, band 41
+    (2048, 64, 66, 0.7),   # a wide band (93 slots) at its own smallest count
+    (3080, 64, (30, 41), 0.2),
+])
+def test_shared_prefix_blocks(nx, ny, t, r):
+    """Full-chip grids (eight x series share a block's window of y prefix sums)
+    against the same rows in calls too small for it: the same terms."""
+    tx, ty = t if isinstance(t, tuple) else (t, t)
+    rng = np.random.default_rng(tx)
+    X = torch.from_numpy(rng.standard_normal((nx, tx)).cumsum(axis=1).astype(np.float32)).cuda()
+    Y = torch.from_numpy(rng.standard_normal((ny, ty)).cumsum(axis=1).astype(np.float32)).cuda()
+    G = torch.from_numpy(rng.uniform(0.5, 2.0, (nx, ny))).cuda()
+    D, gx, gy = _grads(dtw, X, Y, G, r)
+    sy = torch.zeros_like(gy, dtype=torch.float64)
+    for i in np.array_split(np.arange(nx), nx * ny // 17000):  # past the few-pairs form
+        i = slice(i[0], i[-1] + 1)
+        d, px, py = _grads(dtw, X[i], Y, G[i], r)
+        assert torch.equal(D[i], d)
+        assert torch.equal(gx[i], px)  # one order of sums over the row's pairs
+        sy += py.double()
+    # two float32 sums of nx terms in different orders
+    _, _, py = _grads(paired_dtw, X.repeat_interleave(ny, 0), Y.repeat(nx, 1), G.reshape(-1), r)
+    mag = py.double().abs().reshape(nx, ny, ty).sum(0)
+    u = 2.0**-24
+    assert ((gy.double() - sy).abs() <= 2 * nx * u * mag + 1e-30).all()

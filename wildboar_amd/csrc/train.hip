@@ -140,18 +140,25 @@ __global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ src
 // Bit of slot k in its plane word: slots are shifted in from the low end, so
 // slot k of word w sits at bit (count_w - 1 - (k - 32 w)); the last word holds
 // the lastc slots that the forward computed past the others.
-template <int BP>
-__global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
+template <int BP, int NV>
+__global__ __launch_bounds__(64 * NV) __attribute__((
+    amdgpu_waves_per_eu(BP > 64 ? 2 : NV == 1 ? 3 : 4))) void k_lane_backtrack(PairSpec ps, LaneGeo g,
                                                        const float *__restrict__ sq,
                                                        const double *__restrict__ G,
                                                        const uint32_t *__restrict__ dirs,
                                                        int lastc, GradOut go) {
     constexpr int NW = (BP + 31) / 32;
-    const int lane = threadIdx.x;
-    const int64_t wave = blockIdx.x;
+    const int lane = threadIdx.x & 63, wv = NV == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int64_t wave = blockIdx.x;
+    bool mine = true;  // this wave is not a block's filling
+    if constexpr (NV > 1) {
+        const int64_t r = blockIdx.x / go.nbc * NV + wv;
+        mine = r < go.nx;
+        wave = (mine ? r : go.nx - 1) * go.nbc + blockIdx.x % go.nbc;
+    }
     const int64_t p0 = wave * 64 + lane;
-    const bool active = p0 < ps.n_pairs;
-    const int64_t p = active ? p0 : ps.n_pairs - 1;
+    const bool active = mine && p0 < ps.n_pairs;
+    const int64_t p = p0 < ps.n_pairs ? p0 : ps.n_pairs - 1;
     int64_t a, b;
     decode_pair(ps, p, a, b);
     const float *__restrict__ XT = go.XT + a;   // x_i = XT[i * nx]
@@ -162,27 +169,42 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
     const double coefd = (active && D > 0.0) ? G[p] / D : 0.0;
     const float coef = (float)coefd;
     // A column's terms need its first and last path row.  The walk of a row
-    // notes, at the column where the row ends, its exit and entry slots (one
-    // LDS write; of several rows ending in a column the topmost stays), and
-    // columns that no later row can reach are finished by all lanes together,
-    // CG at a time from the right: rows of a column are contiguous and one
-    // row's columns too, so the last note seen gives both rows, and the sum of
-    // x over them is a difference of prefix sums.  Finishing each row's
-    // columns as the row leaves them runs every wave as long as the longest
-    // horizontal run among its 64 paths, row after row: 953 us at 262,144
-    // pairs of 256, B = 49, 769 us this way.
+    // notes its slot at the column where the row ends (one LDS write; of
+    // several rows ending in a column the topmost stays) and how the column
+    // was entered, and columns that no later row can reach are finished by all
+    // lanes together, CG at a time from the right: rows of a column are
+    // contiguous and one row's columns too, so the last note seen gives both
+    // rows, and the sum of x over them is a difference of prefix sums.
+    // Finishing each row's columns as the row leaves them runs every wave as
+    // long as the longest horizontal run among its 64 paths, row after row:
+    // 953 us at 262,144 pairs of 256, B = 49; 769 us this way.
+    // NV > 1: the block's waves have the same lanes of y series and walk the
+    // same rows, so the prefix sums of y come from a window in LDS, advanced by
+    // RB columns a batch (see share_prefix): 519 us.
     constexpr int CG = 8;
     // Rows are taken RB at a time: first the path through the RB rows (bits
     // only, already in registers) while every x and prefix load those rows need
     // is issued, then the sums; the next RB rows' bits are fetched in between.
-    // More rows per batch are fewer memory round trips per pair: 8 rows in 168
-    // registers (three waves per SIMD) 769 us, 4 rows in 125 (four) 838 us.
-    constexpr int RB = BP <= 64 ? 8 : 4;
+    // More rows per batch are fewer memory round trips per pair: with NV = 1,
+    // 8 rows in 165 registers (three waves per SIMD) 769 us, 4 rows in 125
+    // (four) 838 us; with the sums in LDS 4 rows keep four waves.
+    constexpr int RB = NV == 1 && BP <= 64 ? 8 : 4;
     // columns with notes at a time: the band, a batch of rows, a partial group
     constexpr int W = BP + RB + CG - 2;
-    __shared__ uint16_t note[W][64];  // column mod W: 1, exit slot, entry slot (1 + 7 + 7 bits)
+    // column mod W: the row's slot there + 1, bit 7: the column is entered by a
+    // diagonal step; 0: no row ends there
+    __shared__ uint8_t notes[NV][W][64];
+    uint8_t(*note)[64] = notes[wv];
 #pragma unroll
     for (int e = 0; e < W; ++e) note[e][lane] = 0;
+    // the prefix sums of y that the rows of a batch and of the next one need
+    constexpr int RW = NV > 1 ? BP + 2 * RB : 1;
+    __shared__ double ring[RW][64];  // column mod RW
+    if constexpr (NV > 1) {
+        for (int j = lx - RB - off + wv; j <= lx - 1 + B - off; j += NV)
+            if (j >= 0 && j <= ly) ring[j % RW][lane] = PT[j * nys];
+        __syncthreads();
+    }
     typedef float fcg __attribute__((ext_vector_type(CG)));
     fcg *__restrict__ gww = (fcg *)(go.gw + p * go.lyp);
     const fcg *__restrict__ ypw = (const fcg *)(go.YP + b * go.lyp);
@@ -190,7 +212,7 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
     const int64_t pxi = go.pxi;
     int jg = (ly - 1) / CG * CG;  // the next group of columns
     int sg = jg % W;
-    int is = lx - 1, js = 0;  // topmost row of the last column done, its first column
+    int is = lx - 1;  // topmost row of the last column done
     auto finish_group = [&]() {
         double hi[CG], lo[CG];
         float cnt[CG];
@@ -201,11 +223,8 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
             const int sl = sg + e < W ? sg + e : sg + e - W;
             const uint32_t v = note[sl][lane];
             note[sl][lane] = 0;
-            const int last = js > j ? is - 1 : is;  // entered by a diagonal step
-            if (v) {
-                is = j + off - (int)(v >> 7 & 127u);
-                js = is + (int)(v & 127u) - off;
-            }
+            const int last = is - (int)(v >> 7);
+            if (v) is = j + off + 1 - (int)(v & 127u);
             cnt[e] = (float)(last - is + 1);
             hi[e] = PX[(last + 1) * pxi];
             lo[e] = PX[is * pxi];
@@ -239,8 +258,14 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
     int k = g.kf;
     int sb = (lx - 1 - off) % W;  // slot 0 of the row, as a note's place
     if (sb < 0) sb += W;
+    int rb = (lx - 1 - off) % RW;  // and as a place in the ring
+    if (rb < 0) rb += RW;
+    uint32_t ent = 0;  // the column the row ends in: 128 if entered by a diagonal step
     for (int ih = lx - 1; ih >= 0; ih -= RB) {
-        int jer[RB], jxr[RB];
+        const int jn = ih - 2 * RB + 1 - off + wv;  // this wave's new column of the next batch
+        double pn = 0.0;
+        if (NV > 1 && wv < RB && jn >= 0) pn = PT[jn * nys];
+        int nr[RB];  // cells of the row
         float xr[RB];
         double ph[RB], pl[RB];
 #pragma unroll
@@ -276,13 +301,20 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
             if (k < kx) k = kx;  // likewise unreachable; keeps je >= jx
             const int je = i + k - off, jx = i + kx - off;  // in [0, ly)
             const int sl = sb + k;
-            note[sl < W ? sl : sl - W][lane] = (uint16_t)(1u << 14 | k << 7 | kx);
+            note[sl < W ? sl : sl - W][lane] = (uint8_t)(ent | (uint32_t)(k + 1));
             sb = sb == 0 ? W - 1 : sb - 1;
-            jer[r] = je;
-            jxr[r] = jx;
+            ent = isd ? 128u : kx == k ? ent : 0u;
+            nr[r] = k - kx + 1;
             xr[r] = XT[(int64_t)i * nxs];
-            ph[r] = PT[(int64_t)(je + 1) * nys];
-            pl[r] = PT[(int64_t)jx * nys];
+            if constexpr (NV > 1) {
+                const int sh = rb + k + 1, sx = rb + kx;
+                ph[r] = ring[sh < RW ? sh : sh - RW][lane];
+                pl[r] = ring[sx < RW ? sx : sx - RW][lane];
+                rb = rb == 0 ? RW - 1 : rb - 1;
+            } else {
+                ph[r] = PT[(int64_t)(je + 1) * nys];
+                pl[r] = PT[(int64_t)jx * nys];
+            }
             k = isd ? kx : kx + 1;
         }
         if (ih - RB >= 0) load_bits(ih - RB);
@@ -291,14 +323,13 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
             const int i = ih - r;
             if (i < 0) break;  // uniform
             const float xi = xr[r];
-            const int je = jer[r], jx = jxr[r];
             // dD/dx_i: coef * sum over the row's cells of (x_i - y_j)
-            const float gx = (float)(coefd * ((double)(je - jx + 1) * (double)xi - (ph[r] - pl[r])));
+            const float gx = (float)(coefd * ((double)nr[r] * (double)xi - (ph[r] - pl[r])));
             if (go.mode == 1) {
                 if (active) go.dX[p * go.ldx + i] = gx;
             } else if (go.xred) {
                 const float tot = wave_sum(gx);
-                if (lane == 0) {
+                if (lane == 0 && mine) {
                     const int64_t bc = (wave * 64 - a * go.ny) / 64;
                     if (go.nbc == 1)
                         go.dX[a * go.ldx + i] = tot;
@@ -308,6 +339,10 @@ __global__ __launch_bounds__(64) void k_lane_backtrack(PairSpec ps, LaneGeo g,
             } else {
                 go.gxp[(wave * lx + i) * 64 + lane] = gx;
             }
+        }
+        if constexpr (NV > 1) {
+            if (wv < RB && jn >= 0) ring[jn % RW][lane] = pn;
+            __syncthreads();
         }
         // rows up to ih - RB reach columns below ih - RB + B - off
         while (jg >= 0 && (ih < RB || jg >= ih - RB + B - off)) finish_group();
@@ -405,6 +440,15 @@ void launch_sum_cols(const float *gw, int64_t nx, int64_t ny, int ly, int lyp, f
                        ldy_);
 }
 
+// Whether 8 waves (8 x series, the same 64 y series) share a block's window of
+// y prefix sums.  The gathers it replaces touch about 45 lines each, so that a
+// full chip waits for the vector caches (262,144 pairs of 256, B = 49: 769 ->
+// 519 us); at few waves there is no queue and the blocks' barriers cost more.
+// Alone, waves run 3 to a SIMD (2 past 64 slots); the line is where they need
+// a second pass.  One step, alone and shared: 256 blocks, B = 49 678 and 733
+// us, B = 103 1026 and 918; 512 blocks, B = 49 1280 and 1029.
+static bool share_prefix(int BP, int64_t blocks) { return blocks >= (BP > 64 ? 256 : 385); }
+
 static int train_bp(int B) { return (B + 7) / 8 * 8; }
 
 template <int BP, int U>
@@ -418,8 +462,13 @@ template <int BP>
 static void train_bwd_one(const PairSpec &ps, LaneGeo g, const float *sq, const double *G,
                           const uint32_t *dirs, GradOut go, hipStream_t st) {
     const int slots = lane_exact_supported(g.B) ? g.B : BP;  // as the forward computed
-    hipLaunchKernelGGL((k_lane_backtrack<BP>), dim3((unsigned)((ps.n_pairs + 63) / 64)), dim3(64), 0,
-                       st, ps, g, sq, G, dirs, slots - 32 * ((BP + 31) / 32 - 1), go);
+    const int lastc = slots - 32 * ((BP + 31) / 32 - 1);
+    if (go.xred && share_prefix(BP, (go.nx + 7) / 8 * go.nbc))
+        hipLaunchKernelGGL((k_lane_backtrack<BP, 8>), dim3((unsigned)((go.nx + 7) / 8 * go.nbc)),
+                           dim3(512), 0, st, ps, g, sq, G, dirs, lastc, go);
+    else
+        hipLaunchKernelGGL((k_lane_backtrack<BP, 1>), dim3((unsigned)((ps.n_pairs + 63) / 64)),
+                           dim3(64), 0, st, ps, g, sq, G, dirs, lastc, go);
 }
 
 #define TRAIN_CASES(X)                                                                          \
