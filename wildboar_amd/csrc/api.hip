@@ -1,10 +1,12 @@
 // api.hip -- the extern "C" entry points declared in include/wbx.h.
 //
 // Dispatch per request:
-//   FP64 (parity)  euclidean -> exact tiled sum; dtw/wdtw -> plain kernel.
-//   FP32           euclidean -> FP32 tiled sum; dtw -> lane-per-pair register
-//                  kernel when the band fits (B <= 112), plain FP32 kernel
-//                  otherwise; wdtw -> plain FP32 kernel.
+//   euclidean      tiled sums (float64: the reference's order).
+//   dtw/wdtw/adtw  run_pairs: a pair per lane where the band fits a lane's
+//                  registers and the call fills the chip, several lanes per
+//                  pair for wider bands and small calls, columns per lane for
+//                  full matrices, each by its modelled time; the plain kernel
+//                  for the rest.
 //   argmin FP32    FP32 distances -> certified candidate set -> exact FP64
 //                  re-evaluation of the candidates -> heap replay, so indices
 //                  and distances equal the reference's.

@@ -23,9 +23,11 @@
 // below the best.  Each is a sum of non-negative terms, so its partial value
 // reaches the best iff its full value does; hence the window is accepted iff
 //     T(I) = max(K, LK, LK2, max_i(rowmin_i + cb[i + r + 1]), D) < best,
-// with every term computed in full.  The kernels compute T and D for every
-// window in parallel and replay the acceptance rule over the windows in
-// increasing order: the reference's result bit for bit, including windows
+// with every term computed in full.  Matching computes T and D for every
+// window in parallel and replays the acceptance rule over the windows in
+// increasing order; the subsequence search walks each task's windows in blocks
+// of 64 and computes what its best so far leaves open (search_task).  Both
+// give the reference's result bit for bit, including windows
 // its LB_Kim prunes although their DTW is the smallest (its last-but-one
 // term omits the (T[L-2], S[L-1]) cell, and below length 6 the first and
 // last three points overlap).  Below length 3 the reference's LB_Kim reads
