@@ -50,3 +50,30 @@ def test_shared_x_waves_match_group_kernel(nx, ny, tx, ty, r, metric):
     # (1 + u)^(lx + ly) and the rounding of the inputs
     tol = (tx + ty + 8) * 2.0**-24 * (1 + np.abs(X).max() ** 2)
     np.testing.assert_allclose(got[:nx], ref, rtol=1e-5, atol=tol)
+
+
+@pytest.mark.parametrize("metric", ["ddtw", "wddtw"])
+@pytest.mark.parametrize("t,r", [(7, 1.0), (8, 0.9), (15, 1.0), (22, 0.97), (23, 1.0), (30, 0.99),
+                                 (50, 1.0), (57, 0.97), (57, 0.99)])
+def test_slopes_under_a_wider_band(t, r, metric):
+    """Slopes are two values shorter than their series and keep its band, which
+    may be wider than they are long: slots without a weight."""
+    rng = np.random.default_rng(t)
+    X = rng.standard_normal((3, t)).cumsum(axis=1)
+    Y = rng.standard_normal((130, t)).cumsum(axis=1)
+    params = {"r": r} if metric == "ddtw" else {"r": r, "g": 0.1}
+    big = np.tile(X, (400, 1))  # fills the chip: lanes
+    call = lambda x: wd.pairwise_distance(x, Y, metric=metric, metric_params=params,
+                                          precision="fp32")
+    got = call(big)
+    _lib.set_policy(2)
+    try:
+        want = call(big)
+    finally:
+        _lib.set_policy(0)
+    np.testing.assert_array_equal(got, want)
+    np.testing.assert_array_equal(got[:3], call(X))  # few pairs: several lanes each
+    ref = oracle.pairwise(X, Y, metric=metric, r=r, g=0.1)
+    # slopes are rounded to float32 (|slope| <= 2 |x|), then (1 + u)^(lx + ly)
+    tol = (2 * t + 8) * 2.0**-24 * (1 + 4 * np.abs(X).max() ** 2)
+    np.testing.assert_allclose(got[:3], ref, rtol=1e-5, atol=tol)

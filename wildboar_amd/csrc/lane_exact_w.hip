@@ -5,8 +5,12 @@
 
 namespace wbx {
 
+// The kernel reads (B + 1) / 2 weights of the max(lx, ly) there are.  The slopes
+// of a derivative metric keep the band of the longer series they come from,
+// which can be wider than the slopes are long: those calls take the kernels
+// that clamp the index.
 int64_t lane_exact_w_waves(const PairSpec &ps, int lx, int ly, int B) {
-    if (ps.mode != PAIR_GRID || lx != ly || !lane_exact_supported(B)) return 0;
+    if (ps.mode != PAIR_GRID || lx != ly || (B + 1) / 2 > lx || !lane_exact_supported(B)) return 0;
     const int64_t waves = ps.n_pairs / ps.ny * ((ps.ny + 63) / 64);
     return waves <= INT32_MAX ? waves : 0;
 }

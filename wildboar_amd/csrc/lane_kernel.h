@@ -86,13 +86,17 @@ __device__ __forceinline__ void lane_dtw_body(PairSpec ps, Series<float> xs,
                                                  float *__restrict__ sq) {
     constexpr int W = BP + U - 1;
     // WT: lw[0][k] row-0 weight of slot k, lw[1][k] = w[|k - off|]; slots
-    // outside the band get 1 (their cells are +inf or thrown away)
+    // outside the band get 1 (their cells are +inf or thrown away).  A band
+    // wider than the series (slopes, with the band of the series they come
+    // from) has slots past the last weight; they lie outside the matrix and
+    // take the last one.
     __shared__ float lw[WT ? 2 : 1][WT ? BP : 1];
     if constexpr (WT) {
+        const int top = max(g.lx, g.ly) - 1;
         for (int k = threadIdx.x; k < BP; k += 64) {
             const int j = k - g.off;  // column of slot k in row 0
-            lw[0][k] = (j >= 0 && k < g.B) ? weights[j > 0 ? j - 1 : 0] : 1.0f;
-            lw[1][k] = k < g.B ? weights[j < 0 ? -j : j] : 1.0f;
+            lw[0][k] = (j >= 0 && k < g.B) ? weights[min(j > 0 ? j - 1 : 0, top)] : 1.0f;
+            lw[1][k] = k < g.B ? weights[min(j < 0 ? -j : j, top)] : 1.0f;
         }
         __syncthreads();
     }
@@ -300,7 +304,8 @@ typedef const float __attribute__((address_space(4))) *cfloat;
 // B = 101), longer groups gain nothing.  2000 x 2000 x 512 on one box, x per
 // lane -> XU: B = 23 2.92 -> 2.67 ms, B = 49 5.52 -> 5.23, B = 75 8.83 -> 8.10,
 // B = 101 12.02 -> 10.73, B = 111 13.05 -> 11.70.
-// WT: WDTW (equal lengths, XU; weights: at least (B + 1) / 2 values).  1000 x
+// WT: WDTW (equal lengths, XU; weights: at least (B + 1) / 2 values, which
+// lane_exact_w_waves sees to).  1000 x
 // 1000 x 256, B = 49: 1205 us on the group kernel, 873 us.
 template <int B, int U, bool XU, bool WT = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_lane_dtw_exact(
