@@ -1,0 +1,42 @@
+"""The device code in the built library, read from its code objects: no GPU
+needed."""
+
+import os
+import struct
+
+import msgpack
+import numpy as np
+import pytest
+
+from wildboar_amd import _lib
+
+
+@pytest.fixture(scope="module")
+def code_objects():
+    data = open(_lib.load()._name, "rb").read()
+    magic, out, at = b"__CLANG_OFFLOAD_BUNDLE__", [], 0
+    while (at := data.find(magic, at)) >= 0:
+        (count,) = struct.unpack_from("<Q", data, at + 24)
+        entry = at + 32
+        for _ in range(count):
+            off, size, n = struct.unpack_from("<QQQ", data, entry)
+            target = data[entry + 24:entry + 24 + n].decode()
+            entry += 24 + n
+            if "gfx950" in target and size:
+                out.append(data[at + off:at + off + size])
+        at += 24
+    here = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    sources = [f for f in os.listdir(os.path.join(here, "wildboar_amd", "csrc"))
+               if f.endswith(".hip")]
+    assert 0 < len(out) <= len(sources)
+    return out
+
+
+def test_no_scalar_pair_takes_a_literal_for_a_double(code_objects):
+    """The compiler sometimes writes a uniform double +inf to a scalar pair as
+    s_mov_b64 with a 64-bit literal, which the instruction cannot hold: it is
+    encoded with the literal's low half, 0.  (An intended 0 is an inline
+    constant.)  rerank.hip starts its threshold in a vector register for that."""
+    for elf in code_objects:
+        w = np.frombuffer(elf[:len(elf) // 4 * 4], dtype="<u4")
+        assert not (((w[:-1] & 0xFF80FFFF) == 0xBE8001FF) & (w[1:] == 0)).any()
