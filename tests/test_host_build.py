@@ -40,3 +40,30 @@ def test_no_scalar_pair_takes_a_literal_for_a_double(code_objects):
     for elf in code_objects:
         w = np.frombuffer(elf[:len(elf) // 4 * 4], dtype="<u4")
         assert not (((w[:-1] & 0xFF80FFFF) == 0xBE8001FF) & (w[1:] == 0)).any()
+
+
+@pytest.fixture(scope="module")
+def registers(code_objects):
+    """Vector registers of every kernel, by its mangled name."""
+    out = {}
+    for elf in code_objects:
+        at = elf.find(b"AMDGPU\0")
+        size, kind = struct.unpack_from("<II", elf, at - 8)
+        assert kind == 32  # the metadata note: name (8 bytes), then msgpack
+        for k in msgpack.unpackb(elf[at + 8:at + 8 + size])["amdhsa.kernels"]:
+            out[k[".name"]] = k[".vgpr_count"]
+    return out
+
+
+@pytest.mark.parametrize("kernel,most", [
+    ("k_lane64_pairsILi8ELi4ELb0ELb0E", 80),   # six waves per SIMD
+    ("k_lane64_pairsILi8ELi4ELb1ELb0E", 80),
+    ("k_lane64_pairsILi40ELi4ELb1ELb0E", 256),  # two
+    ("k_lane_dtwILi40ELi8ELb1ELb0E", 168),     # three
+    ("k_lane_dtwILi40ELi8ELb0ELb1E", 160),
+])
+def test_writing_distances_in_place_keeps_the_waves(registers, kernel, most):
+    """The pair kernels' registers leave the waves per SIMD that they have
+    without the place of the result kept through the loop."""
+    (got,) = [v for name, v in registers.items() if kernel in name]
+    assert got <= most

@@ -175,7 +175,7 @@ k_full_dtw(PairSpec ps, Series<T> xs, Series<T> ys, FullGeo g, T *__restrict__ s
 #pragma unroll
         for (int m = 0; m < S; ++m)
             if (c0 + m == jf) res = L.row[m];
-        put_cost(ps, p, a, b, res, sq);
+        put_cost(ps, p, res, sq);
     }
 }
 

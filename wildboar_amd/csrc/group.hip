@@ -339,7 +339,7 @@ __global__ __launch_bounds__(64) void k_group_dtw(PairSpec ps, Series<T> xs, Ser
 #pragma unroll
         for (int m = 0; m < S; ++m)
             if (k0 + m == g.kf) res = L.row[m];
-        put_cost(ps, p, a, b, res, sq);
+        put_cost(ps, p, res, sq);
     }
 }
 

@@ -46,7 +46,7 @@ __global__ __launch_bounds__(64) void k_lane64_pairs(PairSpec ps, Series<double>
     decode_pair(ps, p, a, b);
     const double c = lane64_cost<BP, U, WT, AD, lane64_prefetch<0, BP, WT, AD>()>(
         xs.row(a), xs.len, ys.row(b), ys.len, off, B, kf, weights, wn, pen);
-    if (p0 < ps.n_pairs) put_cost(ps, p0, a, b, c, sq);
+    if (p0 < ps.n_pairs) put_cost(ps, p0, c, sq);
 }
 
 // Band slots of a pattern of length L (both sides L): B = 2 w - 1.

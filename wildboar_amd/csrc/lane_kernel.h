@@ -221,7 +221,7 @@ __device__ __forceinline__ void lane_dtw_body(PairSpec ps, Series<float> xs,
 #pragma unroll
     for (int k = 0; k < BP; ++k)
         if (k == g.kf) res = row[k];
-    if (p0 < ps.n_pairs) put_cost(ps, p0, a, b, res, sq);
+    if (p0 < ps.n_pairs) put_cost(ps, p0, res, sq);
 }
 
 // Plain DTW on padded bands is held to two waves per SIMD like the exact
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 #pragma unroll
     for (int k = 0; k < B; ++k)
         if (k == g.kf) res = row[k];
-    if (live) put_cost(ps, p0, a, b, res, sq);
+    if (live) put_cost(ps, p0, res, sq);
 }
 
 }  // namespace wbx

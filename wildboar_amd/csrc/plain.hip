@@ -38,7 +38,7 @@ __global__ __launch_bounds__(64) void k_plain_dtw(PairSpec ps, Series<T> xs,
     const int w = w_fixed > 0 ? w_fixed : band_w(lx, ly, rr);
     const T res = block_dtw<T, AD>(xs.row(a), lx, ys.row(b), ly, w, weights, buf, buf + cap,
                                    buf + 2 * cap, pen);
-    if (threadIdx.x == 0) put_cost(ps, p, a, b, res, sq);
+    if (threadIdx.x == 0) put_cost(ps, p, res, sq);
 }
 
 // A measurement baseline, selected only by the batch plan's policy 2: the
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(64) void k_plain_dtw_padded(PairSpec ps, Series<T> 
         d1 = d0;
         d0 = t;
     }
-    if (tid == 0) put_cost(ps, p, a, b, res, sq);
+    if (tid == 0) put_cost(ps, p, res, sq);
 }
 
 template <typename T>
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void k_euclid_grid(PairSpec ps, Series<T> xs, 
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int64_t b = b0 + tx + 16 * j;
-            if (b < ny) put_cost(ps, a * ny + b, a, b, acc[i][j], sq);
+            if (b < ny) put_cost(ps, a * ny + b, acc[i][j], sq);
         }
     }
 }
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void k_euclid_pairs(PairSpec ps, Series<T> xs,
         }
         if (dist < min_dist) min_dist = dist;
     }
-    put_cost(ps, p, a, b, min_dist, sq);
+    put_cost(ps, p, min_dist, sq);
 }
 
 template <typename T>

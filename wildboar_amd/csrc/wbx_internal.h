@@ -136,28 +136,33 @@ __host__ __device__ inline void decode_pair(const PairSpec &ps, int64_t p,
     }
 }
 
-// The result of pair p = (a, b): its squared cost, or its distance in place.
-// The pair kernels end with it: a separate pass over the costs would cost
-// another launch and, on large matrices, reading them back.
+// The result of pair p: its squared cost, or its distance in place.  The pair
+// kernels end with it: a separate pass over the costs would cost another launch
+// and, on large matrices, reading them back.  Where the place depends on the
+// pair's (a, b) they are decoded again: kept from the kernel's start they take
+// four registers through its whole loop (float64 lanes of 8 slots 78 -> 82, one
+// wave per SIMD less; 1000 x 1000 pairs of 24 105 -> 112 us).
 template <typename T>
-__device__ __forceinline__ void put_cost(const PairSpec &ps, int64_t p, int64_t a, int64_t b, T c,
-                                         T *__restrict__ sq) {
+__device__ __forceinline__ void put_cost(const PairSpec &ps, int64_t p, T c, T *__restrict__ sq) {
     if (!ps.out) {
         sq[p] = c;
         return;
     }
     const double v = sqrt((double)c);
+    if (ps.mode == PAIR_GRID || ps.mode == PAIR_DIAG) {
+        ps.out[p] = v;
+        return;
+    }
+    asm volatile("" : "+v"(p));  // not the values the start of the kernel had
+    int64_t a, b;
+    decode_pair(ps, p, a, b);
+    ps.out[a * ps.ld + b] = v;
     if (ps.mode == PAIR_TRIANGLE) {
-        ps.out[a * ps.ld + b] = v;
         ps.out[b * ps.ld + a] = v;
         if (b == a + 1) {
             ps.out[a * ps.ld + a] = 0.0;
             if (b == ps.ny - 1) ps.out[b * ps.ld + b] = 0.0;
         }
-    } else if (ps.mode == PAIR_LIST) {
-        ps.out[a * ps.ld + b] = v;
-    } else {
-        ps.out[p] = v;
     }
 }
 
