@@ -47,3 +47,19 @@ def test_pruned_scan_is_exact(t, lens, r, kind):
         od, oi = oracle.subsequence(S, x, metric="dtw", r=r)
         np.testing.assert_array_equal(d, od)
         np.testing.assert_array_equal(i, oi)
+
+
+@pytest.mark.parametrize("n,ns", [(1, 1), (7, 1), (8, 1), (9, 1), (65, 2), (2731, 3), (2732, 3),
+                                  (3073, 3), (17000, 3)])
+def test_candidates_of_many_tasks(n, ns):
+    """A wave finishes the candidates of 8 tasks, of more from 8192 tasks on, of
+    48 at most; integers leave from one to too many candidates a task."""
+    rng = np.random.default_rng(n)
+    X = rng.integers(0, 6, (n, 26)).astype(np.float64)
+    X[::3] += rng.standard_normal((len(X[::3]), 26))
+    S = [rng.integers(0, 6, 12).astype(np.float64) for _ in range(ns)]
+    d, i = wd.pairwise_subsequence_distance(S, X, metric="dtw", metric_params={"r": 0.3},
+                                            return_index=True, precision="fp32")
+    od, oi = oracle.subsequence(S, X, metric="dtw", r=0.3)
+    np.testing.assert_array_equal(np.asarray(d).reshape(od.shape), od)
+    np.testing.assert_array_equal(np.asarray(i).reshape(oi.shape), oi)

@@ -641,9 +641,7 @@ int subseq_fast_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void 
     const size_t o_cost = cv.take((size_t)max_tasks * kMaxCand * 8);
     const size_t o_ovf = cv.take((size_t)n * (size_t)n_s * 4);
     const size_t o_list = cv.take((size_t)n_s * 4);
-    // class counters: overflowed tasks (64), the |x| max, candidates (from 128)
-    const size_t o_cnt = cv.take(192 * 4);
-    const size_t o_cl = cv.take((size_t)max_tasks * kMaxCand * 4);
+    const size_t o_cnt = cv.take(80 * 4);  // 64 class counters, then the |x| max
     const size_t o_env = cv.take(euclid ? 0 : (size_t)total * 8);
     MfmaPlan mf;
     size_t o_mf = 0;
@@ -661,7 +659,7 @@ int subseq_fast_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void 
     RC(stage<double>(dtype, X, n, t, xstr, ws, o_x64, &x64, st));
     RC(stage<double>(dtype, S, 1, total, total, ws, o_s64, &s64, st));
     int *cnt = (int *)(ws + o_cnt);
-    RC(launch_fill_i32(cnt, 192, 0, st));
+    RC(launch_fill_i32(cnt, 80, 0, st));
     double absmax = 0.0;
     const bool exact_inputs = dtype == WBX_F32;
     if (!mf_ids.empty()) {
@@ -716,14 +714,13 @@ int subseq_fast_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void 
         sg.A = (float)(eb.A * (1.0 + 1e-6));
         sg.lo = env;
         sg.hi = env + total;
-        const CandOut co{(uint32_t *)(ws + o_cl), cnt + 128 + c};
         TaskMap tm{list + cbeg[c], (int32_t)v.size()};
         const int64_t nt = n * (int64_t)v.size();
         {
             ProfScope pf(st, KERN_SUBSEQ);
-            RC(launch_subseq_fast(m->kind, c, tm, nt, sg, cands, co, st));
+            RC(launch_subseq_fast(m->kind, c, tm, nt, sg, cands, st));
         }
-        RC(launch_subseq_exact_cands(m->kind, c, tm, cands, co, nt, s64.ptr, s_off, s_len, x64.ptr,
+        RC(launch_subseq_exact_cands(m->kind, c, tm, cands, nt, s64.ptr, s_off, s_len, x64.ptr,
                                      x64.stride, (int)t, m->r, cost, st));
         RC(launch_subseq_select(tm, cands, nt, cost, n_s, dist, idx, ovf + n * cbeg[c], cnt + c,
                                 st));

@@ -32,12 +32,6 @@ struct SubCand {
     float best32;
 };
 
-// The candidates of a launch: the task of each (a task's are together).
-struct CandOut {
-    uint32_t *list;
-    int *n;
-};
-
 struct SubGeo {
     const float *S;     // packed shapelets (float32)
     const int64_t *off;
@@ -54,9 +48,9 @@ int launch_subseq_envelope(const float *S, const int64_t *off, const int64_t *le
                            double r, float *lo, float *hi, hipStream_t st);
 
 int launch_subseq_fast(int kind, int B, TaskMap tasks, int64_t n_tasks, SubGeo sg,
-                       SubCand *cands, CandOut co, hipStream_t st);
+                       SubCand *cands, hipStream_t st);
 int launch_subseq_exact_cands(int kind, int B, TaskMap tasks, const SubCand *cands,
-                              CandOut co, int64_t n_tasks, const double *S64, const int64_t *soff,
+                              int64_t n_tasks, const double *S64, const int64_t *soff,
                               const int64_t *slen, const double *X64, int64_t xstride, int T,
                               double r, double *cost64, hipStream_t st);
 int launch_subseq_select(TaskMap tasks, const SubCand *cands, int64_t n_tasks,

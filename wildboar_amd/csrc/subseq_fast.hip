@@ -92,8 +92,7 @@ __device__ __forceinline__ void cand_push(CandList &cl, int *s_win, float *s_cos
 // else the task is marked for the exact rescan (count kMaxCand + 1).
 __device__ __forceinline__ void cand_finish(const CandList &cl, const int *s_win,
                                             const float *s_cost, float tau, float best,
-                                            int64_t task, SubCand *__restrict__ out,
-                                            CandOut co) {
+                                            SubCand *__restrict__ out) {
     const int lane = threadIdx.x;
     __syncthreads();
     const bool has = !cl.overflow && lane < cl.count;
@@ -103,16 +102,11 @@ __device__ __forceinline__ void cand_finish(const CandList &cl, const int *s_win
     const uint64_t km = __ballot(keep);
     const int n = (int)__popcll(km);
     const bool ovf = cl.overflow || n > kMaxCand;
-    const int pos = (int)__popcll(km & ((1ull << lane) - 1ull));
-    if (!ovf && keep) out->win[pos] = w;
-    unsigned base = 0;
+    if (!ovf && keep) out->win[__popcll(km & ((1ull << lane) - 1ull))] = w;
     if (lane == 0) {
         out->count = ovf ? kMaxCand + 1 : n;
         out->best32 = best;
-        if (!ovf) base = atomicAdd((unsigned *)co.n, (unsigned)n);
     }
-    base = (unsigned)__shfl((int)base, 0);
-    if (!ovf && keep) co.list[(size_t)base + pos] = (uint32_t)task;
 }
 
 // Four consecutive floats of a row of length T starting at e (e >= 0): one
@@ -239,7 +233,7 @@ constexpr int kLbTrial = 512;
 // all classes, 7.9 ms when every window's DTW was computed.
 template <int BP, int U>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(subseq_dtw32_waves(BP)))) void
-k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands, CandOut co) {
+k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands) {
     const int lane = threadIdx.x;
     const SubTask tk = tasks.at(blockIdx.x);
     // the shapelet is the same for every lane and is not written by the
@@ -272,7 +266,7 @@ k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands, CandOut co
             tau = sg.rho * (best + sg.A) + sg.A;
             cand_push(cl, s_win, s_cost, active && c <= tau, ws, c, tau);
         }
-        cand_finish(cl, s_win, s_cost, tau, best, blockIdx.x, cands + blockIdx.x, co);
+        cand_finish(cl, s_win, s_cost, tau, best, cands + blockIdx.x);
         return;
     }
     const int step = (nwin + 63) / 64;  // the spread windows are lane * step
@@ -351,7 +345,7 @@ k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands, CandOut co
         tau = sg.rho * (best + sg.A) + sg.A;
         cand_push(cl, s_win, s_cost, active && c <= tau, ws, c, tau);
     }
-    cand_finish(cl, s_win, s_cost, tau, best, blockIdx.x, cands + blockIdx.x, co);
+    cand_finish(cl, s_win, s_cost, tau, best, cands + blockIdx.x);
 }
 
 // Envelope of each packed shapelet over the band's columns, |k - j| < w.
@@ -382,7 +376,7 @@ __global__ __launch_bounds__(64) void k_subseq_envelope(const float *__restrict_
 // with one 16-byte load.  Each window's sum runs over j in order.
 template <int U>
 __global__ __launch_bounds__(64) void k_subseq_euclid32(TaskMap tasks, SubGeo sg,
-                                                        SubCand *__restrict__ cands, CandOut co) {
+                                                        SubCand *__restrict__ cands) {
     static_assert(U == 4, "four windows per lane");
     const int lane = threadIdx.x;
     const SubTask tk = tasks.at(blockIdx.x);
@@ -449,35 +443,53 @@ __global__ __launch_bounds__(64) void k_subseq_euclid32(TaskMap tasks, SubGeo sg
             cand_push(cl, s_win, s_cost, active && c <= tau, ws, c, tau);
         }
     }
-    cand_finish(cl, s_win, s_cost, sg.rho * (best + sg.A) + sg.A, best, blockIdx.x,
-                cands + blockIdx.x, co);
+    cand_finish(cl, s_win, s_cost, sg.rho * (best + sg.A) + sg.A, best,
+                cands + blockIdx.x);
 }
 
 // ------------------------------------------------------------------ exact
 // Float64 cost of one candidate window per lane; per-lane geometry (all lanes
 // of a launch share BP).  Same arithmetic as dtw_distance: rows of S against
-// the window, cost = min(min(up, left), diag) + v * v.  The lanes go over the
-// launch's candidate list (most tasks have one or two of the kMaxCand; a lane
-// for each place left seven of eight idle).
+// the window, cost = min(min(up, left), diag) + v * v.  A wave lists the
+// candidates of `per` tasks in LDS and its lanes go over the list: most tasks
+// have one or two of the kMaxCand, and a lane for each place leaves seven of
+// eight idle.  (A list of the whole launch in memory takes a counter that every
+// task adds to, 13 ns each in turn: 1.03 ms for 80000 tasks of any length, 0.15
+// ms without.  Four waves of a block over one list take three times as long as
+// one wave where there are few tasks.)
+constexpr int kCandTasks = 48;
+
 template <int BP>
 __global__ __launch_bounds__(64) void k_subseq_cand64(TaskMap tasks,
                                                       const SubCand *__restrict__ cands,
-                                                      CandOut co, const double *__restrict__ S64,
+                                                      int64_t n_tasks, int per,
+                                                      const double *__restrict__ S64,
                                                       const int64_t *__restrict__ soff,
                                                       const int64_t *__restrict__ slen,
                                                       const double *__restrict__ X64,
                                                       int64_t xstride, int T, double r, int kind,
                                                       double *__restrict__ cost64) {
-    const int64_t n = (int64_t)(unsigned)*co.n;
-    for (int64_t q = (int64_t)blockIdx.x * 64 + threadIdx.x; q < n; q += (int64_t)gridDim.x * 64) {
-        const int64_t t = co.list[q];
-        int slot = 0;  // a task's entries are together, in the order of its places
-        while (slot < kMaxCand - 1 && q - 1 - slot >= 0 && co.list[q - 1 - slot] == (uint32_t)t)
-            ++slot;
+    __shared__ uint16_t list[kCandTasks * kMaxCand];  // (task - t0) * kMaxCand + place
+    const int lane = threadIdx.x;
+    const int64_t t0 = (int64_t)blockIdx.x * per;
+    int c = lane < per && t0 + lane < n_tasks ? cands[t0 + lane].count : 0;
+    if (c > kMaxCand) c = 0;  // rescanned
+    int inc = c;              // inclusive scan over the lanes
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(inc, d);
+        if (lane >= d) inc += o;
+    }
+    for (int s = 0; s < c; ++s) list[inc - c + s] = (uint16_t)(lane * kMaxCand + s);
+    const int n = __shfl(inc, 63);
+    __syncthreads();
+    for (int q = lane; q < n; q += 64) {
+        const int64_t at = t0 * kMaxCand + list[q];
+        const int64_t t = at / kMaxCand;
         const SubTask tk = tasks.at(t);
         const double *S = S64 + soff[tk.shapelet];
         const int L = (int)slen[tk.shapelet];
-        const double *Y = X64 + (int64_t)tk.sample * xstride + cands[t].win[slot];
+        const double *Y = X64 + (int64_t)tk.sample * xstride + cands[t].win[at - t * kMaxCand];
         double res;
         if (kind == WBX_EUCLIDEAN) {
             double dist = 0.0;
@@ -496,12 +508,12 @@ __global__ __launch_bounds__(64) void k_subseq_cand64(TaskMap tasks,
             res = lane64_cost<BP, 4, false, false, true>(S, L, Y, L, w - 1, 2 * w - 1, w - 1,
                                                          nullptr, L);
         }
-        cost64[t * kMaxCand + slot] = res;
+        cost64[at] = res;
     }
 }
 
-// Per task: first strictly smallest exact cost among the candidates (window
-// order = index order; euclidean candidates are sorted here first).
+// Per task: the smallest exact cost among the candidates, of equal ones the
+// first window (the list is in the order in which the windows were looked at).
 __global__ __launch_bounds__(256) void k_subseq_select(TaskMap tasks,
                                                        const SubCand *__restrict__ cands,
                                                        int64_t n_tasks,
@@ -624,19 +636,17 @@ int launch_subseq_envelope(const float *S, const int64_t *off, const int64_t *le
 }
 
 int launch_subseq_fast(int kind, int B, TaskMap tasks, int64_t n_tasks, SubGeo sg,
-                       SubCand *cands, CandOut co, hipStream_t st) {
+                       SubCand *cands, hipStream_t st) {
     if (n_tasks <= 0) return WBX_OK;
     if (n_tasks > 0x7fffffff) return fail(WBX_EUNSUPPORTED, "too many subsequence tasks");
     const dim3 grid((unsigned)n_tasks);
     if (kind == WBX_EUCLIDEAN) {
-        hipLaunchKernelGGL(k_subseq_euclid32<4>, grid, dim3(64), 0, st, tasks, sg, cands,
-                           co);
+        hipLaunchKernelGGL(k_subseq_euclid32<4>, grid, dim3(64), 0, st, tasks, sg, cands);
     } else {
         switch (B) {
 #define SD_CASE(B_, U_) \
-    case B_:                                                                                  \
-        hipLaunchKernelGGL((k_subseq_dtw32<B_, U_>), grid, dim3(64), 0, st, tasks, sg, cands, \
-                           co);                                                               \
+    case B_:                                                                                   \
+        hipLaunchKernelGGL((k_subseq_dtw32<B_, U_>), grid, dim3(64), 0, st, tasks, sg, cands); \
         break;
             SUB_SCAN_CASES(SD_CASE)
 #undef SD_CASE
@@ -648,19 +658,21 @@ int launch_subseq_fast(int kind, int B, TaskMap tasks, int64_t n_tasks, SubGeo s
 }
 
 int launch_subseq_exact_cands(int kind, int B, TaskMap tasks, const SubCand *cands,
-                              CandOut co, int64_t n_tasks, const double *S64, const int64_t *soff,
+                              int64_t n_tasks, const double *S64, const int64_t *soff,
                               const int64_t *slen, const double *X64, int64_t xstride, int T,
                               double r, double *cost64, hipStream_t st) {
     if (n_tasks <= 0) return WBX_OK;
-    // the list's length stays on the device: a grid for two candidates a task
-    // at most, each block going on by the grid's width
-    const int64_t nb = (n_tasks * 2 + 63) / 64;
-    const dim3 grid((unsigned)(nb < 65536 ? nb : 65536));
+    // A wave per SIMD while it then has eight tasks or more (eight: one turn of
+    // the lanes whatever their candidates), up to kCandTasks in larger launches
+    // (their one or two each about fill the lanes).
+    const int64_t want = (n_tasks + 1023) / 1024;
+    const int per = (int)(want < 8 ? 8 : want < kCandTasks ? want : kCandTasks);
+    const dim3 grid((unsigned)((n_tasks + per - 1) / per));
     switch (kind == WBX_EUCLIDEAN ? 8 : (B + 7) / 8 * 8) {
 #define C_CASE(B_, U_)                                                                            \
     case B_:                                                                                      \
-        hipLaunchKernelGGL(k_subseq_cand64<B_>, grid, dim3(64), 0, st, tasks, cands, co, S64,      \
-                           soff, slen, X64, xstride, T, r, kind, cost64);                         \
+        hipLaunchKernelGGL(k_subseq_cand64<B_>, grid, dim3(64), 0, st, tasks, cands, n_tasks, per, \
+                           S64, soff, slen, X64, xstride, T, r, kind, cost64);                    \
         break;
         SUB_DTW_CASES(C_CASE)
 #undef C_CASE
