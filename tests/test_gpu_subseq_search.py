@@ -1,7 +1,7 @@
 """The pruned float32 subsequence DTW scan: distances and indices are the
 reference's exactly, whatever windows its bounds leave out.  Window counts
-around 64 (the spread windows), 256 (a round of bounds) and its trial length,
-shapelets shorter than a bound's four terms, every kind of band, equal windows
+around 64 (the spread windows), 256 (a round of bounds) and the first rounds
+without them, shapelets shorter than a bound's four terms, every kind of band, equal windows
 (which overflow the candidate list) and data on which no bound prunes."""
 
 import numpy as np
@@ -38,6 +38,8 @@ def _data(kind, n, t, lens, seed):
     (900, (60, 128), 0.24),            # bands to 59 slots
     (600, (40, 33), 0.05),             # one-slot bands
     (400, (47, 50), 1.0),
+    (1400, (60, 63), 0.1),             # on both sides of the fewest windows with bounds
+    (5000, (30, 64), 0.2),             # several pauses between the bounds
 ])
 def test_pruned_scan_is_exact(t, lens, r, kind):
     X, S = _data(kind, 4, t, lens, t + len(lens))

@@ -42,17 +42,17 @@ def test_no_scalar_pair_takes_a_literal_for_a_double(code_objects):
         assert not (((w[:-1] & 0xFF80FFFF) == 0xBE8001FF) & (w[1:] == 0)).any()
 
 
+def _kernels(elf):
+    at = elf.find(b"AMDGPU\0")
+    size, kind = struct.unpack_from("<II", elf, at - 8)
+    assert kind == 32  # the metadata note: name (8 bytes), then msgpack
+    return msgpack.unpackb(elf[at + 8:at + 8 + size])["amdhsa.kernels"]
+
+
 @pytest.fixture(scope="module")
 def registers(code_objects):
     """Vector registers of every kernel, by its mangled name."""
-    out = {}
-    for elf in code_objects:
-        at = elf.find(b"AMDGPU\0")
-        size, kind = struct.unpack_from("<II", elf, at - 8)
-        assert kind == 32  # the metadata note: name (8 bytes), then msgpack
-        for k in msgpack.unpackb(elf[at + 8:at + 8 + size])["amdhsa.kernels"]:
-            out[k[".name"]] = k[".vgpr_count"]
-    return out
+    return {k[".name"]: k[".vgpr_count"] for elf in code_objects for k in _kernels(elf)}
 
 
 @pytest.mark.parametrize("kernel,most", [
@@ -67,3 +67,16 @@ def test_writing_distances_in_place_keeps_the_waves(registers, kernel, most):
     without the place of the result kept through the loop."""
     (got,) = [v for name, v in registers.items() if kernel in name]
     assert got <= most
+
+
+def test_subsequence_scans_do_not_spill(code_objects):
+    """The band's offset is a constant of the class, so the tests of which
+    window entries lie inside the window are scalar: as wave masks kept over all
+    windows they were several hundred spilled registers."""
+    spilled = {}
+    for elf in code_objects:
+        for k in _kernels(elf):
+            if "k_subseq_dtw32" in k[".name"]:
+                spilled[k[".name"]] = (k[".vgpr_spill_count"], k[".sgpr_spill_count"])
+    assert len(spilled) == 32
+    assert all(v == 0 and s <= 128 for v, s in spilled.values())

@@ -688,7 +688,10 @@ int subseq_fast_impl(DeviceCtx *ctx, const wbx_metric *m, int dtype, const void 
     WBX_HIP_CHECK(hipMemcpyAsync(list, lists.data(), sizeof(int32_t) * lists.size(),
                                  hipMemcpyHostToDevice, st));
     float *env = (float *)(ws + o_env);
-    if (!euclid)
+    bool bounds = false;  // whether any task forms LB_Keogh sums
+    for (int c = 1; c < 64 && !euclid; ++c)
+        for (int32_t j : cls[c]) bounds = bounds || subseq_bounds(c, (int)(t - hl[j] + 1));
+    if (bounds)
         RC(launch_subseq_envelope(s32.ptr, s_off, s_len, n_s, m->r, env, env + total, st));
     // FP32 scan, FP64 finish of the candidates and selection for every class;
     // tasks whose candidates overflowed are listed per class and rescanned

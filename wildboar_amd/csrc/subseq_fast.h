@@ -44,6 +44,14 @@ struct SubGeo {
     const float *lo, *hi;  // the shapelets' envelopes, packed like S (DTW)
 };
 
+// Whether a task of `nwin` windows at band width B looks at LB_Keogh sums.  The
+// trial whether they pay takes about 3 / B of the time of 64 windows' DTW and,
+// while a task has its SIMD to itself, waits for its loads: with few windows it
+// shows.
+__host__ __device__ constexpr bool subseq_bounds(int B, int nwin) {
+    return B > 3 && (int64_t)nwin * B >= 6000;
+}
+
 int launch_subseq_envelope(const float *S, const int64_t *off, const int64_t *len, int64_t n_s,
                            double r, float *lo, float *hi, hipStream_t st);
 

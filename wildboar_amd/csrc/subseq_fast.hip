@@ -128,10 +128,13 @@ __device__ __forceinline__ f4u row4(const float *__restrict__ row, int e, int T)
 template <int BP, int U>
 __device__ __forceinline__ float window_cost32(const float *__restrict__ S,
                                                const __attribute__((address_space(4))) float *Sc,
-                                               int L, int off, const float *__restrict__ Y, int sw,
+                                               int L, const float *__restrict__ Y, int sw,
                                                float lim) {
     static_assert(U % 4 == 0, "groups of whole 16-byte loads");
-    constexpr int W = BP + U - 1;
+    constexpr int W = BP + U - 1, off = (BP - 1) / 2;
+    // the tests on it below stay here: formed once for all calls they are
+    // several hundred scalar values, spilled and read back for every call
+    asm volatile("" : "+s"(L));
     float row[BP];
 #pragma unroll
     for (int k = 0; k < BP; ++k) row[k] = (k == off) ? 0.0f : WBX_INF_F;
@@ -216,24 +219,27 @@ __device__ __forceinline__ float window_cost32(const float *__restrict__ S,
     return c;
 }
 
-// Waves per SIMD the register allocation is held to, by band class: left
-// alone the allocator spreads the window-batch set-up over many registers;
-// 13 and 15 fit four waves and 17 .. 23 three without spills (wider classes
-// would spill).
-constexpr int subseq_dtw32_waves(int BP) {
-    return BP <= 11 ? 1 : BP <= 15 ? 4 : BP <= 23 ? 3 : 1;
+// LB_Keogh sums against the DTW they save: per value of the shapelet the sums
+// of 256 windows take the time of about 24 instructions and their DTW has 12 B,
+// so they pay where more than 2 / B of the windows fall to them.  What share
+// that is shows on the spread windows first; where it is smaller, the next four
+// groups of 256 go straight to the DTW, after a further group that falls short
+// the next eight, and so on up to kLbPause (the best so far falls, so a task can
+// come to pay).  Tasks of few windows (subseq_bounds) take them in order.
+// Starting with one group takes 1 % less time on the shapelets below and 5 %
+// more on white noise.
+constexpr int kLbPause = 16;
+// whether `kept` of n windows are too many for the sums to pay
+__device__ __forceinline__ bool subseq_short(int B, int kept, int n) {
+    return (n - kept) * B < 2 * n;
 }
-
-// Windows whose LB_Keogh sums were formed before the scan decides whether
-// they are worth forming: with more than three quarters of them left, the
-// rest of the task's windows go straight to the DTW.
-constexpr int kLbTrial = 512;
 
 // 256 shapelets of 16 .. 128 over 500 series of 1024, r = 0.1: 3.4 ms for
 // all classes, 7.9 ms when every window's DTW was computed.
 template <int BP, int U>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(subseq_dtw32_waves(BP)))) void
-k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands) {
+__global__ __launch_bounds__(64) void k_subseq_dtw32(TaskMap tasks, SubGeo sg,
+                                                     SubCand *__restrict__ cands) {
+    // every shapelet of the launch has a band of 2 w - 1 == BP slots
     const int lane = threadIdx.x;
     const SubTask tk = tasks.at(blockIdx.x);
     // the shapelet is the same for every lane and is not written by the
@@ -243,8 +249,7 @@ k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands) {
     const int64_t so = sg.off[tk.shapelet];
     const float *__restrict__ S = sg.S + so;
     const cfp Sc = (cfp)S, lo = (cfp)(sg.lo + so), hi = (cfp)(sg.hi + so);
-    const int L = (int)sg.len[tk.shapelet];
-    const int off = band_w(L, L, sg.r) - 1;  // the band has 2 w - 1 == BP slots
+    const int L = __builtin_amdgcn_readfirstlane((int)sg.len[tk.shapelet]);
     const int T = sg.T, nwin = T - L + 1;
     const float *__restrict__ Xrow = sg.X + (int64_t)tk.sample * sg.xstride;
     __shared__ int s_win[kCap];
@@ -252,15 +257,12 @@ k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands) {
     __shared__ int queue[64 + 256];
     CandList cl{0, false};
     float best = WBX_INF_F, tau = WBX_INF_F;
-    if constexpr (BP <= 3) {
-        // a row costs about what its LB_Keogh terms would: every window, in
-        // order (B = 1: 36 us so, 82 us pruned; B = 3: 111 and 149; B = 5:
-        // 181 and 163)
+    if (!subseq_bounds(BP, nwin)) {
         for (int b0 = 0; b0 < nwin; b0 += 64) {
             const int ws = b0 + lane;
             const bool active = ws < nwin;
             const int wc = active ? ws : nwin - 1;
-            float c = window_cost32<BP, U>(S, Sc, L, off, Xrow + wc, wc, WBX_INF_F);
+            float c = window_cost32<BP, U>(S, Sc, L, Xrow + wc, wc, tau);
             if (!active) c = WBX_INF_F;
             best = fminf(best, wave_min(c));
             tau = sg.rho * (best + sg.A) + sg.A;
@@ -269,19 +271,42 @@ k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands) {
         cand_finish(cl, s_win, s_cost, tau, best, cands + blockIdx.x);
         return;
     }
-    const int step = (nwin + 63) / 64;  // the spread windows are lane * step
-    int nq = 0, b0 = 0, tested = 0, left = 0;
+    const int step = (nwin + 63) / 64;  // >= 2; the spread windows are lane * step
+    int nq = 0, b0 = 0;
+    // The windows that go straight to the DTW: the others of [.., b0), by their
+    // number i0 .. i1 - 1 among the others; di, dr: the lane's number over and
+    // modulo step - 1.
+    int i0 = 0, i1 = 0, di = 0, dr = 0, pause = 4;
+    auto others = [&](int s) { return s - (s + step - 1) / step; };  // below window s
+    auto straight = [&]() {
+        const int e = b0 + 256 * pause < nwin ? b0 + 256 * pause : nwin;
+        pause = 2 * pause < kLbPause ? 2 * pause : kLbPause;
+        i0 = others(b0);
+        i1 = others(e);
+        di = (i0 + lane) / (step - 1);
+        dr = (i0 + lane) % (step - 1);
+        b0 = e;
+    };
     for (bool first = true;; first = false) {
         int ws = lane * step;
         bool active = ws < nwin;
-        if (!first) {
-            const bool bound = tested < kLbTrial || left * 4 <= tested * 3;
+        if (!first && i0 < i1) {
+            active = i0 + lane < i1;
+            ws = active ? di * step + dr + 1 : 0;
+            i0 += 64;
+            di += 64 / (step - 1);
+            dr += 64 % (step - 1);
+            if (dr >= step - 1) {
+                dr -= step - 1;
+                ++di;
+            }
+        } else if (!first) {
             while (nq < 64 && b0 < nwin) {
                 // lane l forms the sums of the windows w0 .. w0 + 3
                 const int w0 = b0 + 4 * lane;
                 const float lim = tau * sg.rho * sg.rho * 1.000001f;
                 float lb[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (bound) {
+                {
                     float xw[8];
                     const f4u a = row4(Xrow, w0 < T ? w0 : T - 1, T),
                               b = row4(Xrow, w0 + 4 < T ? w0 + 4 : T - 1, T);
@@ -314,23 +339,27 @@ k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands) {
                         }
                     }
                 }
-                int kept = 0;
+                int kept = 0, rem = w0 % step;  // rem 0: a spread window
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int s = w0 + q;
-                    const bool keep = s < nwin && s % step != 0 && !(lb[q] > lim);
+                    const bool keep = s < nwin && rem != 0 && !(lb[q] > lim);
                     const uint64_t km = __ballot(keep);
                     if (keep) queue[nq + kept + (int)__popcll(km & ((1ull << lane) - 1ull))] = s;
                     kept += (int)__popcll(km);
+                    rem = rem + 1 == step ? 0 : rem + 1;
                 }
                 nq += kept;
-                if (bound) {
-                    tested += 256;
-                    left += kept;
-                }
+                const bool few = subseq_short(BP, kept, min(256, nwin - b0));
                 b0 += 256;
                 __syncthreads();
+                if (few && b0 < nwin) {
+                    straight();
+                    break;
+                }
+                if (!few) pause = 4;
             }
+            if (nq < 64 && i0 < i1) continue;
             if (nq == 0) break;
             active = lane < nq;
             // the newest 64 of the queue
@@ -339,11 +368,26 @@ k_subseq_dtw32(TaskMap tasks, SubGeo sg, SubCand *__restrict__ cands) {
             __syncthreads();
         }
         const int wc = active ? ws : (first ? 0 : ws);
-        float c = window_cost32<BP, U>(S, Sc, L, off, Xrow + wc, wc, tau);
+        float c = window_cost32<BP, U>(S, Sc, L, Xrow + wc, wc, tau);
         if (!active) c = WBX_INF_F;
         best = fminf(best, wave_min(c));
         tau = sg.rho * (best + sg.A) + sg.A;
         cand_push(cl, s_win, s_cost, active && c <= tau, ws, c, tau);
+        if (first) {  // how many of these would their sums have kept
+            const float lim = tau * sg.rho * sg.rho * 1.000001f;
+            const float *__restrict__ x = Xrow + wc;
+            float lb = 0.0f;
+            for (int j0 = 0; j0 + 4 <= L; j0 += 4) {
+                const f4a v = *(const f4a *)(x + j0);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const float d = fmaxf(fmaxf(v[u] - hi[j0 + u], lo[j0 + u] - v[u]), 0.0f);
+                    lb = __builtin_fmaf(d, d, lb);
+                }
+            }
+            const int kept = (int)__popcll(__ballot(active && !(lb > lim)));
+            if (subseq_short(BP, kept, (int)__popcll(__ballot(active)))) straight();
+        }
     }
     cand_finish(cl, s_win, s_cost, tau, best, cands + blockIdx.x);
 }
