@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import oracle
-from wildboar_amd import device
+from wildboar_amd import _lib, device
 
 pytestmark = pytest.mark.gpu
 
@@ -71,3 +71,18 @@ def test_output_in_the_memory_of_an_input(metric):
     flat = Pd.view(-1)[:300]
     assert torch.equal(device.paired(Pd, Pd.flip(0), metric=metric, r=0.1, precision="fp64",
                                      out=flat), want)
+
+
+@pytest.mark.parametrize("nx,ny,kind", [(100, 200, 6), (300, 300, 2), (400, 320, 2)])
+def test_two_waves_per_simd_take_the_lanes(nx, ny, kind):
+    """B = 49: the lanes (kind 2) from a second wave per SIMD on, where they
+    take 265 us on 90000 pairs of 800 and the group kernel (6) 307."""
+    X = torch.randn((nx, 256), device="cuda")
+    Y = torch.randn((ny, 256), device="cuda")
+    _lib.prof_enable(True)
+    try:
+        device.pairwise(X, Y, metric="dtw", r=0.1, precision="fp32")
+        _, launches, last = _lib.prof_take()
+    finally:
+        _lib.prof_enable(False)
+    assert (launches, last) == (1, kind)

@@ -276,9 +276,12 @@ int run_pairs(const wbx_metric *m, const PairSpec &ps, Series<T> xs, Series<T> y
         // One pair per lane does the fewest instructions per cell, a group of
         // lanes per pair has the shorter chain: whichever is estimated
         // faster for this many pairs.  Per row, a lane wave alone on its SIMD
-        // takes 5.5 ns a slot and shares it at 3.3 (float32 DTW; measured at
+        // takes 5.5 ns a slot and shares it at 3.4 (float32 DTW; measured at
         // B = 23, 49, 101; at 20000 pairs of 512, B = 101, 293 us against
-        // 124 us of six lanes a pair, at 100000 359 against 469).  Padded
+        // 124 us of six lanes a pair, at 100000 359 against 469).  A second
+        // wave issues in the first one's gaps, so two take the larger of one
+        // alone and their two shares (90000 pairs of 800, B = 49: 265 us, the
+        // group kernel 307).  Padded
         // widths, weights and float64 cost more; float32 WDTW and float64
         // lanes are for bands up to 40 slots (at 49 the group kernel is
         // 1.1-1.4x faster at any size); ADTW has no group form.
@@ -290,8 +293,11 @@ int run_pairs(const wbx_metric *m, const PairSpec &ps, Series<T> xs, Series<T> y
             lane = lane_supported(xs.len, ys.len, m->r, wt, w_fixed) && (!wt || B <= 40);
             const bool exact = !wt && lane_exact_supported(B);
             const int slots = exact ? B : (B + 7) / 8 * 8;
-            lane_ns = pair_launch_ns(lane_waves, bd.lx, (exact ? 20.0 : 30.0) + (wt ? 7.5 : 5.5) * slots,
-                                     (wt ? 4.8 : 3.4) * slots);
+            const double alone = (exact ? 20.0 : 30.0) + (wt ? 7.5 : 5.5) * slots;
+            const double share = (wt ? 4.8 : 3.4) * slots;
+            const bool two = !wt && lane_waves > 1024 && lane_waves <= 2048;
+            lane_ns = two ? pair_launch_ns(1, bd.lx, std::max(alone, 2.0 * share), 0.0)
+                          : pair_launch_ns(lane_waves, bd.lx, alone, share);
         } else {
             const int slots = lane64_pairs_class(B, wt);
             lane = slots != 0 && (B <= 40 || pen);
