@@ -45,3 +45,15 @@ def test_replay_heap_in_lds_and_in_memory(k):
     oi, od = oracle.argmin(X, Y, k=k, metric="dtw", r=0.1)
     np.testing.assert_array_equal(idx, oi)
     np.testing.assert_array_equal(dist, od)
+
+
+@pytest.mark.parametrize("nx,ny,k", [(4096, 3, 1), (4097, 66, 5), (8193, 70, 3), (266300, 3, 2)])
+def test_many_rows(nx, ny, k):
+    """From 4097 rows on a wave takes several, 64 at most."""
+    X, Y = _series(nx, 12, 5, "walks"), _series(ny, 12, 6, "walks")
+    X[::5] = Y[0]  # some rows with a distance of 0
+    idx, dist = wd.argmin_distance(X, Y, k=k, metric="dtw", metric_params={"r": 0.2},
+                                   return_distance=True, precision="fp32")
+    oi, od = oracle.argmin(X, Y, k=k, metric="dtw", r=0.2)
+    np.testing.assert_array_equal(idx, oi)
+    np.testing.assert_array_equal(dist, od)

@@ -63,100 +63,116 @@ __device__ __forceinline__ double lane_value(double v, int q) {
 // the start of its 64 can neither be a candidate nor change T (hi >= lo), and
 // one comparison with the cost at which lo reaches T drops it.  The others
 // are taken in column order, which selects what a scan of the row selects.
-// A row's candidates are one bit per column in `words` (the lane that stores
-// a word reads it back); when the row is done the wave reserves their places in the pair list with one atomic and writes
-// them there in column order (the order of the rows in the list is free).
+// A row's candidates are one bit per column in `words` (the lane that stores a
+// word reads it back).  When the `per` rows of a wave are done it reserves
+// their places in the pair list with one atomic and writes them there, each
+// row's in column order (the order of the rows in the list is free).
 //
 // Bound by the latency of the loads and of the selection steps (a row needs
-// about k ln(ny / k) of them).  500 rows of 4000, k = 5: 40 us.  One
-// lane per row, in two passes with a division and a square root for every
-// cost, took 2 x 2390 us there: 8 waves, their loads ny floats apart.
+// about k ln(ny / k) of them).  500 rows of 4000, k = 5: 40 us.  One lane per
+// row, in two passes with a division and a square root for every cost, took 2 x
+// 2390 us there: 8 waves, their loads ny floats apart.  The atomics of a launch
+// run one after the other, 13 ns each: with one per row 100000 rows of 10
+// took 1.3 ms for them alone.
 __global__ __launch_bounds__(64) void k_argmin_candidates(
-    const float *__restrict__ sq, int64_t nx, int64_t ny, int k, ErrBound eb,
+    const float *__restrict__ sq, int64_t nx, int64_t ny, int k, int per, ErrBound eb,
     const unsigned *__restrict__ absmax_bits, uint64_t *words, int64_t *__restrict__ offs,
     int64_t *__restrict__ counts, unsigned long long *__restrict__ total,
     int32_t *__restrict__ pa, int32_t *__restrict__ pb) {
-    const int64_t i = (int64_t)blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
-    if (i >= nx) return;  // uniform
+    const int64_t i0 = (int64_t)blockIdx.x * per;
+    const int rows = (int)(nx - i0 < per ? nx - i0 : per);
     const int lane = threadIdx.x;
     if (absmax_bits) {  // A was made for |x| <= 1
         const double m = (double)__uint_as_float(*absmax_bits);
         eb.A *= m * m;
     }
-    const float *__restrict__ row = sq + i * ny;
     const int64_t nw = (ny + 63) / 64;
-    uint64_t *wrow = words + i * nw;
-    // the starting +inf goes through a vector register: as a constant in a
-    // scalar pair the compiler writes it with one 32-bit literal, which is 0
-    double top = WBX_INF_D;
-    asm volatile("" : "+v"(top));
-    double T = lane_value(top, 0), cth = T;
-    int64_t cnt = 0;
-    constexpr int UC = 4;  // groups of 64 costs in flight
-    for (int64_t w0 = 0; w0 < nw; w0 += UC) {
-        float cv[UC];
+    int64_t own_cnt = 0;  // of row i0 + lane
+    for (int e = 0; e < rows; ++e) {
+        const float *__restrict__ row = sq + (i0 + e) * ny;
+        uint64_t *wrow = words + (i0 + e) * nw;
+        // the starting +inf goes through a vector register: as a constant in a
+        // scalar pair the compiler writes it with one 32-bit literal, which is 0
+        double top = WBX_INF_D;
+        asm volatile("" : "+v"(top));
+        double T = lane_value(top, 0), cth = T;
+        int64_t cnt = 0;
+        constexpr int UC = 4;  // groups of 64 costs in flight
+        for (int64_t w0 = 0; w0 < nw; w0 += UC) {
+            float cv[UC];
 #pragma unroll
-        for (int u = 0; u < UC; ++u) {
-            const int64_t j = (w0 + u) * 64 + lane;
-            cv[u] = j < ny ? row[j] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < UC; ++u) {
-            const int64_t j = (w0 + u) * 64 + lane;
-            if (w0 + u >= nw) break;  // uniform
-            const float c = cv[u];
-            // a cost that is not finite has lo = 0
-            uint64_t mask = __ballot(j < ny && (!(c < WBX_INF_F) || (double)c < cth));
-            uint64_t word = 0;
-            if (mask) {
-                double lo, hi;
-                dist_bounds(c, eb, lo, hi);
-                while (mask) {
-                    const int q = __builtin_ctzll(mask);
-                    mask &= mask - 1;
-                    if (lane_value(lo, q) < T) word |= (uint64_t)1 << q;
-                    const double hq = lane_value(hi, q);
-                    if (hq < T) {
-                        const int pos =
-                            __popcll(__ballot(lane < k && top <= hq));
-                        const double below = __shfl_up(top, 1);
-                        top = lane < pos ? top : lane == pos ? hq : below;
-                        T = lane_value(top, k - 1);
-                    }
-                }
-                // lo(c) < T only if c is below this
-                cth = (T * T / (1.0 - eb.e64) * eb.e_up + eb.A) * (1.0 + 1e-9);
-                cnt += __popcll(word);
+            for (int u = 0; u < UC; ++u) {
+                const int64_t j = (w0 + u) * 64 + lane;
+                cv[u] = j < ny ? row[j] : 0.0f;
             }
-            if (lane == (int)((w0 + u) & 63)) wrow[w0 + u] = word;
+#pragma unroll
+            for (int u = 0; u < UC; ++u) {
+                const int64_t j = (w0 + u) * 64 + lane;
+                if (w0 + u >= nw) break;  // uniform
+                const float c = cv[u];
+                // a cost that is not finite has lo = 0
+                uint64_t mask = __ballot(j < ny && (!(c < WBX_INF_F) || (double)c < cth));
+                uint64_t word = 0;
+                if (mask) {
+                    double lo, hi;
+                    dist_bounds(c, eb, lo, hi);
+                    while (mask) {
+                        const int q = __builtin_ctzll(mask);
+                        mask &= mask - 1;
+                        if (lane_value(lo, q) < T) word |= (uint64_t)1 << q;
+                        const double hq = lane_value(hi, q);
+                        if (hq < T) {
+                            const int pos =
+                                __popcll(__ballot(lane < k && top <= hq));
+                            const double below = __shfl_up(top, 1);
+                            top = lane < pos ? top : lane == pos ? hq : below;
+                            T = lane_value(top, k - 1);
+                        }
+                    }
+                    // lo(c) < T only if c is below this
+                    cth = (T * T / (1.0 - eb.e64) * eb.e_up + eb.A) * (1.0 + 1e-9);
+                    cnt += __popcll(word);
+                }
+                if (lane == (int)((w0 + u) & 63)) wrow[w0 + u] = word;
+            }
         }
+        if (lane == e) own_cnt = cnt;
+    }
+    int64_t inc = own_cnt;  // inclusive scan over the rows
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t o = __shfl_up(inc, d);
+        if (lane >= d) inc += o;
     }
     unsigned long long base = 0;
-    if (lane == 0) {
-        base = atomicAdd(total, (unsigned long long)cnt);
-        offs[i] = (int64_t)base;
-        counts[i] = cnt;
+    if (lane == 63) base = atomicAdd(total, (unsigned long long)inc);
+    base = (unsigned long long)__shfl((long long)base, 63);
+    if (lane < rows) {
+        offs[i0 + lane] = (int64_t)base + inc - own_cnt;
+        counts[i0 + lane] = own_cnt;
     }
-    base = (unsigned long long)__shfl((long long)base, 0);
-    for (int64_t w0 = 0; w0 < nw; w0 += 64) {
-        const int64_t wi = w0 + lane;
-        uint64_t word = wi < nw ? wrow[wi] : 0;  // stored by this lane
-        const int own = __popcll(word);
-        int inc = own;  // inclusive scan over the lanes
+    for (int e = 0; e < rows; ++e) {
+        const uint64_t *wrow = words + (i0 + e) * nw;
+        for (int64_t w0 = 0; w0 < nw; w0 += 64) {
+            const int64_t wi = w0 + lane;
+            uint64_t word = wi < nw ? wrow[wi] : 0;  // stored by this lane
+            const int own = __popcll(word);
+            int pre = own;  // inclusive scan over the lanes
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int o = __shfl_up(inc, d);
-            if (lane >= d) inc += o;
+            for (int d = 1; d < 64; d <<= 1) {
+                const int o = __shfl_up(pre, d);
+                if (lane >= d) pre += o;
+            }
+            unsigned long long q = base + (unsigned long long)(pre - own);
+            while (word) {
+                const int z = __builtin_ctzll(word);
+                word &= word - 1;
+                pa[q] = (int32_t)(i0 + e);
+                pb[q] = (int32_t)(wi * 64 + z);
+                ++q;
+            }
+            base += (unsigned long long)__shfl(pre, 63);
         }
-        unsigned long long q = base + (unsigned long long)(inc - own);
-        while (word) {
-            const int e = __builtin_ctzll(word);
-            word &= word - 1;
-            pa[q] = (int32_t)i;
-            pb[q] = (int32_t)(wi * 64 + e);
-            ++q;
-        }
-        base += (unsigned long long)__shfl(inc, 63);
     }
 }
 
@@ -171,10 +187,13 @@ int launch_argmin_candidates(const float *sq, int64_t nx, int64_t ny, int k, con
     if (k > KMAX) return fail(WBX_EUNSUPPORTED, "certified argmin supports k <= %d", KMAX);
     int rc = launch_fill_i32((int *)total, 2, 0, st);
     if (rc) return rc;
-    const int64_t gx = nx < 65535 ? nx : 65535;
-    hipLaunchKernelGGL(k_argmin_candidates, dim3((unsigned)gx, (unsigned)((nx + gx - 1) / gx)),
-                       dim3(64), 0, st, sq, nx, ny, k, eb, absmax_bits, (uint64_t *)words, offs,
-                       counts, total, pa, pb);
+    // a row a wave while four waves per SIMD do, at most 64 (a lane has a row's
+    // count)
+    const int64_t want = (nx + 4095) / 4096;
+    const int per = (int)(want < 64 ? want : 64);
+    hipLaunchKernelGGL(k_argmin_candidates, dim3((unsigned)((nx + per - 1) / per)), dim3(64), 0,
+                       st, sq, nx, ny, k, per, eb, absmax_bits, (uint64_t *)words, offs, counts,
+                       total, pa, pb);
     WBX_HIP_CHECK(hipGetLastError());
     WBX_HIP_CHECK(hipMemcpyAsync(total_host, total, sizeof(int64_t), hipMemcpyDeviceToHost, st));
     WBX_HIP_CHECK(hipStreamSynchronize(st));
