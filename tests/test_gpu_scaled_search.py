@@ -30,6 +30,9 @@ def _data(kind, n, t, lens, seed):
             s = S[i % len(S)]
             for o in range(0, t - len(s) + 1, len(s) + 3):
                 X[i, o:o + len(s)] = s * (1.0 + o) + i
+    elif kind == "sine":  # every period again, up to rounding
+        X = np.sin(np.arange(t) * (2 * np.pi / 25) + rng.uniform(0, 6, (n, 1)))
+        S = [np.sin(np.arange(L) * (2 * np.pi / 25) + rng.uniform(0, 6)) for L in lens]
     elif kind == "flat":
         X[:, t // 3: t // 3 + min(40, t // 2)] = 1.5
     return X, S
@@ -46,7 +49,8 @@ CASES = [  # t, lengths, r
 ]
 
 
-@pytest.mark.parametrize("kind", ["walks", "integers", "planted", "copies", "flat"])
+@pytest.mark.parametrize("kind", ["walks", "integers", "planted", "copies", "flat",
+                                  "sine"])
 @pytest.mark.parametrize("t,lens,r", CASES)
 def test_pruned_search_equals_every_window(t, lens, r, kind):
     n = 6

@@ -1196,8 +1196,15 @@ constexpr size_t kChunkCap = (size_t)512 << 20;    // window statistics + envelo
 constexpr size_t kTDCap = (size_t)256 << 20;       // per-window (T, D)
 constexpr int64_t kMaxWaves = 8192;
 // Smallest class (series times patterns) for the pruned search: a task is one
-// wave's 0.3 ms in turn, every window of 256 tasks in parallel takes that too.
-constexpr int64_t kSearchTasks = 256;
+// wave's work in turn, so few tasks leave SIMDs idle that every window in
+// parallel would use.  Time of the search against every window, series of 1024:
+//             256 tasks                      512 tasks
+//   B = 13    walks 0.72, noise 0.93         0.51, 0.63
+//   B = 25    0.76, 0.96                     0.52, 0.65
+//   B = 51    1.07, 1.27                     0.63, 0.75
+// Sines without noise, whose windows repeat up to rounding, leave the search
+// undecided and take 1.6, 2.6 and 3.3 there, 1.1, 1.7 and 2.0 with 512 tasks.
+constexpr int64_t search_tasks(int BP) { return BP <= 16 ? 256 : 512; }
 
 size_t scratch_bytes(int64_t max_len) {
     const size_t one = (size_t)64 * 8 * (size_t)(4 * max_len);  // at least one wave
@@ -1379,7 +1386,7 @@ int launch_scaled_subseq(int kind, double r, const double *S, const int64_t *s_o
         std::vector<char> searched(kMaxBPS / 8 + 1, 0);
         for (int c = 1; dtw && !wide_only && c <= kMaxBPS / 8; ++c) {
             const int64_t np = cls_beg[c + 1] - cls_beg[c];
-            if (np == 0 || np * cn < kSearchTasks) continue;
+            if (np == 0 || np * cn < search_tasks(8 * c)) continue;
             searched[c] = 1;
             SearchArgs sa{};
             sa.a.X = xc;
