@@ -586,7 +586,7 @@ int wbx_dtw_train_sizes(const wbx_metric *metric, int mode, int64_t nx, int64_t 
     if (rc) return rc;
     const int64_t np = mode == 0 ? nx * ny : nx;
     const Band bd = make_band((int)tx, (int)ty, metric->r);
-    if (small_train_ok(np, bd)) {
+    if (small_train_ok(mode, nx, ny, bd)) {
         small_train_sizes(mode, nx, ny, bd, state_bytes, scratch_bytes);
         return WBX_OK;
     }
@@ -621,7 +621,7 @@ int wbx_dev_dtw_train_forward(const wbx_metric *metric, int mode, const float *X
     float *sq = (float *)((char *)state + waves * tx * 2 * tg.NW * 64 * 4);
     Series<float> xs{X, x_stride, (int)tx, nullptr}, ys{Y, y_stride, (int)ty, nullptr};
     const Band bd = make_band((int)tx, (int)ty, metric->r);
-    if (small_train_ok(ps.n_pairs, bd)) return small_train_forward(ps, xs, ys, bd, D, state, st);
+    if (small_train_ok(mode, nx, ny, bd)) return small_train_forward(ps, xs, ys, bd, D, state, st);
     if (lane_exact_supported(tg.g.B)) {
         RCT(launch_lane_train_exact(ps, xs, ys, tg.g, sq, dirs, st));
         return launch_finish<float>(ps, sq, D, ny, st);
@@ -660,7 +660,7 @@ int wbx_dev_dtw_train_backward(const wbx_metric *metric, int mode, const float *
     PairSpec ps{mode == 0 ? PAIR_GRID : PAIR_DIAG, mode == 0 ? nx * ny : nx, mode == 0 ? ny : nx,
                 nullptr, nullptr};
     const Band bd = make_band((int)tx, (int)ty, metric->r);
-    if (small_train_ok(ps.n_pairs, bd))
+    if (small_train_ok(mode, nx, ny, bd))
         return small_train_backward(ps, Series<float>{X, x_stride, (int)tx, nullptr},
                                     Series<float>{Y, y_stride, (int)ty, nullptr}, bd, nx, ny, G,
                                     state, dX, ldx, dY, ldy_, scratch, st);

@@ -5,9 +5,9 @@
 
 namespace wbx {
 
-// Whether the small form serves a DTW call of n_pairs pairs (decided by the
-// sizes alone: forward, backward and the size query agree).
-bool small_train_ok(int64_t n_pairs, const Band &bd);
+// Whether the small form serves a DTW call of all (mode 0) or paired (1) series
+// (decided by the sizes alone: forward, backward and the size query agree).
+bool small_train_ok(int mode, int64_t nx, int64_t ny, const Band &bd);
 // Bytes of the state (decisions, squared costs) and of the backward's scratch.
 void small_train_sizes(int mode, int64_t nx, int64_t ny, const Band &bd, int64_t *state_bytes,
                        int64_t *scratch_bytes);

@@ -19,6 +19,8 @@
 // Bound by latency: the chain of cells of a row in the forward, the chain of
 // rows in the walk.  1 x 512 pairs of 256, r = 0.1, against one pair per lane
 // (8 waves): forward 221 -> 36 us, backward 334 -> 59 us.
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "lane_train.h"
@@ -31,10 +33,7 @@ namespace {
 constexpr int SU = 8;        // steps whose loads are issued together
 constexpr int kSmallMaxB = 112;
 constexpr int kSmallMaxLen = 2048;  // LDS of the backward
-// Pairs up to which the small form is used: both forms on 256-step series at
-// B = 49 take the same time at about 20000 pairs (one pair per lane takes
-// 560 us from 64 to 60000 pairs).
-constexpr int64_t kSmallPairs = 16384;
+constexpr double kSmallPairs = 16384;
 
 __device__ __forceinline__ float sshr1(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x138,
@@ -414,9 +413,24 @@ SmallScratch small_scratch(int mode, int64_t nx, int64_t ny, int lx, int ly) {
 
 }  // namespace
 
-bool small_train_ok(int64_t n_pairs, const Band &bd) {
-    return n_pairs <= kSmallPairs && bd.B <= kSmallMaxB && bd.lx <= kSmallMaxLen &&
-           bd.ly <= kSmallMaxLen;
+// Pairs up to which the small form is the faster one.  Its walk takes a wave a
+// pair whatever the band, the other form's time grows with the band, and its
+// walk with the length at one wave per SIMD.  Where they cross, one step
+// forward and backward (measured at 256 .. 32768 pairs, matrices and lists):
+//   series of 64:   B <= 9 16000 pairs
+//   series of 256:  B <= 9 6000, 25 8200, 49 11500, 111 13500
+//   series of 1000: B <= 9 3900, 25 5200, 49 7900, 111 9500
+// Matrices with many columns that are no multiple of 64 stay here: dX is a sum
+// over a row's pairs in turn there, 0.11 us a column (1 x 10000 pairs of 128,
+// B = 9: 191 us, 1285 us).
+bool small_train_ok(int mode, int64_t nx, int64_t ny, const Band &bd) {
+    if (bd.B > kSmallMaxB || bd.lx > kSmallMaxLen || bd.ly > kSmallMaxLen) return false;
+    const double n_pairs = mode == 0 ? (double)nx * (double)ny : (double)nx;
+    if (mode == 0 && ny % 64 != 0 && ny >= 1024) return n_pairs <= kSmallPairs;
+    const double at256 = bd.B <= 49 ? 6000.0 + 137.5 * (bd.B > 9 ? bd.B - 9 : 0)
+                                    : 11500.0 + 32.0 * (bd.B - 49);
+    return n_pairs <=
+           std::min(kSmallPairs, at256 * std::pow(256.0 / bd.lx, bd.lx < 256 ? 0.7 : 0.3));
 }
 
 static int64_t small_dec_bytes(int64_t n_pairs, const SmallGeo &g) {
