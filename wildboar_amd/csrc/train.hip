@@ -161,6 +161,7 @@ __global__ __launch_bounds__(64 * NV) __attribute__((
     const int64_t p = p0 < ps.n_pairs ? p0 : ps.n_pairs - 1;
     int64_t a, b;
     decode_pair(ps, p, a, b);
+    if constexpr (NV > 1) a = __builtin_amdgcn_readfirstlane((int)a);  // the wave's series
     const float *__restrict__ XT = go.XT + a;   // x_i = XT[i * nx]
     const double *__restrict__ PT = go.PT + b;  // prefix of y_b up to j: PT[j * ny]
     const int64_t nxs = go.nx, nys = go.ny;
@@ -213,7 +214,12 @@ __global__ __launch_bounds__(64 * NV) __attribute__((
     int jg = (ly - 1) / CG * CG;  // the next group of columns
     int sg = jg % W;
     int is = lx - 1;  // topmost row of the last column done
-    auto finish_group = [&]() {
+    // A value of x that is not finite belongs to the columns it is matched to,
+    // not to all behind it: the lanes of such series (whose total is not finite
+    // either) add the column's values up instead.
+    const bool odd = !(fabs(PX[lx * pxi]) < WBX_INF_D);
+    const bool any_odd = __ballot(odd) != 0;
+    auto finish_group = [&](auto odd_lanes) {
         double hi[CG], lo[CG];
         float cnt[CG];
         const fcg yv_ = ypw[jg / CG];
@@ -228,6 +234,12 @@ __global__ __launch_bounds__(64 * NV) __attribute__((
             cnt[e] = (float)(last - is + 1);
             hi[e] = PX[(last + 1) * pxi];
             lo[e] = PX[is * pxi];
+            if constexpr (decltype(odd_lanes)::value) {
+                if (odd) {
+                    hi[e] = lo[e] = 0.0;
+                    for (int i = is; i <= last; ++i) hi[e] += (double)XT[(int64_t)i * nxs];
+                }
+            }
         }
         fcg o;
 #pragma unroll
@@ -345,7 +357,12 @@ __global__ __launch_bounds__(64 * NV) __attribute__((
             __syncthreads();
         }
         // rows up to ih - RB reach columns below ih - RB + B - off
-        while (jg >= 0 && (ih < RB || jg >= ih - RB + B - off)) finish_group();
+        while (jg >= 0 && (ih < RB || jg >= ih - RB + B - off)) {
+            if (any_odd)
+                finish_group(std::true_type());
+            else
+                finish_group(std::false_type());
+        }
     }
 }
 

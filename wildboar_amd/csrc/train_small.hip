@@ -363,11 +363,19 @@ __global__ __launch_bounds__(64) void k_small_backward(PairSpec ps, Series<float
     __syncthreads();
     prefix(X, lx);
     __syncthreads();
+    // a value of x that is not finite belongs to the columns it is matched to,
+    // not to all behind it
+    const bool sums = fabs(pt[lx]) < WBX_INF_D;  // uniform
     for (int j = lane; j < ly; j += 64) {
         const uint32_t v = cols[j];
         const int i0 = v & 0xffff, i1 = v >> 16;
         const float cnt = (float)(i1 - i0 + 1);
-        gy[j] = __builtin_fmaf(coef * cnt, Y[j], -(coef * (float)(pt[i1 + 1] - pt[i0])));
+        double sx = 0.0;
+        if (sums)
+            sx = pt[i1 + 1] - pt[i0];
+        else
+            for (int i = i0; i <= i1; ++i) sx += (double)X[i];
+        gy[j] = __builtin_fmaf(coef * cnt, Y[j], -(coef * (float)sx));
     }
 }
 

@@ -117,6 +117,10 @@ def dtw(X, Y, r=1.0, *, metric="dtw", g=0.05, checkpoint=False):
     and recomputes each band in the backward (memory ~ B (t + n) / 32 floats
     per pair) instead of recording two decision bits per band cell; WDTW and
     bands wider than 112 slots always use it.
+
+    Where a pair's distance is not finite (values that are not, or costs past
+    float32) its gradient is 0, and NaN where such a value enters: which cells
+    its path takes there is not defined.
     """
     return _DtwFunction.apply(X, Y, float(r), 2 if checkpoint else 0, metric, float(g))
 
