@@ -20,6 +20,12 @@ namespace wbx {
 // instructions, three of them subtractions that issue beside another wave's
 // minimum or shift: 17.1 cycles a cell with x in an SGPR, 22.5 with two
 // compares into SGPR masks and two add-with-carry (x in a VGPR 17.9).
+// Costs that are not finite (then neither is the distance, and the gradient 0 or
+// NaN) are not equal even to themselves here: +inf - +inf has its sign set.  The
+// walk stays inside the band without their bits.
+// The two shifts stay last: gfx950 wants two instructions between the fma and a
+// DPP move that reads c (the strips of train_small.hip), and the compiler
+// does not look into the block.
 // XU: x is the same for the whole wave, an SGPR operand.
 #define WBX_TRAIN_CELL(X)                                                                    \
     asm("v_min3_f32 %[t], %[up], %[left], %[c]\n\t"                                          \
