@@ -62,6 +62,8 @@ def test_exact_forms(slots, nx, ny, data):
     (3073, 64, 20, 0.1),   # 385 blocks of 8 series, the last with one; band 5 (padded to 8)
     (1540, 128, 45, 0.45), # two waves per x series, band 41
     (2048, 64, 66, 0.7),   # a wide band (93 slots) at its own smallest count
+    (2048, 64, 110, 0.47), # bands of 101 and 111 slots: the most shared memory
+    (2055, 64, 120, 0.4675),
     (3080, 64, (30, 41), 0.2),
 ])
 def test_shared_prefix_blocks(nx, ny, t, r):
