@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 CASES = [  # tx, ty, r
     (5, 5, 0.4), (9, 9, 0.9), (16, 15, 0.2), (31, 31, 0.1), (64, 64, 0.1), (65, 61, 0.1),
-    (71, 72, 0.2), (128, 128, 0.1), (150, 150, 0.1), (203, 203, 0.25), (129, 129, 0.8),
+    (71, 72, 0.2), (128, 128, 0.1), (150, 150, 0.1), (203, 203, 0.25), (129, 129, 0.8), (24, 24, 1.0), (43, 43, 0.52),
 ]
 
 

@@ -280,8 +280,8 @@ int run_pairs(const wbx_metric *m, const PairSpec &ps, Series<T> xs, Series<T> y
         // B = 23, 49, 101; at 20000 pairs of 512, B = 101, 293 us against
         // 124 us of six lanes a pair, at 100000 359 against 469).  A second
         // wave issues in the first one's gaps, so two take the larger of one
-        // alone and their two shares (90000 pairs of 800, B = 49: 265 us, the
-        // group kernel 307).  Padded
+        // alone and their two shares (exact widths; 90000 pairs of 800, B = 49: 265
+        // us, the group kernel 307).  Padded
         // widths, weights and float64 cost more; float32 WDTW and float64
         // lanes are for bands up to 40 slots (at 49 the group kernel is
         // 1.1-1.4x faster at any size); ADTW has no group form.
@@ -295,12 +295,12 @@ int run_pairs(const wbx_metric *m, const PairSpec &ps, Series<T> xs, Series<T> y
             const int slots = exact ? B : (B + 7) / 8 * 8;
             const double alone = (exact ? 20.0 : 30.0) + (wt ? 7.5 : 5.5) * slots;
             const double share = (wt ? 4.8 : 3.4) * slots;
-            const bool two = !wt && lane_waves > 1024 && lane_waves <= 2048;
+            const bool two = exact && lane_waves > 1024 && lane_waves <= 2048;
             lane_ns = two ? pair_launch_ns(1, bd.lx, std::max(alone, 2.0 * share), 0.0)
                           : pair_launch_ns(lane_waves, bd.lx, alone, share);
         } else {
             const int slots = lane64_pairs_class(B, wt);
-            lane = slots != 0 && (B <= 40 || pen);
+            lane = slots != 0 && (B <= 40 || pen || (wt && B <= 48));
             lane_ns = pair_launch_ns(lane_waves, bd.lx, (wt ? 13.5 : 11.5) * slots,
                                      (wt ? 13.0 : 11.0) * slots);
         }
@@ -320,6 +320,10 @@ int run_pairs(const wbx_metric *m, const PairSpec &ps, Series<T> xs, Series<T> y
                     sq, st);
             }
         }
+        // float64 WDTW bands of 41 .. 48 slots: the lanes where the group kernel
+        // has no strip that fits the band well (B = 47, 10^6 pairs of 24: 304 us,
+        // strips of 7 slots 660)
+        if (dbl && wt && B > 40 && group && lane_ns > 0.7 * group_ns) lane = false;
         if (group && group_ns < lane_ns) lane = false;
         if (policy == 2 && group) lane = false;  // group kernel wherever it applies
         if (lane) {
