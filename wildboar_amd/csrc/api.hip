@@ -247,9 +247,9 @@ bool lane64_ok(const DeviceCtx *ctx, const void *weights) {
     return !weights || cached_weights_min(ctx, weights) > 0.0;
 }
 
-// The pairs of ps (squared costs into sq, or distances to ps.out).  m->kind is EUCLIDEAN, DTW, WDTW or ADTW
-// (the derivative kinds arrive here as DTW / WDTW on slopes); w_fixed > 0
-// replaces every pair's band width.
+// The pairs of ps (squared costs into sq, or distances to ps.out).  m->kind is
+// EUCLIDEAN, DTW, WDTW or ADTW (the derivative kinds arrive here as DTW / WDTW
+// on slopes); w_fixed > 0 replaces every pair's band width.
 template <typename T>
 int run_pairs(const wbx_metric *m, const PairSpec &ps, Series<T> xs, Series<T> ys,
               const T *weights, T *sq, hipStream_t st, int w_fixed = 0) {
@@ -280,11 +280,11 @@ int run_pairs(const wbx_metric *m, const PairSpec &ps, Series<T> xs, Series<T> y
         // B = 23, 49, 101; at 20000 pairs of 512, B = 101, 293 us against
         // 124 us of six lanes a pair, at 100000 359 against 469).  A second
         // wave issues in the first one's gaps, so two take the larger of one
-        // alone and their two shares (exact widths; 90000 pairs of 800, B = 49: 265
-        // us, the group kernel 307).  Padded
-        // widths, weights and float64 cost more; float32 WDTW and float64
-        // lanes are for bands up to 40 slots (at 49 the group kernel is
-        // 1.1-1.4x faster at any size); ADTW has no group form.
+        // alone and their two shares (exact widths; 90000 pairs of 800, B = 49:
+        // 265 us, the group kernel 307).  Padded widths, weights and float64
+        // cost more.  Padded float32 WDTW and float64 DTW lanes are for bands
+        // up to 40 slots (at 49 the group kernel is 1.1-1.4x faster at any
+        // size), float64 WDTW to 48 (below); ADTW has no group form.
         constexpr bool dbl = !std::is_same<T, float>::value;
         bool lane;
         double lane_ns = 0.0;

@@ -305,8 +305,8 @@ typedef const float __attribute__((address_space(4))) *cfloat;
 // lane -> XU: B = 23 2.92 -> 2.67 ms, B = 49 5.52 -> 5.23, B = 75 8.83 -> 8.10,
 // B = 101 12.02 -> 10.73, B = 111 13.05 -> 11.70.
 // WT: WDTW (equal lengths, XU; weights: at least (B + 1) / 2 values, which
-// lane_exact_w_waves sees to).  1000 x
-// 1000 x 256, B = 49: 1205 us on the group kernel, 873 us.
+// lane_exact_w_waves sees to).  1000 x 1000 x 256, B = 49: 1205 us on the
+// group kernel, 873 us.
 template <int B, int U, bool XU, bool WT = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_lane_dtw_exact(
     PairSpec ps, Series<float> xs, Series<float> ys, LaneGeo g,

@@ -103,9 +103,9 @@ constexpr int train_waves(int slots) {
 // with the sign-bit cell and a shared x.
 template <int BP, int U, bool EX, bool XU>
 __global__ __launch_bounds__(64) __attribute__((
-    amdgpu_waves_per_eu(train_waves(XU ? BP : BP + 4)))) void k_lane_train(PairSpec ps, Series<float> xs, Series<float> ys,
-                                                   LaneGeo g, float *__restrict__ sq,
-                                                   uint32_t *__restrict__ dirs) {
+    amdgpu_waves_per_eu(train_waves(XU ? BP : BP + 4)))) void
+k_lane_train(PairSpec ps, Series<float> xs, Series<float> ys, LaneGeo g, float *__restrict__ sq,
+             uint32_t *__restrict__ dirs) {
     constexpr int W = BP + U - 1;
     constexpr int NW = (BP + 31) / 32;
     const int lane = threadIdx.x;
