@@ -678,7 +678,7 @@ def main():
             "measured_valu_peak_cells_per_s": probe / 3,
             "frac_of_measured": achieved / (probe / 3),
             "traffic_note": "HBM bytes per launch from rocprofv3 FETCH_SIZE x 2.0 + WRITE_SIZE "
-                            "x 1.0 (copy-kernel calibration); algorithmic bytes 24.6 MB",
+                            "x 1.0 (copy-kernel calibration); algorithmic bytes 40.2 MB",
         },
     }
 
